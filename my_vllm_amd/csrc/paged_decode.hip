@@ -37,24 +37,51 @@ int launch_paged_decode(const DecodeParams& p, int waves_per_group, hipStream_t 
   return check_launch("paged_decode");
 }
 
-// Split-K merges: four wavefronts per workgroup, one per (merge entry,
-// query head), in the first merge_blocks workgroups.  Graph launches size the
-// grid for the merge capacity and read this step's merge count from
-// p.counts[2].  After a fused-store launch the workgroups past merge_blocks
-// write the late rows, one wavefront per new token.
-template <typename T>
-__global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p, const int32_t* __restrict__ merges,
-                                                           int64_t num_waves, int64_t merge_blocks) {
+// Split-K merges.  kWide 1: four wavefronts per workgroup, one per (merge
+// entry, query head).  kWide > 1: a workgroup of kWide wavefronts per (merge
+// entry, query head).  Graph launches size the grid for the merge capacity
+// and read this step's merge count from p.counts[2].  After a fused-store
+// launch the workgroups past merge_blocks write the late rows, one wavefront
+// per new token.
+template <typename T, int kWide>
+__global__ __launch_bounds__(kWide == 1 ? 256 : 64 * kWide) void decode_merge_kernel(
+    DecodeParams p, const int32_t* __restrict__ merges, int64_t num_waves, int64_t merge_blocks) {
+  constexpr int kGroup = kWide == 1 ? 4 : kWide;  // wavefronts per workgroup
+  __shared__ __attribute__((aligned(16))) float red[kWide == 1 ? 1 : kWide * (kHeadDim + 2)];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if ((int64_t)blockIdx.x >= merge_blocks) {
-    const int64_t row = ((int64_t)blockIdx.x - merge_blocks) * 4 + w;
+    const int64_t row = ((int64_t)blockIdx.x - merge_blocks) * kGroup + w;
     if (row < p.num_new) decode_late_store_wave<T>(p, row);
     return;
   }
-  const int64_t v = (int64_t)blockIdx.x * 4 + w;
+  const int64_t v = kWide == 1 ? (int64_t)blockIdx.x * 4 + w : (int64_t)blockIdx.x;
   if (v >= num_waves) return;
   if (p.counts != nullptr && v >= (int64_t)max(sload(p.counts, 2), 0) * p.group) return;
-  decode_merge_wave<T>(p, merges, v);
+  // v is wave-uniform: the descriptor comes in through scalar loads.
+  const i32x8 d = ((const_i32x8*)merges)[v / p.group];
+  merge_segment<T, false, kWide>(p, d, (int)(v % p.group), kWide == 1 ? 0 : w, red);
+}
+
+// Wavefronts per merge of a launch of `num_merges` merges over
+// `num_part_slots` slots a KV head.  One wavefront takes 32 chunks in one
+// memory round trip, eight take 256; but most of the eight idle where merges
+// are short, and the launch then spends its time starting them.  Decode call
+// at 32 / 8 heads, one / eight wavefronts a merge: 1 sequence of 8192 tokens
+// (256 chunks) 23.4 / 15.0 us, 8 of 768 (33) 15.7 / 14.9 us, 16 (17) 19.6 /
+// 19.4 us, 24 (12) 22.6 / 23.4 us, 64 (5) 48.8 / 52.1 us: eight above 16
+// chunks on average.
+constexpr int kWideMergeWaves = 8;
+constexpr int kWideMergeChunks = 16;
+
+template <typename T>
+void launch_merge_kernel(const DecodeParams& p, const int32_t* merges, int64_t waves, bool wide, int64_t merge_blocks,
+                         int64_t blocks, hipStream_t stream) {
+  if (wide)
+    hipLaunchKernelGGL((decode_merge_kernel<T, kWideMergeWaves>), dim3((uint32_t)blocks), dim3(64 * kWideMergeWaves),
+                       0, stream, p, merges, waves, merge_blocks);
+  else
+    hipLaunchKernelGGL((decode_merge_kernel<T, 1>), dim3((uint32_t)blocks), dim3(256), 0, stream, p, merges, waves,
+                       merge_blocks);
 }
 
 }  // namespace
@@ -63,20 +90,18 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p, const
 // same stream; `merges` lists the split segments (piece descriptors).  After
 // a fused-store launch (p.k_new set) it always runs: its late-store
 // workgroups write the new rows the decode launch left.
-int launch_decode_merge(const DecodeParams& p, const int32_t* merges, int64_t num_merges, int dtype,
-                        hipStream_t stream) {
+int launch_decode_merge(const DecodeParams& p, const int32_t* merges, int64_t num_merges, int64_t num_part_slots,
+                        int dtype, hipStream_t stream) {
   const int64_t late_rows = p.k_new != nullptr ? p.num_new : 0;
   if (num_merges == 0 && late_rows == 0) return 0;
   const int64_t waves = num_merges * p.group;
-  const int64_t merge_blocks = (waves + 3) / 4;
-  const int64_t blocks = merge_blocks + (late_rows + 3) / 4;
+  const bool wide = num_merges > 0 && num_part_slots * p.num_kv_heads > kWideMergeChunks * num_merges;
+  const int64_t per_block = wide ? kWideMergeWaves : 4;
+  const int64_t merge_blocks = wide ? waves : (waves + 3) / 4;
+  const int64_t blocks = merge_blocks + (late_rows + per_block - 1) / per_block;
   if (blocks > 0x7fffffffLL) return set_error("paged attention: too many split-K merges");
-  if (dtype == kBF16)
-    hipLaunchKernelGGL(decode_merge_kernel<__bf16>, dim3((uint32_t)blocks), dim3(256), 0, stream, p, merges, waves,
-                       merge_blocks);
-  else
-    hipLaunchKernelGGL(decode_merge_kernel<_Float16>, dim3((uint32_t)blocks), dim3(256), 0, stream, p, merges,
-                       waves, merge_blocks);
+  if (dtype == kBF16) launch_merge_kernel<__bf16>(p, merges, waves, wide, merge_blocks, blocks, stream);
+  else launch_merge_kernel<_Float16>(p, merges, waves, wide, merge_blocks, blocks, stream);
   return check_launch("decode_merge");
 }
 
@@ -199,7 +224,7 @@ extern "C" int mva_paged_decode(const void* q, int64_t q_token_stride, int64_t q
   else if (dtype == kF16) rc = launch_paged_decode<_Float16>(p, waves_per_group, s);
   else return set_error("paged attention: dtype must be bf16 or fp16");
   if (rc) return rc;
-  return launch_decode_merge(p, merges, num_merges, dtype, s);
+  return launch_decode_merge(p, merges, num_merges, num_part_slots, dtype, s);
 }
 
 extern "C" int mva_paged_decode_store(const void* q, int64_t q_token_stride, int64_t q_head_stride,
@@ -250,7 +275,7 @@ extern "C" int mva_paged_decode_store(const void* q, int64_t q_token_stride, int
                         : launch_paged_decode<_Float16>(p, waves_per_group, s);
     if (rc) return rc;
   }
-  return launch_decode_merge(p, merges, num_merges, dtype, s);
+  return launch_decode_merge(p, merges, num_merges, num_part_slots, dtype, s);
 }
 
 extern "C" int mva_paged_decode_graph(const void* q, int64_t q_token_stride, int64_t q_head_stride,
@@ -283,7 +308,7 @@ extern "C" int mva_paged_decode_graph(const void* q, int64_t q_token_stride, int
   else if (dtype == kF16) rc = launch_paged_decode<_Float16>(p, waves_per_group, s);
   else return set_error("paged attention: dtype must be bf16 or fp16");
   if (rc) return rc;
-  return launch_decode_merge(p, merges, merge_capacity, dtype, s);
+  return launch_decode_merge(p, merges, merge_capacity, num_part_slots, dtype, s);
 }
 
 // ---- decode with no allocation: static device scratch ---------------------

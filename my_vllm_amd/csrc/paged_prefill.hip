@@ -15,8 +15,6 @@ int fill_decode_params(DecodeParams& p, const void* q, int64_t q_token_stride, i
                        int64_t out_head_stride, void* workspace, int64_t workspace_bytes,
                        int num_q_heads, int num_kv_heads, int head_dim, int page_size,
                        float softmax_scale);
-int launch_decode_merge(const DecodeParams& p, const int32_t* merges, int64_t num_merges, int dtype,
-                        hipStream_t stream);
 int32_t* decode_arrival_counters(void* workspace);
 
 namespace {

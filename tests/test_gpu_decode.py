@@ -189,6 +189,31 @@ def test_merge_of_one_page_pieces_for_every_group_shape(gpu, hq, hkv):
     assert torch.equal(out, first)
 
 
+@pytest.mark.parametrize("hq,hkv,pages", [
+    (32, 8, [257, 33]),             # eight wavefronts a merge, a second round of one chunk
+    (8, 8, [256, 32, 31]),          # whole rounds; merges that end in the first wavefront
+    (40, 8, [65, 20]),              # three wavefronts with work, odd group
+    (16, 1, [100] + [2] * 40),      # one wavefront a merge walks four rounds
+    (16, 2, [33] + [2] * 30 + [1]),  # a round of one chunk; a segment without a merge
+])
+def test_merge_widths_and_rounds(gpu, hq, hkv, pages):
+    # One-page pieces: a context of n pages merges n chunks.  The launch gives
+    # a merge eight wavefronts above 16 chunks on average, else one; 32 chunks
+    # a wavefront and round.
+    ctx = [16 * n - (n % 3) for n in pages]
+    batch = make_paged_batch(68, [1] * len(ctx), ctx, 0, hq, hkv)
+    common, q, kc, vc = _to(batch, gpu)
+    items, nw, slots = make_decode_plan(np.asarray(pages), 0, 0, hkv, 100000, 64, 1, 1)
+    merges = ops.decode_merge_list(items)
+    assert int(items[:, 4].max()) == max(pages) and merges.shape[0] == hkv * sum(n > 1 for n in pages)
+    assert (slots * hkv > 16 * merges.shape[0]) == (len(pages) <= 3)
+    ws = torch.zeros(ops.decode_workspace_bytes(slots, hkv, hq // hkv), dtype=torch.uint8, device=gpu)
+    out = torch.full_like(q, float("nan"))
+    ops.paged_decode(q, kc, vc, common.block_tables, common.seq_lens, _to_device(items, gpu), items.shape[0], nw,
+                     _to_device(merges, gpu), merges.shape[0], slots, out, ws, 128 ** -0.5)
+    assert_attention_close(out, _expected(batch))
+
+
 def test_stale_nan_rows_past_seq_len_do_not_leak(gpu, monkeypatch):
     set_decode_planning(monkeypatch, waves=100000)
     ctx = [5, 16, 33, 300, 129]
