@@ -280,6 +280,9 @@ __device__ inline void store16_device_untracked(void* addr, u32x4 v) {
 __device__ inline void store4_device_untracked(void* addr, float v) {
   asm volatile("global_store_dword %0, %1, off sc1" ::"v"(addr), "v"(v) : "memory");
 }
+__device__ inline void store8_device_untracked(void* addr, u32x2 v) {
+  asm volatile("global_store_dwordx2 %0, %1, off sc1\n\ts_nop 1" ::"v"(addr), "v"(v) : "memory");
+}
 __device__ inline void store8_untracked(void* addr, u32x2 v) {
   asm volatile("global_store_dwordx2 %0, %1, off\n\ts_nop 1" ::"v"(addr), "v"(v) : "memory");
 }

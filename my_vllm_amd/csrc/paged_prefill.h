@@ -558,9 +558,35 @@ constexpr int kPrefillPlanItemInts = 16;
 constexpr int kPrefillPlanDroppedInt = 1;
 constexpr int kPrefillPlanExitInt = 16;
 constexpr int kPrefillPlanGridInt = 17;
+// Batches of at most one item per workgroup of a head (the fixed form of the
+// launch): words 18 .. 21 = {pieces, word offsets into the plan buffer of the
+// piece list and the arrival counters, the partials' offset in
+// kPrefillPartUnit bytes}.  pieces > 0: the items are the pieces of the piece
+// list; 0: the tiles.
+constexpr int kPrefillPlanPiecesInt = 18;
+constexpr int kPrefillPlanPieceListInt = 19;
+constexpr int kPrefillPlanArriveInt = 20;
+constexpr int kPrefillPlanPartInt = 21;
 constexpr int kPrefillPlanLineInts = 32;
 constexpr int kPrefillPlanMaxHeads = 127;
 constexpr int kPrefillPlanHeaderInts = kPrefillPlanLineInts * (1 + kPrefillPlanMaxHeads);
+// A split-K piece: a tile record whose key counts, positions and pages are
+// those of the piece's keys, then {first page of the piece in the sequence,
+// pieces of the tile, the tile's first piece}.  Piece i of KV head h has
+// partial slot i * Hkv + h, and the tile's arrival counter is number
+// (first piece) * Hkv + h.
+constexpr int kPrefillPieceInts = 32;
+constexpr int kPrefillPieceFirstPage = 16;
+constexpr int kPrefillPieceCount = 17;
+constexpr int kPrefillPieceFirst = 18;
+// A tile is cut into at most this many pieces (one workgroup reads all of a
+// tile's partials), and a plan has at most this many (piece, KV head) pairs.
+constexpr int kPrefillMaxPieces = 8;
+constexpr int kPrefillPieceSlots = 256;
+// One partial: 64 floats of O, m and l of each of 512 threads.
+constexpr int kPrefillPartBytes = 512 * (64 + 2) * 4;
+constexpr int kPrefillPartUnit = 256;
+static_assert(kPrefillPartBytes % kPrefillPartUnit == 0, "partials stay aligned");
 // Largest batch the planner sorts longest-context first (a larger batch is
 // planned in batch order).
 constexpr int kPrefillPlanSortMax = 2048;

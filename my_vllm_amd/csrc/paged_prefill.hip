@@ -19,6 +19,118 @@ int32_t* decode_arrival_counters(void* workspace);
 
 namespace {
 
+// Piece list and arrival counters, before the partials, in words.
+constexpr int64_t kPrefillSplitMetaInts = kPrefillPieceSlots * (kPrefillPieceInts + 1);
+static_assert(kPrefillSplitMetaInts * 4 % kPrefillPartUnit == 0, "partials stay aligned");
+// Word offset of the piece list of a plan of at most max_tiles tiles, and the
+// bytes of such a plan with its split-K area.
+int64_t prefill_piece_list(int64_t max_tiles) {
+  const int64_t unit = kPrefillPartUnit / 4;
+  return (kPrefillPlanHeaderInts + max_tiles * kPrefillPlanItemInts + unit - 1) / unit * unit;
+}
+int64_t prefill_plan_bytes(int64_t max_tiles) {
+  return (kPrefillPlanHeaderInts + max_tiles * kPrefillPlanItemInts) * 4;
+}
+int64_t prefill_split_bytes(int64_t max_tiles) {
+  return (prefill_piece_list(max_tiles) + kPrefillSplitMetaInts) * 4 + (int64_t)kPrefillPieceSlots * kPrefillPartBytes;
+}
+
+// Split-K pieces of the n planned tiles, for a batch whose tiles leave most
+// workgroups idle: returns their number, or 0 when whole tiles are as good.
+// A launch of few tiles lasts as long as its longest one (1.5 to 1.85 us per
+// 64 keys), so tiles longer than L key tiles are cut into near-equal pieces of
+// at most L.  L is ceil(longest / k) for the k in 1 .. kPrefillMaxPieces with
+// the smallest L + 2.5 + 0.75 k (key tiles; a split costs writing the partials
+// and one workgroup reading k of them: 4.7 and 5.3 us at k = 4 with all 256
+// workgroups busy), among those whose pieces fit one per workgroup.  All 1024 threads call it; nt, first and best are LDS
+// arrays of at least 1024 ints.  piece_list <= 0: no room for partials.
+__device__ int plan_pieces(int32_t* __restrict__ plan, int n, int per_head, int num_kv_heads,
+                           const int32_t* __restrict__ block_tables, int64_t bt_stride, int64_t num_pages,
+                           int piece_list, int* nt, int* first, int* best) {
+  const int tid = threadIdx.x;
+  const int limit = min(per_head, kPrefillPieceSlots / num_kv_heads);
+  if (piece_list <= 0 || n == 0 || n > limit) return 0;  // limit <= kPrefillPieceSlots
+  const int32_t* tiles = plan + kPrefillPlanHeaderInts;
+  __syncthreads();
+  if (tid < n) nt[tid] = tiles[tid * kPrefillPlanItemInts + 5];
+  __syncthreads();
+  // Wave k - 1 counts the pieces at k and prices them.
+  const int lane = tid & 63, k = (tid >> 6) + 1;
+  if (k <= kPrefillMaxPieces) {
+    int longest = 0;
+    for (int i = lane; i < n; i += 64) longest = max(longest, nt[i]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
+    const int len = max((longest + k - 1) / k, 1);
+    int count = 0;
+    for (int i = lane; i < n; i += 64) count += (nt[i] + len - 1) / len;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) count += __shfl_xor(count, off);
+    if (lane == 0) {
+      best[2 * k] = count > limit ? 0x7fffffff : k == 1 ? 4 * len : 4 * len + 10 + 3 * k;
+      best[2 * k + 1] = len;
+    }
+  }
+  __syncthreads();
+  int pick = 1;
+  for (int c = 2; c <= kPrefillMaxPieces; ++c)
+    if (best[2 * c] < best[2 * pick]) pick = c;
+  if (pick == 1) return 0;
+  const int len = best[2 * pick + 1];
+  // First piece of each tile (n <= 256: wave 0 scans 64 tiles at a time).
+  if (tid < 64) {
+    int carry = 0;
+    for (int c = 0; c < n; c += 64) {
+      const int v = c + lane < n ? (nt[c + lane] + len - 1) / len : 0;
+      int incl = v;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int up = __shfl_up(incl, off);
+        if (lane >= off) incl += up;
+      }
+      if (c + lane < n) first[c + lane] = carry + incl - v;
+      carry += __shfl(incl, 63);
+    }
+    if (lane == 0) first[n] = carry;
+  }
+  __syncthreads();
+  const int total = first[n];
+  for (int i = tid; i < kPrefillPieceSlots; i += 1024) plan[piece_list + kPrefillPieceSlots * kPrefillPieceInts + i] = 0;
+  for (int i = tid; i < total; i += 1024) {
+    int lo = 0, hi = n - 1;  // last tile whose first piece is <= i
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (first[mid] <= i) lo = mid;
+      else hi = mid - 1;
+    }
+    const int cuts = first[lo + 1] - first[lo];
+    const int c = i - first[lo];
+    const int a = (int)((int64_t)c * nt[lo] / cuts), b = (int)((int64_t)(c + 1) * nt[lo] / cuts);
+    const int32_t* t = tiles + lo * kPrefillPlanItemInts;
+    const int pages_per_tile = kPrefillKeys / kPageSize;
+    const int npages = min(t[7] - a * pages_per_tile, (b - a) * pages_per_tile);
+    const int32_t* bt = block_tables + (int64_t)t[0] * bt_stride + a * pages_per_tile;
+    int32_t* d = plan + piece_list + (int64_t)i * kPrefillPieceInts;
+    d[0] = t[0];
+    d[1] = t[1];
+    d[2] = t[2];
+    d[3] = t[3];
+    d[4] = t[4] - a * kPrefillKeys;
+    d[5] = b - a;
+    d[6] = min(max(t[6] - a, 0), b - a);
+    d[7] = npages;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int v = bt[min(j, npages - 1)];
+      d[8 + j] = (v >= 0 && v < num_pages) ? v : 0;
+    }
+    d[kPrefillPieceFirstPage] = a * pages_per_tile;
+    d[kPrefillPieceCount] = cuts;
+    d[kPrefillPieceFirst] = first[lo];
+  }
+  return total;
+}
+
 // Exact tile list of a prefill batch, built on the device from
 // query_start_loc / seq_lens (one workgroup; see kPrefillPlanHeaderInts for
 // the format).  Sequences are ordered longest context first (batches of up
@@ -38,7 +150,7 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(const int32_t* __res
                                                             int64_t bt_stride, int64_t num_pages, int num_seqs,
                                                             int tile_tokens, int num_kv_heads,
                                                             int32_t* __restrict__ plan, int capacity, int tail,
-                                                            int grid) {
+                                                            int grid, int per_head, int piece_list) {
   // Sequences in plan order (rank -> sequence) and the first tile of each
   // rank; beyond kPrefillPlanSortMax sequences, all keep batch order and are
   // planned in passes of kPrefillPlanSortMax.
@@ -163,13 +275,19 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(const int32_t* __res
       }
     }
   }
+  const int pieces = plan_pieces(plan, min(carry, capacity), per_head, num_kv_heads, block_tables, bt_stride,
+                                 num_pages, piece_list, scan, first_tile, order);
   if (tid == 0) {
+    plan[kPrefillPlanPiecesInt] = pieces;
+    plan[kPrefillPlanPieceListInt] = piece_list;
+    plan[kPrefillPlanArriveInt] = piece_list + kPrefillPieceSlots * kPrefillPieceInts;
+    plan[kPrefillPlanPartInt] = (int)((piece_list + kPrefillSplitMetaInts) / (kPrefillPartUnit / 4));
     plan[0] = min(carry, capacity);
     plan[kPrefillPlanDroppedInt] = max(carry - capacity, 0);
     plan[kPrefillPlanExitInt] = 0;
     plan[kPrefillPlanGridInt] = grid;
   }
-  if (tid < num_kv_heads) plan[kPrefillPlanLineInts * (1 + tid)] = 0;  // claim counters
+  if (tid < kPrefillPlanMaxHeads) plan[kPrefillPlanLineInts * (1 + tid)] = 0;  // claim counters
 }
 
 // Persistent prefill: workgroup b serves KV head b % num_kv_heads (so head
@@ -185,9 +303,9 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_stream_kernel
   __shared__ int nextq[4];
   const int h = (int)(blockIdx.x % (uint32_t)p.num_kv_heads);
   if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) == 0)
-    prefill_items_pingpong<T, 0>(p, plan, h, (lds_u8*)tiles, (lds_i32*)nextq);
+    prefill_items_pingpong<T, 0, false>(p, plan, h, 0, (lds_u8*)tiles, (lds_i32*)nextq);
   else
-    prefill_items_pingpong<T, 1>(p, plan, h, (lds_u8*)tiles, (lds_i32*)nextq);
+    prefill_items_pingpong<T, 1, false>(p, plan, h, 0, (lds_u8*)tiles, (lds_i32*)nextq);
   // The last workgroup out zeroes the claim counters and the exit count, so
   // the plan serves the next launch as it is.  Every claim and counter read
   // of a workgroup has returned (its result decided the exit) before thread 0
@@ -207,6 +325,21 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_stream_kernel
       if (threadIdx.x == 0) __hip_atomic_store(plan + kPrefillPlanExitInt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
+}
+
+// The fixed form, for a batch of at most one tile per workgroup of a head: no
+// claims, and tiles may be cut into split-K pieces (plan_pieces).
+template <typename T>
+__global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_fixed_kernel(PrefillParams p,
+                                                                                int32_t* __restrict__ plan) {
+  __shared__ __attribute__((aligned(16))) uint8_t tiles[kPrefillPPLdsBytes];
+  __shared__ int nextq[8];
+  const int h = (int)(blockIdx.x % (uint32_t)p.num_kv_heads);
+  const int rank = (int)(blockIdx.x / (uint32_t)p.num_kv_heads);
+  if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) == 0)
+    prefill_items_pingpong<T, 0, true>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
+  else
+    prefill_items_pingpong<T, 1, true>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
 }
 
 int device_cu_count() {
@@ -446,7 +579,9 @@ extern "C" int mva_prefill_tile_tokens(int num_q_heads, int num_kv_heads) {
 
 extern "C" int64_t mva_prefill_workspace_bytes(int64_t max_tiles) {
   if (max_tiles < 0 || max_tiles > 0x7fffffffLL / mva::kPrefillPlanItemInts) return -1;
-  return (mva::kPrefillPlanHeaderInts + max_tiles * mva::kPrefillPlanItemInts) * 4;
+  // Up to this many tiles a plan may be cut into split-K pieces.
+  if (max_tiles <= mva::kPrefillPieceSlots) return mva::prefill_split_bytes(max_tiles);
+  return mva::prefill_plan_bytes(max_tiles);
 }
 
 namespace {
@@ -468,8 +603,9 @@ int prefill_launch(const void* q, int64_t q_token_stride, int64_t q_head_stride,
                                num_kv_heads, head_dim, page_size, softmax_scale);
   if (rc) return rc;
   if (dtype != kBF16 && dtype != kF16) return set_error("paged attention: dtype must be bf16 or fp16");
-  const int64_t need = mva_prefill_workspace_bytes(max_tiles);
-  if (need < 0) return set_error("paged attention: invalid tile capacity");
+  if (mva_prefill_workspace_bytes(max_tiles) < 0) return set_error("paged attention: invalid tile capacity");
+  // The plan itself must fit; without room for partials no tile is split.
+  const int64_t need = prefill_plan_bytes(max_tiles);
   if (num_seqs == 0 || max_tiles == 0) return 0;
   if (workspace == nullptr || workspace_bytes < need)
     return set_error("paged attention: prefill workspace too small for max_tiles");
@@ -479,20 +615,33 @@ int prefill_launch(const void* q, int64_t q_token_stride, int64_t q_head_stride,
   if (num_kv_heads > kPrefillPlanMaxHeads) return set_error("paged attention: at most 127 KV heads");
   p.tile_tokens = kPrefillPPRows / p.group;
   // Persistent grid: one workgroup per CU (96 KB of LDS and two waves per
-  // SIMD each), a whole number per KV head, never more than the tiles can use.
+  // SIMD each), a whole number per KV head, also where the tiles are fewer:
+  // they may be planned as pieces.
   int64_t per_head = (int64_t)device_cu_count() / num_kv_heads;
-  per_head = per_head < 1 ? 1 : (per_head > max_tiles ? max_tiles : per_head);
+  per_head = per_head < 1 ? 1 : per_head;
+  // A batch of at most one tile per workgroup runs the fixed form.
+  const bool fixed = max_tiles <= per_head;
   if (plan_it) {
     // The last three tiles per workgroup of a head go largest first.
-    const int tail = (int)(3 * per_head < 1024 ? 3 * per_head : 1024);
+    const int64_t last = 3 * (per_head < max_tiles ? per_head : max_tiles);
+    const int tail = (int)(last < 1024 ? last : 1024);
+    const bool split = fixed && max_tiles <= kPrefillPieceSlots && workspace_bytes >= prefill_split_bytes(max_tiles);
     hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(1024), 0, s, query_start_loc, seq_lens, block_tables,
                        block_table_stride, num_pages, (int)num_seqs, p.tile_tokens, num_kv_heads, plan,
-                       (int)max_tiles, tail, (int)(per_head * num_kv_heads));
+                       (int)max_tiles, tail, (int)(per_head * num_kv_heads), (int)per_head,
+                       split ? (int)prefill_piece_list(max_tiles) : 0);
     rc = check_launch("paged_prefill plan");
     if (rc) return rc;
   }
   if (!run_it) return 0;
   const dim3 grid((uint32_t)(per_head * num_kv_heads));
+  if (fixed) {
+    if (dtype == kBF16)
+      hipLaunchKernelGGL(paged_prefill_fixed_kernel<__bf16>, grid, dim3(kPrefillPPThreads), 0, s, p, plan);
+    else
+      hipLaunchKernelGGL(paged_prefill_fixed_kernel<_Float16>, grid, dim3(kPrefillPPThreads), 0, s, p, plan);
+    return check_launch("paged_prefill");
+  }
   if (dtype == kBF16)
     hipLaunchKernelGGL(paged_prefill_stream_kernel<__bf16>, grid, dim3(kPrefillPPThreads), 0, s, p, plan);
   else

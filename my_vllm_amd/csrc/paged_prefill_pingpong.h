@@ -34,12 +34,25 @@ constexpr int kPrefillPPThreads = 512;  // 8 wavefronts
 constexpr int kPrefillPPBufs = 3;       // LDS buffers per K and V
 constexpr int kPrefillPPLdsBytes = 2 * kPrefillPPBufs * kPrefillTileBytes;
 
-// The plan record of tile `idx` with the page ids of page slot `slot` (0..3)
-// of 64-key tiles 0 and 1.
-__device__ inline PrefillWork plan_work_slot(const int32_t* plan, int idx, int slot) {
-  const i32x16 d = ((const_i32x16*)(plan + kPrefillPlanHeaderInts))[idx];
-  PrefillWork wk;
-  wk.s = d[0];
+// One item of the stream: a query tile over a range of its keys (the whole
+// range, or one split-K piece of it).  Key counts and positions are relative
+// to the range's first key, and btp points at its first page id.
+struct StreamWork {
+  const int32_t* btp;
+  int t0, q0, q_len, kv, ntiles, full_tiles, npages, pg0, pg1;
+};
+
+// Item `idx` of the plan's tile list (kFixed: of its piece list, when it has
+// one) with the page ids of page slot `slot` (0..3) of its 64-key tiles 0 and 1.
+template <bool kFixed>
+__device__ inline StreamWork plan_work_slot(const PrefillParams& p, const int32_t* plan, int idx, int slot) {
+  const bool pieces = kFixed && sload(plan, kPrefillPlanPiecesInt) > 0;
+  const int32_t* rec = pieces ? plan + sload(plan, kPrefillPlanPieceListInt) + (int64_t)idx * kPrefillPieceInts
+                              : plan + kPrefillPlanHeaderInts + (int64_t)idx * kPrefillPlanItemInts;
+  const i32x16 d = *(const_i32x16*)rec;
+  const int first_page = pieces ? sload(rec, kPrefillPieceFirstPage) : 0;
+  StreamWork wk;
+  wk.btp = p.block_tables + (int64_t)d[0] * p.bt_stride + first_page;
   wk.t0 = d[1];
   wk.q0 = d[2];
   wk.q_len = d[3];
@@ -54,15 +67,104 @@ __device__ inline PrefillWork plan_work_slot(const int32_t* plan, int idx, int s
 
 typedef __attribute__((address_space(3))) int32_t lds_i32;
 
+// 16 and 8 bytes of a partial, read past this XCD's L2 (sc1).
+__device__ inline f32x4 part_ld16(__amdgpu_buffer_rsrc_t r, int off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 16));
+}
+__device__ inline f32x2 part_ld8(__amdgpu_buffer_rsrc_t r, int off) {
+  return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 16));
+}
+
+// End of a split-K piece of KV head `head`: writes the workgroup's fp32
+// partial (O, the row max m and the row sum l, each thread its own registers,
+// so every access is 16 bytes a lane and contiguous), counts the piece in,
+// and, when it is the tile's last piece to arrive, replaces o, l by
+//   sum_c w_c o_c, sum_c w_c l_c,  w_c = 2^(m_c - max_c m_c)
+// over the tile's pieces c in key order, whichever piece arrived last, so the
+// result does not depend on timing.  Returns whether the caller now holds the
+// tile's result (true also for a piece that is its tile's only one).  Every
+// thread of the workgroup calls it; `word` is a free LDS word.
+//
+// Visibility across XCDs: the partials are written through (sc1) and retired
+// (vmcnt(0), every wave, then the barrier) before thread 0 counts the piece
+// in, and the merging workgroup reads them with sc1 loads.  No workgroup
+// waits for another.
+__device__ __attribute__((always_inline)) inline bool settle_piece(int32_t* plan, int idx, int head, int num_heads,
+                                                                   f32x16 (&o)[4], float m, float& l, lds_i32* word) {
+  const int32_t* rec = plan + sload(plan, kPrefillPlanPieceListInt) + (int64_t)idx * kPrefillPieceInts;
+  const int n = sload(rec, kPrefillPieceCount);
+  if (n <= 1) return true;
+  const int first = sload(rec, kPrefillPieceFirst);
+  const int tid = threadIdx.x;
+  char* const part = (char*)plan + (int64_t)sload(plan, kPrefillPlanPartInt) * kPrefillPartUnit;
+  auto slot = [&](int piece) { return part + ((int64_t)piece * num_heads + head) * kPrefillPartBytes; };
+  {
+    char* const mine = slot(idx);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const f32x4 v = {o[j >> 2][4 * (j & 3)], o[j >> 2][4 * (j & 3) + 1], o[j >> 2][4 * (j & 3) + 2],
+                       o[j >> 2][4 * (j & 3) + 3]};
+      store16_device_untracked(mine + (j * kPrefillPPThreads + tid) * 16, __builtin_bit_cast(u32x4, v));
+    }
+    store8_device_untracked(mine + 16 * 16 * kPrefillPPThreads + tid * 8, __builtin_bit_cast(u32x2, f32x2{m, l}));
+  }
+  __builtin_amdgcn_s_waitcnt(kVmcnt0);
+  __syncthreads();
+  int32_t* const ctr = plan + sload(plan, kPrefillPlanArriveInt) + first * num_heads + head;
+  if (tid == 0) *word = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(*word) != n - 1) return false;
+  if (tid == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  f32x2 ml[kPrefillMaxPieces];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int c = 0; c < kPrefillMaxPieces; ++c) {
+    ml[c] = f32x2{-INFINITY, 0.f};
+    if (c < n) {
+      const __amdgpu_buffer_rsrc_t r =
+          __builtin_amdgcn_make_buffer_rsrc(slot(first + c), 0, kPrefillPartBytes, 0x00027000);
+      ml[c] = part_ld8(r, 16 * 16 * kPrefillPPThreads + tid * 8);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < kPrefillMaxPieces; ++c) mx = fmaxf(mx, ml[c][0]);
+  const float m_use = mx == -INFINITY ? 0.f : mx;
+  l = 0.f;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
+#pragma unroll
+  for (int c = 0; c < kPrefillMaxPieces; ++c) {
+    if (c < n) {
+      const __amdgpu_buffer_rsrc_t r =
+          __builtin_amdgcn_make_buffer_rsrc(slot(first + c), 0, kPrefillPartBytes, 0x00027000);
+      const float w = fast_exp2(ml[c][0] - m_use);  // m = -inf -> 0
+      l += w * ml[c][1];
+      f32x4 v[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = part_ld16(r, (j * kPrefillPPThreads + tid) * 16);
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[j >> 2][4 * (j & 3) + e] += w * v[j][e];
+    }
+  }
+  return true;
+}
+
 // The items one workgroup claims, run back to back by one wave group (kGrp:
 // 0 = waves 0-3, 1 = waves 4-7; a compile-time constant, so that the K and
 // V cache pointers are not a run-time choice, which the compiler would serve
 // by copying the kernel argument block to scratch).  `tiles` holds
 // kPrefillPPBufs K tile buffers then as many V tile buffers
-// (kPrefillTileBytes each); `nextq` holds four LDS words through which
+// (kPrefillTileBytes each); `nextq` holds five LDS words through which
 // thread 0 publishes claimed items: words 0 / 3 the first item's plan
 // index and KV head, words 1 / 2 those of the successor of the item that
-// starts next.
+// starts next; word 4 serves settle_piece.  `rank` is the workgroup's number
+// among those of head h0.
+//
+// kFixed: the launch has at least one workgroup per item of a head, workgroup
+// `rank` of a head runs item `rank` of the piece or tile list and nothing
+// else, and what follows about claims and successors does not apply.
 //
 // Claims: a workgroup of KV head h0 claims from h0's counter.  Once that
 // queue is exhausted it reads every head's counter (one per lane of wave 0)
@@ -94,9 +196,9 @@ typedef __attribute__((address_space(3))) int32_t lds_i32;
 // known: no plan read, query load, copy wait or claim sits between items.
 // Only when A has a single tile does group 1 copy V(B, 0) at B's start
 // (it is first read at B's phase 2, after the wait that ends phase 1).
-template <typename T, int kGrp>
+template <typename T, int kGrp, bool kFixed>
 __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(const PrefillParams& p, int32_t* plan,
-                                                                             int h0, lds_u8* tiles, lds_i32* nextq) {
+                                                                             int h0, int rank, lds_u8* tiles, lds_i32* nextq) {
   typedef typename Elem<T>::v8 V8;
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // 0..7
@@ -106,7 +208,8 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
   const int hi = lane >> 5;
   const int G = p.group;
   const int BMT = p.tile_tokens;  // 256 / G
-  const int n_items = sload(plan, 0);
+  const int n_pieces = kFixed ? sload(plan, kPrefillPlanPiecesInt) : 0;
+  const int n_items = n_pieces > 0 ? n_pieces : sload(plan, 0);
   const int H = p.num_kv_heads;
   auto claim = [&](int head) {
     return __hip_atomic_fetch_add(plan + kPrefillPlanLineInts * (1 + head), 1, __ATOMIC_RELAXED,
@@ -181,7 +284,7 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
   V8 qf[8];
   // Query fragments of item `it` of KV head `kvh` (rows past the sequence or
   // the heads read zeros).
-  auto load_q = [&](const PrefillWork& it, int kvh) __attribute__((always_inline)) {
+  auto load_q = [&](const StreamWork& it, int kvh) __attribute__((always_inline)) {
     const int tq = it.t0 + rr;
     const bool ok = g < G && tq < it.q_len;
     const int row_tok = it.q0 + (ok ? tq : 0);
@@ -226,33 +329,37 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
   };
 
   // Page id of tile `tile` of item `it` at this wave's page slot.
-  auto page_of_item = [&](const PrefillWork& it, int tile) {
-    const int32_t* btp = p.block_tables + (int64_t)it.s * p.bt_stride;
-    const int pg = sload(btp, min(tile * (kPrefillKeys / kPageSize) + slot, it.npages - 1));
+  auto page_of_item = [&](const StreamWork& it, int tile) {
+    const int pg = sload(it.btp, min(tile * (kPrefillKeys / kPageSize) + slot, it.npages - 1));
     return (pg >= 0 && pg < p.num_pages) ? pg : 0;
   };
 
   // ---- the first item ---------------------------------------------------------
   int claim_head = h0;  // wave 0: the head claimed from last
   int claim_ret = 0;    // thread 0: the latest claim
-  if (w == 0) {
-    int r = 0;
-    if (lane == 0) r = claim(h0);
-    r = claim_on(r, claim_head);
-    if (lane == 0) {
-      nextq[0] = r;
-      nextq[3] = claim_head;
+  int idx = rank, cur_h = h0;
+  if constexpr (!kFixed) {
+    if (w == 0) {
+      int r = 0;
+      if (lane == 0) r = claim(h0);
+      r = claim_on(r, claim_head);
+      if (lane == 0) {
+        nextq[0] = r;
+        nextq[3] = claim_head;
+      }
     }
+    __syncthreads();
+    idx = __builtin_amdgcn_readfirstlane(nextq[0]);
+    cur_h = __builtin_amdgcn_readfirstlane(nextq[3]);
   }
-  __syncthreads();
-  int idx = __builtin_amdgcn_readfirstlane(nextq[0]);
   if (idx >= n_items) return;  // uniform: nothing for this workgroup
-  int cur_h = __builtin_amdgcn_readfirstlane(nextq[3]);
-  PrefillWork cur = plan_work_slot(plan, idx, slot);
+  StreamWork cur = plan_work_slot<kFixed>(p, plan, idx, slot);
   // The page of the item's tile 2, which the item's first copies need; for
   // later items it is loaded during the item before (see below).
   int pg2_next = page_of_item(cur, 2);
-  if (tid == 0) claim_ret = claim(claim_head);
+  if constexpr (!kFixed) {
+    if (tid == 0) claim_ret = claim(claim_head);
+  }
   load_q(cur, cur_h);
   if constexpr (kGrp == 0) {
     copy_page(0, cur.pg0, cur_h);
@@ -261,11 +368,13 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     copy_page(0, cur.pg0, cur_h);
   }
   __builtin_amdgcn_s_waitcnt(kVmcnt0);
-  if (w == 0) {
-    const int r = claim_on(claim_ret, claim_head);
-    if (lane == 0) {
-      nextq[1] = r;
-      nextq[2] = claim_head;
+  if constexpr (!kFixed) {
+    if (w == 0) {
+      const int r = claim_on(claim_ret, claim_head);
+      if (lane == 0) {
+        nextq[1] = r;
+        nextq[2] = claim_head;
+      }
     }
   }
   phase_barrier();
@@ -275,9 +384,9 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
   const std::true_type yes;
   const std::false_type no;
   while (true) {
-    const int nidx = __builtin_amdgcn_readfirstlane(nextq[1]);
-    const int nh = __builtin_amdgcn_readfirstlane(nextq[2]);  // B's KV head
-    const bool has_next = nidx < n_items;
+    const int nidx = kFixed ? n_items : __builtin_amdgcn_readfirstlane(nextq[1]);
+    const int nh = kFixed ? cur_h : __builtin_amdgcn_readfirstlane(nextq[2]);  // B's KV head
+    const bool has_next = !kFixed && nidx < n_items;
     const int n = cur.ntiles;
     const int full_tiles = cur.full_tiles;
     const int kv = cur.kv;
@@ -285,10 +394,10 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     const bool row_ok = g < G && tq < cur.q_len;
     const int pos = row_ok ? kv - cur.q_len + tq : -1;  // keys j <= pos are visible
     auto page_of = [&](int tile) { return page_of_item(cur, tile); };
-    PrefillWork nx;  // B's record, loaded at this item's first S phase
+    StreamWork nx;  // B's record, loaded at this item's first S phase
     nx.ntiles = 0;
     auto load_next = [&]() __attribute__((always_inline)) {
-      if (has_next) nx = plan_work_slot(plan, nidx, slot);
+      if (has_next) nx = plan_work_slot<kFixed>(p, plan, nidx, slot);
     };
     if constexpr (kGrp == 1) {
       if (!v0_done) copy_page(G0, cur.pg0, cur_h);
@@ -558,10 +667,17 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     }
     phase_barrier();
 
-    // Epilogue: O^T / l -> out[token][head][d].
-    const float l_tot = pair_sum(l);
+    // Epilogue: O^T / l -> out[token][head][d], of a split tile by the
+    // workgroup that finishes it.
+    float l_tot = pair_sum(l);
+    bool done = true;
+    if constexpr (kFixed) {
+      if (n_pieces > 0) done = settle_piece(plan, idx, cur_h, H, o, m, l_tot, nextq + 4);
+    }
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-    if (p.out16) {
+    if (!done) {
+      // Another piece of the tile is still out.
+    } else if (p.out16) {
       // Staged in this wave's page slot of the K buffer (group 0) or V
       // buffer (group 1) of the item's last tile: the K buffer is next
       // written by this wave's own copy at the next item's phase 0, the V

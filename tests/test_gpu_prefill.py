@@ -431,3 +431,48 @@ def test_split_mixed_route_reuses_the_prefill_plan_across_layers(gpu):
         out = backend.forward(qd, empty, empty, kc, vc, plan).clone()
         assert backend._prefill_planned_for is plan.metadata
         assert_attention_close(out.cpu(), expected(batch))
+
+
+# Few tiles over long contexts: the device plan cuts them into split-K pieces
+# (words 18 / 19 of the plan: their number and the word offset of their list).
+# Key counts at and around multiples of a 64-key tile and of a page, tiles
+# whose last piece is partly past the sequence or wholly masked for some rows,
+# one head and many, and up to the most pieces a tile is cut into.
+@pytest.mark.parametrize("hq,hkv,dtype,q,kv", [
+    (32, 8, torch.bfloat16, [70, 1], [70 + 4096, 1]),
+    (16, 8, torch.float16, [200, 3, 129], [200 + 1900, 3 + 64 * 21, 129]),
+    (8, 1, torch.bfloat16, [64, 33], [64 * 40, 33 + 64 * 32 - 1]),
+    (12, 4, torch.float16, [5], [64 * 30 + 1]),
+    (80, 80, torch.bfloat16, [6], [1500]),
+    (64, 8, torch.bfloat16, [40], [40 + 8192 - 17]),
+])
+def test_split_key_ranges(gpu, hq, hkv, dtype, q, kv):
+    batch = make_paged_batch(211 + hq, q, kv, len(q), hq, hkv, dtype=dtype, extra_pages=1)
+    bt = batch.common.block_tables
+    for s, n in enumerate(kv):  # stale rows of the last page
+        last = int(bt[s, (n - 1) // 16])
+        batch.k_cache[last, (n - 1) % 16 + 1:] = float("nan")
+        batch.v_cache[last, (n - 1) % 16 + 1:] = float("nan")
+    common, qd, kc, vc = to_device(batch, gpu)
+    n_tiles = ops.prefill_max_tiles(sum(q), len(q), hq, hkv)
+    full = ops.prefill_workspace_bytes(n_tiles)
+    plan_only = 4 * (ops.PREFILL_PLAN_HEADER_INTS + n_tiles * ops.PREFILL_PLAN_ITEM_INTS)
+    outs = []
+    for nbytes in (full, full, plan_only):  # without room for partials nothing is split
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
+        for planned in (False, True):
+            out = torch.full_like(qd, float("nan"))
+            ops.paged_prefill(qd, kc, vc, common.block_tables, common.seq_lens, common.query_start_loc, len(q),
+                              n_tiles, ws, out, 128 ** -0.5, planned=planned)
+            outs.append(out)
+        pieces = int(ws[72:76].view(torch.int32).item())
+        cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+        tiles = int(ws[:4].view(torch.int32).item())
+        assert pieces <= min(cus, 256) // hkv
+        assert (pieces > tiles) == (nbytes == full)
+    want = expected(batch)
+    for out in outs:
+        assert_attention_close(out.cpu(), want)
+    # The merge takes a tile's pieces in key order, whichever ends last.
+    assert all(torch.equal(out, outs[0]) for out in outs[:4])
+    assert torch.equal(outs[4], outs[5])
