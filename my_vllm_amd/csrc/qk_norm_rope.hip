@@ -14,9 +14,10 @@
 // Queries and keys are written to their output rows (which may alias the
 // inputs); V is only copied into the cache.
 //
-// Sixteen lanes per (token, head) row of q, k or v; each lane owns four
-// elements of each half of the 128-wide head, so the pairs the rotation mixes
-// sit in one lane and the norm's sum of squares is the only cross-lane step.
+// Eight lanes per (token, head) row of q, k or v (sixteen when the buffers are
+// only 8-byte aligned); each lane owns eight (four) elements of each half of
+// the 128-wide head, so the pairs the rotation mixes sit in one lane and the
+// norm's sum of squares is the only cross-lane step.
 #include "mva_capi.h"
 #include "mva_common.h"
 
@@ -51,37 +52,37 @@ struct PrologueArgs {
   int64_t num_tokens;
 };
 
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct Vec4;
-template <>
-struct Vec4<__bf16> {
-  typedef __bf16 type __attribute__((ext_vector_type(4)));
+template <typename T, int kPer>
+struct VecOf {
+  typedef T type __attribute__((ext_vector_type(kPer)));
 };
-template <>
-struct Vec4<_Float16> {
-  typedef _Float16 type __attribute__((ext_vector_type(4)));
+template <int kPer>
+struct FloatsOf {
+  typedef float type __attribute__((ext_vector_type(kPer)));
 };
 
-template <typename W>
-__device__ inline f32x4v load_w4(const void* w, int i) {
-  if constexpr (sizeof(W) == 4) {
-    return *reinterpret_cast<const f32x4v*>((const float*)w + i);
-  } else {
-    const typename Vec4<W>::type v = *reinterpret_cast<const typename Vec4<W>::type*>((const W*)w + i);
-    return f32x4v{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+// kPer elements as fp32, 16 bytes of them aligned.
+template <typename W, int kPer>
+__device__ inline typename FloatsOf<kPer>::type load_w(const void* w, int64_t i) {
+  constexpr int kStep = sizeof(W) == 4 ? 4 : kPer;
+  typename FloatsOf<kPer>::type f;
+#pragma unroll
+  for (int s = 0; s < kPer; s += kStep) {
+    const typename VecOf<W, kStep>::type v = *reinterpret_cast<const typename VecOf<W, kStep>::type*>((const W*)w + i + s);
+#pragma unroll
+    for (int e = 0; e < kStep; ++e) f[s + e] = (float)v[e];
   }
+  return f;
 }
 
 // Rows r of a token: [0, Hq) queries, [Hq, Hq + Hkv) keys, then (with a
-// store) [Hq + Hkv, Hq + 2 Hkv) values; a quad is four consecutive rows.
-// Within a quad the 16 lanes of group g = lane / 16 own row 4q + g; lane
-// c = lane % 16 holds elements 4c .. 4c+3 of the first half of the head and
-// 64 + 4c .. 64 + 4c + 3 of the second (the pairs the rotation mixes),
-// loaded and stored 8 bytes at a time.
+// store) [Hq + Hkv, Hq + 2 Hkv) values; a set is kPer consecutive rows.
+// Within a set the 64 / kPer lanes of group g own row kPer * set + g; lane
+// c of a group holds elements kPer * c .. + kPer - 1 of the first half of the
+// head and the same of the second (the pairs the rotation mixes), 2 * kPer
+// bytes a load or store.
 //
-// A wavefront takes one item at a time: up to kChunk quads of one token.
+// A wavefront takes one item at a time: up to kChunk sets of one token.
 // The token is uniform over the wavefront, so its position and slot are
 // two loads, and the item issues them, then every row load, then (once the
 // position is in) the one cos / sin row all its rows share: two memory
@@ -89,44 +90,46 @@ __device__ inline f32x4v load_w4(const void* w, int i) {
 // position, then the cos / sin row, then the data, and the compiler cannot
 // hoist the next row's loads above this row's stores, since the outputs
 // may alias the inputs.  Distinct rows never overlap, so reading an item's
-// rows before writing any of them is exact even in place.
-constexpr int kChunk = 6;
-
-template <typename T, typename W, typename SlotT>
+// rows before writing any of them is exact even in place.  The q / k outputs
+// are stored non-temporally (the launch does not read them again): 3 us of
+// 4000 tokens at 32 / 8 heads.
+template <typename T, typename W, typename SlotT, int kPer, int kChunk>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(PrologueArgs a) {
   // Separate fp32 multiplies and adds, as torch evaluates the rotation (no
   // fused multiply-add contraction).
 #pragma clang fp contract(off)
-  typedef typename Vec4<T>::type V4;
+  typedef typename VecOf<T, kPer>::type V;
+  typedef typename FloatsOf<kPer>::type F;
+  constexpr int kLanes = 64 / kPer;  // lanes per row
   const int lane = threadIdx.x & 63;
-  const int g = lane >> 4;
-  const int c4 = 4 * (lane & 15);
+  const int g = lane / kLanes;
+  const int c0 = kPer * (lane % kLanes);
   const int hqk = a.num_q_heads + a.num_kv_heads;
   const bool store = a.k_cache != nullptr;
   const int R = hqk + (store ? a.num_kv_heads : 0);
-  const int nq = (R + 3) / 4;
-  const int S = (nq + kChunk - 1) / kChunk;  // items per token
+  const int sets = (R + kPer - 1) / kPer;
+  const int S = (sets + kChunk - 1) / kChunk;  // items per token
   const int64_t waves = (int64_t)gridDim.x * 4;
   const bool norm = a.q_norm_w != nullptr;
-  f32x4v wq1{}, wq2{}, wk1{}, wk2{};
+  F wq1{}, wq2{}, wk1{}, wk2{};
   if (norm) {
-    wq1 = load_w4<W>(a.q_norm_w, c4);
-    wq2 = load_w4<W>(a.q_norm_w, 64 + c4);
-    wk1 = load_w4<W>(a.k_norm_w, c4);
-    wk2 = load_w4<W>(a.k_norm_w, 64 + c4);
+    wq1 = load_w<W, kPer>(a.q_norm_w, c0);
+    wq2 = load_w<W, kPer>(a.q_norm_w, 64 + c0);
+    wk1 = load_w<W, kPer>(a.k_norm_w, c0);
+    wk2 = load_w<W, kPer>(a.k_norm_w, 64 + c0);
   }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   for (int64_t it = (int64_t)blockIdx.x * 4 + wave; it < a.num_tokens * S; it += waves) {
-    const int64_t t = it / S;
-    const int j0 = (int)(it - t * S) * kChunk;  // this item's quads [j0, j0 + kChunk) within [0, nq)
+    const int64_t t = it >> 31 ? it / S : (int64_t)((uint32_t)it / (uint32_t)S);
+    const int j0 = (int)(it - t * S) * kChunk;  // this item's sets [j0, j0 + kChunk) within [0, sets)
     // Without a store the slot pointer is the positions (a valid int64
     // array of the same length) and the value goes unused.
     const int64_t pos_in = a.positions[t];
     const int64_t slot_in = (int64_t)((const SlotT*)a.slots)[t];
-    V4 lo[kChunk], hi[kChunk];
+    V lo[kChunk], hi[kChunk];
 #pragma unroll
     for (int k = 0; k < kChunk; ++k) {
-      int r = 4 * (j0 + k) + g;
+      int r = kPer * (j0 + k) + g;
       r = r < R ? r : 0;  // rows past the token read row 0 and are not written
       const T* src;
       if (r >= hqk)
@@ -135,91 +138,105 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(PrologueArgs a)
         src = (const T*)a.q_in + t * a.q_tok_stride + r * a.q_head_stride;
       else
         src = (const T*)a.k_in + t * a.k_tok_stride + (r - a.num_q_heads) * a.k_head_stride;
-      lo[k] = *reinterpret_cast<const V4*>(src + c4);
-      hi[k] = *reinterpret_cast<const V4*>(src + 64 + c4);
+      lo[k] = *reinterpret_cast<const V*>(src + c0);
+      hi[k] = *reinterpret_cast<const V*>(src + 64 + c0);
     }
     const int64_t pos = pos_in < 0 ? 0 : (pos_in >= a.max_position ? a.max_position - 1 : pos_in);  // stay in bounds
-    const f32x4v cs = *reinterpret_cast<const f32x4v*>(a.cos_sin + pos * kRopeDim + c4);
-    const f32x4v sn = *reinterpret_cast<const f32x4v*>(a.cos_sin + pos * kRopeDim + 64 + c4);
+    const F cs = load_w<float, kPer>(a.cos_sin, pos * kRopeDim + c0);
+    const F sn = load_w<float, kPer>(a.cos_sin, pos * kRopeDim + 64 + c0);
     const int64_t slot = (store && slot_in < a.num_slots) ? slot_in : -1;  // negative: skipped
     const int64_t cache_row = (slot >= 0) ? slot * a.num_kv_heads : 0;  // rows of [slots * Hkv, 128]
 #pragma unroll
     for (int k = 0; k < kChunk; ++k) {
-      const int r = 4 * (j0 + k) + g;
-      if (r >= R) continue;  // a whole 16-lane group: no shuffle partner is lost
+      const int r = kPer * (j0 + k) + g;
+      if (r >= R) continue;  // a whole group of lanes: no shuffle partner is lost
       if (r >= hqk) {  // V: copy into the cache
         if (slot >= 0) {
           T* dst = (T*)a.v_cache + (cache_row + r - hqk) * kRopeDim;
-          *reinterpret_cast<V4*>(dst + c4) = lo[k];
-          *reinterpret_cast<V4*>(dst + 64 + c4) = hi[k];
+          *reinterpret_cast<V*>(dst + c0) = lo[k];
+          *reinterpret_cast<V*>(dst + 64 + c0) = hi[k];
         }
         continue;
       }
       const bool is_q = r < a.num_q_heads;
       const int h = is_q ? r : r - a.num_q_heads;
-      float x1[4], x2[4];
+      float x1[kPer], x2[kPer];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
+      for (int e = 0; e < kPer; ++e) {
         x1[e] = (float)lo[k][e];
         x2[e] = (float)hi[k][e];
       }
       if (norm) {
         float ss = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ss += x1[e] * x1[e] + x2[e] * x2[e];
+        for (int e = 0; e < kPer; ++e) ss += x1[e] * x1[e] + x2[e] * x2[e];
 #pragma unroll
-        for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off);  // within the 16-lane group
+        for (int off = kLanes / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);  // within the row's lanes
         const float rs = 1.0f / __builtin_sqrtf(ss / (float)kRopeDim + a.eps);
-        const f32x4v w1 = is_q ? wq1 : wk1;
-        const f32x4v w2 = is_q ? wq2 : wk2;
+        const F w1 = is_q ? wq1 : wk1;
+        const F w2 = is_q ? wq2 : wk2;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < kPer; ++e) {
           x1[e] = (float)(T)((float)(T)(x1[e] * rs) * w1[e]);
           x2[e] = (float)(T)((float)(T)(x2[e] * rs) * w2[e]);
         }
       }
-      V4 y1, y2;
+      V y1, y2;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
+      for (int e = 0; e < kPer; ++e) {
         y1[e] = (T)(x1[e] * cs[e] - x2[e] * sn[e]);
         y2[e] = (T)(x2[e] * cs[e] + x1[e] * sn[e]);
       }
       T* dst = is_q ? (T*)a.q_out + t * a.q_tok_stride + h * a.q_head_stride
                     : (T*)a.k_out + t * a.k_tok_stride + h * a.k_head_stride;
-      *reinterpret_cast<V4*>(dst + c4) = y1;
-      *reinterpret_cast<V4*>(dst + 64 + c4) = y2;
+      __builtin_nontemporal_store(y1, reinterpret_cast<V*>(dst + c0));
+      __builtin_nontemporal_store(y2, reinterpret_cast<V*>(dst + 64 + c0));
       if (!is_q && slot >= 0) {
         T* kd = (T*)a.k_cache + (cache_row + h) * kRopeDim;
-        *reinterpret_cast<V4*>(kd + c4) = y1;
-        *reinterpret_cast<V4*>(kd + 64 + c4) = y2;
+        *reinterpret_cast<V*>(kd + c0) = y1;
+        *reinterpret_cast<V*>(kd + 64 + c0) = y2;
       }
     }
   }
 }
-
-template <typename T, typename W>
-void launch_prologue_kernel(PrologueArgs a, int64_t blocks, hipStream_t s) {
+template <typename T, typename W, int kPer, int kChunk>
+void launch_prologue_kernel(PrologueArgs a, hipStream_t s) {
+  const int rows = a.num_q_heads + a.num_kv_heads + (a.k_cache != nullptr ? a.num_kv_heads : 0);
+  const int64_t items = a.num_tokens * (((rows + kPer - 1) / kPer + kChunk - 1) / kChunk);
+  // Four wavefronts per workgroup; at most 16 workgroups per CU's worth,
+  // beyond which the wavefronts loop.
+  const uint32_t blocks = (uint32_t)std::min<int64_t>((items + 3) / 4, 256 * 16);
   if (a.k_cache == nullptr) {
     a.slots = a.positions;
-    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, W, int64_t>), dim3((uint32_t)blocks), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, W, int64_t, kPer, kChunk>), dim3(blocks), dim3(256), 0, s, a);
   } else if (a.slot_is_int64) {
-    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, W, int64_t>), dim3((uint32_t)blocks), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, W, int64_t, kPer, kChunk>), dim3(blocks), dim3(256), 0, s, a);
   } else {
-    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, W, int32_t>), dim3((uint32_t)blocks), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((qk_norm_rope_store_kernel<T, W, int32_t, kPer, kChunk>), dim3(blocks), dim3(256), 0, s, a);
   }
 }
 
-template <typename T>
-int launch_prologue(const PrologueArgs& a, int weight_dtype, hipStream_t s) {
+// Sixteen-byte accesses where the alignment allows: one set of rows per item
+// while that leaves no more items than 4 wavefronts per SIMD (the item's two
+// memory round trips are then the launch), two beyond (the position, the cos /
+// sin row and the weights serve twice the rows; three and six sets measured the
+// same or slower).  Four launches of a layer (norms, this kernel, SiLU),
+// with this kernel at 8 bytes a lane and six sets and the norms one wavefront
+// a row / as they are: 61 tokens 18.8 / 10.1 us, 512 tokens 33.5 / 21.1 us, 4000
+// tokens 124.1 / 108.2 us at hidden 4096, 32 / 8 heads; 8 tokens 12.8 / 9.1 us at
+// hidden 1024, 16 / 8 heads.
+template <typename T, typename W>
+void pick_prologue_kernel(const PrologueArgs& a, bool wide, hipStream_t s) {
   const int rows = a.num_q_heads + a.num_kv_heads + (a.k_cache != nullptr ? a.num_kv_heads : 0);
-  const int64_t items = a.num_tokens * (((rows + 3) / 4 + kChunk - 1) / kChunk);
-  // Four wavefronts per workgroup; at most 16 workgroups per CU's worth,
-  // beyond which the wavefronts loop.
-  const int64_t blocks = std::min<int64_t>((items + 3) / 4, 256 * 16);
-  if (weight_dtype == kF32)
-    launch_prologue_kernel<T, float>(a, blocks, s);
-  else
-    launch_prologue_kernel<T, T>(a, blocks, s);
+  if (!wide) launch_prologue_kernel<T, W, 4, 6>(a, s);
+  else if (a.num_tokens * ((rows + 7) / 8) <= 4096) launch_prologue_kernel<T, W, 8, 1>(a, s);
+  else launch_prologue_kernel<T, W, 8, 2>(a, s);
+}
+
+template <typename T>
+int launch_prologue(const PrologueArgs& a, int weight_dtype, bool wide, hipStream_t s) {
+  if (weight_dtype == kF32) pick_prologue_kernel<T, float>(a, wide, s);
+  else pick_prologue_kernel<T, T>(a, wide, s);
   return check_launch("qk_norm_rope_store");
 }
 
@@ -262,8 +279,9 @@ extern "C" int mva_qk_norm_rope_store(const void* q_in, void* q_out, int64_t q_t
                  v, v_token_stride, v_head_stride, num_q_heads, num_kv_heads, positions, cos_sin_cache,
                  max_position, q_norm_weight, k_norm_weight, eps, k_cache, v_cache, num_slots, slot_mapping,
                  slot_is_int64, num_tokens};
+  const bool wide = align % 16 == 0;  // the cos / sin rows and the weights are 16-byte aligned either way
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == kBF16) return launch_prologue<__bf16>(a, weight_dtype, s);
-  if (dtype == kF16) return launch_prologue<_Float16>(a, weight_dtype, s);
+  if (dtype == kBF16) return launch_prologue<__bf16>(a, weight_dtype, wide, s);
+  if (dtype == kF16) return launch_prologue<_Float16>(a, weight_dtype, wide, s);
   return set_error("qk_norm_rope: dtype must be bf16 or fp16");
 }

@@ -10,11 +10,10 @@
 // product is rounded again (torch multiplies two T tensors in fp32 and rounds
 // once).  `w` is T or fp32.
 //
-// HBM-bound: one wavefront per row (four rows per 256-thread workgroup); each
-// lane keeps its 16-byte chunks of the row in registers between the sum of
-// squares and the output, so a row is read once and written once, and an
-// in-place call (out == x, residual_out == residual) is safe: every element is
-// read before any element of its row is written.
+// HBM-bound: each lane keeps its 16-byte chunks of a row in registers between
+// the sum of squares and the output, so a row is read once and written once,
+// and an in-place call (out == x, residual_out == residual) is safe: every
+// element is read before any element of its row is written.
 #include "mva_capi.h"
 #include "mva_common.h"
 
@@ -42,8 +41,11 @@ struct RmsArgs {
   int64_t out_group_stride;
 };
 
+// Rows and rows per group below 2^31 (the usual case) divide in 32 bits: a
+// 64-bit division is about a hundred instructions at the start of every row.
 __device__ inline int64_t row_offset(int64_t r, int64_t per_group, int64_t group_stride, int64_t stride) {
-  const int64_t g = r / per_group;
+  const bool narrow = ((uint64_t)r | (uint64_t)per_group) >> 31 == 0;
+  const int64_t g = narrow ? (int64_t)((uint32_t)r / (uint32_t)per_group) : r / per_group;
   return g * group_stride + (r - g * per_group) * stride;
 }
 
@@ -78,56 +80,76 @@ __device__ inline void load_w8<_Float16>(const _Float16* w, float (&f)[8]) {
   for (int i = 0; i < 8; ++i) f[i] = (float)a[i];
 }
 
-// Vector path: hidden % 8 == 0, 16-byte aligned rows, hidden <= 512 * kChunks
-// (at most 8192: larger rows take the scalar path).
-template <typename T, typename W, int kChunks, bool kAdd>
-__global__ __launch_bounds__(256) void rms_norm_vec_kernel(RmsArgs a) {
+// Vector path: hidden % 8 == 0, 16-byte aligned rows, hidden <= 512 * kWaves *
+// kChunks (at most 8192: larger rows take the scalar path).  kWaves 1: four
+// rows per workgroup, a wavefront each.  kWaves > 1: a workgroup of kWaves
+// wavefronts per row, whose partial sums meet in LDS.  The row, the residual
+// and the weight are all requested before the sum, one memory round trip.
+template <typename T, typename W, int kWaves, int kChunks, bool kAdd>
+__global__ __launch_bounds__(kWaves == 1 ? 256 : 64 * kWaves) void rms_norm_vec_kernel(RmsArgs a) {
   typedef typename Elem<T>::v8 V;
+  __shared__ float part[kWaves];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = kWaves == 1 ? (int64_t)blockIdx.x * 4 + w : (int64_t)blockIdx.x;
   if (row >= a.rows) return;
+  const int j0 = kWaves == 1 ? lane : (int)threadIdx.x;
   const int nvec = a.hidden >> 3;
-  const T* xr = (const T*)a.x + row_offset(row, a.rows_per_group, a.x_group_stride, a.x_stride);
+  const T* xr = (const T*)a.x +
+                (kAdd ? row * a.x_stride : row_offset(row, a.rows_per_group, a.x_group_stride, a.x_stride));
   const T* rr = kAdd ? (const T*)a.residual + row * a.res_stride : nullptr;
+  const W* wp = (const W*)a.weight;
+  V xv[kChunks], rv[kChunks];
+  float wf[kChunks][8];
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const int j = j0 + 64 * kWaves * c;
+    if (j < nvec) {
+      xv[c] = *reinterpret_cast<const V*>(xr + 8 * j);
+      if constexpr (kAdd) rv[c] = *reinterpret_cast<const V*>(rr + 8 * j);
+      load_w8<W>(wp + 8 * j, wf[c]);
+    }
+  }
   float v[kChunks][8];
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < kChunks; ++c) {
-    const int j = lane + 64 * c;
-    if (j < nvec) {
-      const V xv = *reinterpret_cast<const V*>(xr + 8 * j);
-      V rv;
-      if constexpr (kAdd) rv = *reinterpret_cast<const V*>(rr + 8 * j);
+    if (j0 + 64 * kWaves * c < nvec) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        float f = (float)xv[i];
-        if constexpr (kAdd) f += (float)rv[i];
+        float f = (float)xv[c][i];
+        if constexpr (kAdd) f += (float)rv[c][i];
         v[c][i] = f;
         ss += f * f;
       }
     }
   }
   ss = wave_sum(ss);
+  if constexpr (kWaves > 1) {
+    if (lane == 0) part[w] = ss;
+    __syncthreads();
+    ss = part[0];
+#pragma unroll
+    for (int k = 1; k < kWaves; ++k) ss += part[k];
+  }
   const float r = 1.0f / __builtin_sqrtf(ss / (float)a.hidden + a.eps);
-  T* orow = (T*)a.out + row_offset(row, a.rows_per_group, a.out_group_stride, a.out_stride);
+  T* orow = (T*)a.out +
+            (kAdd ? row * a.out_stride : row_offset(row, a.rows_per_group, a.out_group_stride, a.out_stride));
   T* ro = kAdd ? (T*)a.residual_out + row * a.res_out_stride : nullptr;
-  const W* w = (const W*)a.weight;
 #pragma unroll
   for (int c = 0; c < kChunks; ++c) {
-    const int j = lane + 64 * c;
+    const int j = j0 + 64 * kWaves * c;
     if (j < nvec) {
-      float wf[8];
-      load_w8<W>(w + 8 * j, wf);
       V o;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = (T)((float)(T)(v[c][i] * r) * wf[i]);
+      for (int i = 0; i < 8; ++i) o[i] = (T)((float)(T)(v[c][i] * r) * wf[c][i]);
       if constexpr (kAdd) {
         V s;
 #pragma unroll
         for (int i = 0; i < 8; ++i) s[i] = (T)v[c][i];
-        *reinterpret_cast<V*>(ro + 8 * j) = s;
+        __builtin_nontemporal_store(s, reinterpret_cast<V*>(ro + 8 * j));
       }
-      *reinterpret_cast<V*>(orow + 8 * j) = o;
+      __builtin_nontemporal_store(o, reinterpret_cast<V*>(orow + 8 * j));
     }
   }
 }
@@ -161,6 +183,13 @@ __global__ __launch_bounds__(256) void rms_norm_scalar_kernel(RmsArgs a) {
   }
 }
 
+template <typename T, typename W, bool kAdd, int kWaves, int kChunks>
+void launch_vec(const RmsArgs& a, hipStream_t s) {
+  const uint32_t blocks = (uint32_t)(kWaves == 1 ? (a.rows + 3) / 4 : a.rows);
+  hipLaunchKernelGGL((rms_norm_vec_kernel<T, W, kWaves, kChunks, kAdd>), dim3(blocks),
+                     dim3(kWaves == 1 ? 256 : 64 * kWaves), 0, s, a);
+}
+
 template <typename T, typename W, bool kAdd>
 int launch_rms(const RmsArgs& a, hipStream_t s) {
   const int64_t blocks = (a.rows + 3) / 4;
@@ -174,13 +203,17 @@ int launch_rms(const RmsArgs& a, hipStream_t s) {
     bits |= (uint64_t)(uintptr_t)a.residual | (uint64_t)(uintptr_t)a.residual_out |
             (uint64_t)(a.res_stride * (int64_t)sizeof(T)) | (uint64_t)(a.res_out_stride * (int64_t)sizeof(T));
   const int nvec = a.hidden / 8;
-  if (a.hidden % 8 == 0 && bits % 16 == 0 && nvec <= 64 * 16) {
-    const int chunks = (nvec + 63) / 64;
-    if (chunks <= 1) hipLaunchKernelGGL((rms_norm_vec_kernel<T, W, 1, kAdd>), grid, block, 0, s, a);
-    else if (chunks <= 2) hipLaunchKernelGGL((rms_norm_vec_kernel<T, W, 2, kAdd>), grid, block, 0, s, a);
-    else if (chunks <= 4) hipLaunchKernelGGL((rms_norm_vec_kernel<T, W, 4, kAdd>), grid, block, 0, s, a);
-    else if (chunks <= 8) hipLaunchKernelGGL((rms_norm_vec_kernel<T, W, 8, kAdd>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((rms_norm_vec_kernel<T, W, 16, kAdd>), grid, block, 0, s, a);
+  if (a.hidden % 8 == 0 && bits % 16 == 0 && nvec <= 64 * 16 && (nvec <= 64 || a.rows <= 0x7fffffffLL)) {
+    // One 16-byte chunk a lane up to 8 wavefronts a row, two beyond.  One
+    // wavefront a row with 8 chunks a lane (hidden 4096) left 61 rows on 16 CUs
+    // (6.2 us a launch) and read and wrote 4096 rows in two separate bursts (33 us):
+    // see pick_prologue_kernel for a layer's launches.  Non-temporal stores:
+    // 110.4 against 120.9 us for those of 4000 tokens.
+    if (nvec <= 64) launch_vec<T, W, kAdd, 1, 1>(a, s);
+    else if (nvec <= 128) launch_vec<T, W, kAdd, 2, 1>(a, s);
+    else if (nvec <= 256) launch_vec<T, W, kAdd, 4, 1>(a, s);
+    else if (nvec <= 512) launch_vec<T, W, kAdd, 8, 1>(a, s);
+    else launch_vec<T, W, kAdd, 8, 2>(a, s);
   } else {
     hipLaunchKernelGGL((rms_norm_scalar_kernel<T, W, kAdd>), grid, block, 0, s, a);
   }

@@ -152,3 +152,30 @@ def test_prologue_strided_slot_mapping_and_host_slots(gpu):
     idx = slots.long()
     assert torch.equal(kc[idx], rope(k, pos, table)) and torch.equal(vc[idx], v)
     assert bool((kc[idx - 1] == 0).all())  # the even slots the view skips stay untouched
+
+
+# Buffers at 16-byte and at only 8-byte alignment take kernels of other access
+# widths, and the item size changes past 4096 sets of eight rows (682 tokens at
+# 32 / 8 heads): RoPE and the store stay bit-exact in all of them.
+@pytest.mark.parametrize("shift", [0, 4])
+@pytest.mark.parametrize("tokens,hq,hkv", [(682, 32, 8), (683, 32, 8), (3, 10, 1), (1400, 12, 3)])
+def test_prologue_alignment_and_item_sizes(gpu, shift, tokens, hq, hkv):
+    qkv, pos = _packed(tokens, hq, hkv, 28)
+    table = rope_cos_sin_cache(128, 4096, 1e6)
+    q, k, v = _views(qkv, hq, hkv)
+    flat = torch.empty(qkv.numel() + 8, dtype=qkv.dtype, device=gpu)
+    buf = flat[shift:shift + qkv.numel()].view(qkv.shape)
+    buf.copy_(qkv.to(gpu))
+    assert (buf.data_ptr() % 16 == 0) == (shift == 0)
+    num_slots = ((tokens + 15) // 16) * 16
+    slots = torch.randperm(num_slots, generator=torch.Generator().manual_seed(29))[:tokens].to(torch.int32)
+    k_cache = torch.full((num_slots // 16, 16, hkv, 128), 7.0, dtype=torch.bfloat16, device=gpu)
+    v_cache = torch.full_like(k_cache, 7.0)
+    qd, kd, vd = _views(buf, hq, hkv)
+    got_q, got_k = ops.qk_norm_rope_store(pos.to(gpu), qd, kd, table.to(gpu), None, None, 1e-6,
+                                          vd, k_cache, v_cache, slots.to(gpu))
+    exp_k = rope(k, pos, table)
+    assert torch.equal(got_q.cpu(), rope(q, pos, table)) and torch.equal(got_k.cpu(), exp_k)
+    idx = slots.long()
+    assert torch.equal(k_cache.cpu().view(-1, hkv, 128)[idx], exp_k)
+    assert torch.equal(v_cache.cpu().view(-1, hkv, 128)[idx], v)

@@ -126,3 +126,16 @@ def test_rms_norm_of_head_views_of_a_packed_projection(gpu):
     with torch.no_grad():
         norm.weight.copy_(w)
     assert_rms_matches(norm(qd), q.float(), w, 1e-6)
+
+
+# Widths at the edges of the wavefronts a row gets (512, 1024, 2048, 4096
+# elements) and 16-byte chunks that only some lanes hold, in place and not.
+@pytest.mark.parametrize("hidden", [504, 512, 520, 1024, 1032, 2048, 2056, 4096, 4104, 8184])
+@pytest.mark.parametrize("inplace", [False, True])
+def test_wavefronts_per_row(gpu, hidden, inplace):
+    x, r, w = _inputs((5, hidden), torch.bfloat16, torch.bfloat16, 13)
+    _, exp_res = fused_add_rms_norm(x, r, w, 1e-6)
+    out, res = ops.fused_add_rms_norm(x.to(gpu), r.to(gpu), w.to(gpu), 1e-6, inplace=inplace)
+    assert torch.equal(res.cpu(), exp_res)
+    assert_rms_matches(out, x.float() + r.float(), w, 1e-6)
+    assert_rms_matches(ops.rms_norm(x.to(gpu), w.to(gpu), 1e-6), x.float(), w, 1e-6)
