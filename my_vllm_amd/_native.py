@@ -9,12 +9,17 @@ the build command, so a GPU run can never silently use another implementation.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 from pathlib import Path
+from types import ModuleType
 
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libmy_vllm_amd.so"
+# CPython module over the same library: the operators' launch path.
+HOST_PATH = LIB_PATH.parent / "mva_host.so"
 
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1}
 # Weight element codes of the RMSNorm entry points (MVA_DTYPE_F32 = 2).
@@ -187,6 +192,7 @@ ABI_VERSION = 11
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 _load_error: Exception | None = None
+_host: ModuleType | None = None
 
 
 def load_library() -> ctypes.CDLL:
@@ -233,6 +239,29 @@ def load_library() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = lib
         return lib
+
+
+def host_ops() -> ModuleType:
+    """The native launch path (csrc/host_ops.cpp), loaded once; RuntimeError if
+    it is missing or of another ABI revision."""
+    global _host
+    if _host is not None:
+        return _host
+    load_library()  # the module binds to the library already in the process
+    rebuild = "build it with `python -m my_vllm_amd.build`"
+    if not HOST_PATH.exists():
+        raise RuntimeError(f"my_vllm_amd native library is missing ({HOST_PATH}); {rebuild}")
+    loader = importlib.machinery.ExtensionFileLoader("mva_host", str(HOST_PATH))
+    try:
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mva_host", loader))
+        loader.exec_module(module)
+    except ImportError as error:
+        raise RuntimeError(f"cannot load {HOST_PATH}: {error}; {rebuild}") from error
+    if module.ABI_VERSION != ABI_VERSION:
+        raise RuntimeError(f"{HOST_PATH} has C ABI revision {module.ABI_VERSION}, this package expects "
+                           f"{ABI_VERSION}; re{rebuild}")
+    _host = module
+    return module
 
 
 def native_available() -> bool:

@@ -805,6 +805,9 @@ class MI355XAttentionBackendMixin:
 
     # ---- forward ------------------------------------------------------------------
     def _validate_inputs(self, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
+        if _native.host_ops().forward_inputs_ok(q, k_cache, v_cache, _native.DTYPE_CODES[self.dtype],
+                                                self.num_q_heads, self.num_kv_heads, self.head_dim, self.block_size):
+            return
         if q.device.type != "cuda" or q.dtype != self.dtype:
             raise ValueError("query must be a CUDA tensor with the backend dtype")
         if q.ndim != 3 or q.shape[1:] != (self.num_q_heads, self.head_dim):

@@ -2,7 +2,8 @@
 
 Every ``csrc/*.hip`` translation unit is compiled with ``hipcc`` for gfx950
 only and linked into one shared library that exports the ``extern "C"`` entry
-points declared in ``include/my_vllm_amd.h``.  The library is built in-tree so
+points declared in ``include/my_vllm_amd.h``; ``csrc/host_ops.cpp`` becomes
+``lib/mva_host.so``, the Python operators' launch path over it.  The library is built in-tree so
 that it travels with the source tree; no JIT cache is involved.
 
 Run ``python -m my_vllm_amd.build`` (or ``__graft_entry__.build()``).
@@ -14,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -67,6 +69,34 @@ def _compile(hipcc: str, source: Path, obj: Path) -> None:
         )
 
 
+def _build_host_module() -> None:
+    """Compile ``csrc/host_ops.cpp`` (host code only) against torch's headers
+    into ``lib/mva_host.so``, bound to the library beside it."""
+    import torch
+
+    from . import _native
+
+    root = Path(torch.__file__).resolve().parent
+    target = _native.HOST_PATH
+    fd, tmp = tempfile.mkstemp(prefix=".mva_host.", suffix=".so.tmp", dir=LIB_DIR)
+    os.close(fd)
+    cmd = [
+        os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++") or "g++",
+        "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+        "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-DMVA_HOST_ABI_VERSION={_native.ABI_VERSION}",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f"-I{root / 'include'}", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
+        str(CSRC_DIR / "host_ops.cpp"), "-o", tmp,
+        f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+        f"-L{LIB_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN",
+    ]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        os.unlink(tmp)
+        raise RuntimeError(f"{cmd[0]} failed for host_ops.cpp:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, target)
+
+
 def build(verbose: bool = False) -> Path:
     """Compile all kernels for gfx950 and link the shared library; return its path."""
     hipcc = _hipcc()
@@ -87,6 +117,7 @@ def build(verbose: bool = False) -> Path:
         os.unlink(tmp)
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, LIB_PATH)
+    _build_host_module()
     if verbose:
         print(f"built {LIB_PATH} from {len(sources)} sources", file=sys.stderr)
     return LIB_PATH

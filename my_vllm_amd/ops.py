@@ -3,9 +3,16 @@
 Each function checks shapes, dtypes, devices and layout on the host, with the
 reference's exception classes and messages, then launches the kernel on
 torch's current stream.  None of them synchronizes or reads device memory.
+
+The common form of a call is checked and launched by the native module
+(``_native.host_ops``, csrc/host_ops.cpp), which returns None, having done
+nothing, for every other: the checks below then raise, or launch through
+ctypes.
 """
 
 from __future__ import annotations
+
+import functools
 
 import torch
 
@@ -35,6 +42,9 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     (csrc/silu_and_mul.cpp:8-18); an empty input gives an empty output
     (csrc/silu_and_mul_kernel.cu:61-63).
     """
+    fast = _native.host_ops().silu_and_mul(x)
+    if fast is not None:
+        return fast
     if not x.is_cuda:
         raise RuntimeError("silu_and_mul expects a CUDA tensor")
     if not x.is_contiguous():
@@ -105,6 +115,10 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tenso
     slice of a packed qkv projection (the reference's q_norm input); the
     result is a new contiguous tensor unless ``out`` is given.
     """
+    if out is None:
+        fast = _native.host_ops().rms_norm(x, weight, eps)
+        if fast is not None:
+            return fast
     hidden = weight.numel()
     _check_rows("rms_norm", x, hidden)
     if weight.dtype not in (x.dtype, torch.float32) or not weight.is_contiguous() or weight.device != x.device:
@@ -136,6 +150,9 @@ def fused_add_rms_norm(
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """``(rms_norm(x + residual), x + residual)`` (reference layernorm.py:42-52);
     ``inplace`` writes them into ``x`` and ``residual``."""
+    fast = _native.host_ops().fused_add_rms_norm(x, residual, weight, eps, inplace)
+    if fast is not None:
+        return fast
     hidden = weight.numel()
     _check_rows("fused_add_rms_norm", x, hidden)
     if residual.shape != x.shape or residual.dtype != x.dtype or residual.device != x.device:
@@ -193,6 +210,10 @@ def qk_norm_rope_store(
     ``cos_sin_cache`` is the RotaryEmbedding buffer, ``[max_pos, (1,) 128]``
     fp32 (cos | sin); ``positions`` int64 ``[T]``.  Returns ``(q_out, k_out)``.
     """
+    if k_cache is not None and _native.host_ops().qk_norm_rope_store(
+            positions, q, k, cos_sin_cache, q_norm_weight, k_norm_weight, eps, v, k_cache, v_cache, slot_mapping,
+            q if q_out is None else q_out, k if k_out is None else k_out):
+        return q if q_out is None else q_out, k if k_out is None else k_out
     if not q.is_cuda:
         raise RuntimeError("qk_norm_rope_store expects CUDA tensors")
     dtype, device = q.dtype, q.device
@@ -335,6 +356,7 @@ def store_kvcache(
     )
 
 
+@functools.lru_cache(maxsize=256)
 def decode_workspace_bytes(num_part_slots: int, num_kv_heads: int, group: int) -> int:
     """Workspace bytes of a decode (or MIXED) launch with ``num_part_slots`` split-K slots."""
     nbytes = int(_native.query("mva_decode_workspace_bytes", num_part_slots, num_kv_heads, group))
@@ -405,6 +427,10 @@ def paged_decode(
     ``merges`` (see :func:`decode_merge_list`) lists the split segments whose
     partials the follow-up merge kernel combines.
     """
+    if _native.host_ops().paged_decode(q, k_cache, v_cache, block_tables, seq_lens, items, num_items, num_waves, merges,
+                                       num_merges, num_part_slots, out, workspace, softmax_scale, wave_extra,
+                                       waves_per_group):
+        return
     if validate:
         _check_paged(q, out, k_cache, v_cache,
                      (("block_tables", block_tables), ("seq_lens", seq_lens), ("items", items),
@@ -465,6 +491,10 @@ def paged_decode_store(
     (token, KV head) rows.  ``key``/``value`` are ``[T, Hkv, D]`` with unit
     inner stride; ``slot_mapping`` int32/int64 ``[T]`` (``< 0`` = skip).
     """
+    if _native.host_ops().paged_decode(q, k_cache, v_cache, block_tables, seq_lens, items, num_items, num_waves, merges,
+                                       num_merges, num_part_slots, out, workspace, softmax_scale, wave_extra,
+                                       waves_per_group, key, value, slot_mapping):
+        return
     if validate:
         _check_paged(q, out, k_cache, v_cache,
                      (("block_tables", block_tables), ("seq_lens", seq_lens), ("items", items),
@@ -627,6 +657,7 @@ MIXED_MAX_KV_HEADS = 64
 MIXED_ARRIVAL_COUNTERS = 65536
 
 
+@functools.lru_cache(maxsize=256)
 def prefill_workspace_bytes(max_tiles: int) -> int:
     nbytes = int(_native.query("mva_prefill_workspace_bytes", max_tiles))
     if nbytes < 0:
@@ -674,6 +705,9 @@ def paged_prefill(
     streams the plan that :func:`paged_prefill_plan` (or an earlier launch)
     left in ``workspace`` for the same batch metadata, and plans nothing.
     """
+    if _native.host_ops().paged_prefill(q, k_cache, v_cache, block_tables, seq_lens, query_start_loc, num_seqs,
+                                        max_tiles, workspace, out, softmax_scale, planned):
+        return
     if validate:
         _check_paged(q, out, k_cache, v_cache,
                      (("block_tables", block_tables), ("seq_lens", seq_lens), ("query_start_loc", query_start_loc)),
@@ -744,6 +778,10 @@ def paged_mixed(
     inside the launch (no merge list).  ``workspace`` is the decode
     workspace.
     """
+    if _native.host_ops().paged_mixed(q, k_cache, v_cache, block_tables, seq_lens, query_start_loc, num_prefill_seqs,
+                                      max_prefill_tiles, decode_items, num_decode_items, num_decode_waves,
+                                      num_part_slots, out, workspace, softmax_scale):
+        return
     if validate:
         _check_paged(q, out, k_cache, v_cache,
                      (("block_tables", block_tables), ("seq_lens", seq_lens), ("query_start_loc", query_start_loc),
