@@ -400,7 +400,7 @@ int mva_paged_prefill_run(const void* q, int64_t q_token_stride, int64_t q_head_
                           int page_size, float softmax_scale, int dtype, void* stream);
 
 /*
- * MIXED batch in one launch: prefill tiles write the rows of the leading
+ * MIXED batch in one launch without a plan: prefill tiles write the rows of the leading
  * num_prefill_seqs (<= 1024) sequences and decode pieces (as
  * mva_paged_decode, claim schedule) write the trailing decode rows of the
  * same `out` buffer.  The prefill tiles (mva_prefill_tile_tokens() tokens
@@ -426,6 +426,44 @@ int mva_paged_mixed(const void* q, int64_t q_token_stride, int64_t q_head_stride
                     int64_t num_part_slots, void* out, int64_t out_token_stride, int64_t out_head_stride,
                     void* workspace, int64_t workspace_bytes, int num_q_heads, int num_kv_heads,
                     int head_dim, int page_size, float softmax_scale, int dtype, void* stream);
+
+/*
+ * Workgroups (CUs) that mva_paged_mixed_run should give the prefill part of a
+ * MIXED step: the multiple of num_kv_heads, below num_cus, whose estimated
+ * prefill time and decode time on the CUs left are closest.  prefill_pages
+ * holds the pages of each prefill sequence, decode_pages those of all decode
+ * sequences.  0 without prefill tokens and where mva_paged_mixed is faster
+ * (many prefill tiles, little decode), -1 for invalid arguments.  Host only.
+ */
+int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, int64_t num_prefill_seqs,
+                                     int64_t num_prefill_tokens, int64_t decode_pages, int num_q_heads,
+                                     int num_kv_heads, int64_t num_cus);
+
+/*
+ * MIXED batch with a per-step prefill plan and decode piece lists: one launch
+ * whose first prefill_workgroups workgroups (a multiple of num_kv_heads; one
+ * workgroup fills a CU) run the prefill tiles and whose others run eight
+ * decode wavefronts each, then the merge kernel of mva_paged_decode when
+ * num_merges > 0.  Prefill arguments are those of mva_paged_prefill (256-row
+ * tiles, workspace of mva_prefill_workspace_bytes(max_prefill_tiles)), decode
+ * arguments those of mva_paged_decode with piece lists.  planned == 0 builds
+ * the tile plan first; planned != 0 runs the plan that an earlier call with
+ * the same lengths, page tables, max_prefill_tiles, prefill_workgroups and
+ * num_decode_waves left in prefill_workspace.  Either part may be empty.
+ * Serves the same route as mva_paged_mixed.
+ */
+int mva_paged_mixed_run(const void* q, int64_t q_token_stride, int64_t q_head_stride,
+                        const void* k_cache, const void* v_cache, int64_t num_pages,
+                        int64_t page_stride, int64_t token_stride, const int32_t* block_tables,
+                        int64_t block_table_stride, const int32_t* seq_lens,
+                        const int32_t* query_start_loc, int64_t num_prefill_seqs, int64_t max_prefill_tiles,
+                        int64_t prefill_workgroups, void* prefill_workspace, int64_t prefill_workspace_bytes,
+                        int planned, const int32_t* decode_items, int64_t num_decode_items,
+                        int64_t num_decode_waves, const int32_t* wave_extra, const int32_t* merges,
+                        int64_t num_merges, int64_t num_part_slots, void* out, int64_t out_token_stride,
+                        int64_t out_head_stride, void* workspace, int64_t workspace_bytes, int num_q_heads,
+                        int num_kv_heads, int head_dim, int page_size, float softmax_scale, int dtype,
+                        void* stream);
 
 #ifdef __cplusplus
 }

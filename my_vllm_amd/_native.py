@@ -183,11 +183,27 @@ _SIGNATURES = {
             _i32, _i32, _i32, _i32, _f32, _i32, _c_void_p,
         ],
     ),
+    "mva_mixed_prefill_workgroups": (_i64, [_c_void_p, _i64, _i64, _i64, _i32, _i32, _i64]),
+    "mva_paged_mixed_run": (
+        _i32,
+        [
+            _c_void_p, _i64, _i64,
+            _c_void_p, _c_void_p, _i64, _i64, _i64,
+            _c_void_p, _i64, _c_void_p, _c_void_p,
+            _i64, _i64, _i64,  # prefill seqs, max prefill tiles, prefill workgroups
+            _c_void_p, _i64, _i32,  # prefill workspace, its bytes, planned
+            _c_void_p, _i64, _i64, _c_void_p,  # decode items, their number, waves, wave_extra
+            _c_void_p, _i64, _i64,  # merges, num_merges, num_part_slots
+            _c_void_p, _i64, _i64,
+            _c_void_p, _i64,
+            _i32, _i32, _i32, _i32, _f32, _i32, _c_void_p,
+        ],
+    ),
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 # The C ABI revision these signatures describe (mva_abi_version()).
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -14,7 +14,8 @@ backend-owned output buffer:
 
 * DECODE        -> paged GQA decode (piece lists or claims, split-K merge kernel)
 * PREFILL       -> ragged causal chunked prefill over prefix-cached pages
-* MIXED_UNIFIED -> one launch writing ``out[:P]`` (prefill) and ``out[P:]`` (decode)
+* MIXED_UNIFIED -> one launch writing ``out[:P]`` (prefill) and ``out[P:]`` (decode),
+  then the merge kernel of its split decode sequences
 * MIXED_SPLIT   -> prefill launch into ``out[:P]`` + decode launch into ``out[P:]``
 * WARMUP        -> cacheless causal attention (no pages; one-time memory probe)
 """
@@ -66,9 +67,10 @@ class MI355XAttentionMetadata:
     wavefronts claim pieces (``make_decode_plan``).  ``decode_merges`` lists the split segments
     (``ops.decode_merge_list``) whose partials the merge kernel combines.
     Prefill query tiles are derived on the device from ``query_start_loc``
-    and ``seq_lens``: ``prefill_max_tiles`` bounds those of the PREFILL and
-    split routes (256-row tiles), ``mixed_prefill_max_tiles`` those of the
-    single MIXED launch (128-row tiles).  ``kv_indptr`` is the page CSR
+    and ``seq_lens``: ``prefill_max_tiles`` bounds those of the planned
+    launches (256-row tiles), ``mixed_prefill_max_tiles`` those of
+    ``ops.paged_mixed`` (128-row tiles).  A one-launch MIXED step with piece
+    lists gives ``mixed_prefill_workgroups`` CUs to its prefill tiles.  ``kv_indptr`` is the page CSR
     offset list (host ints): sequence ``s`` owns pages
     ``block_tables[s, :kv_indptr[s+1]-kv_indptr[s]]``.
     """
@@ -97,6 +99,7 @@ class MI355XAttentionMetadata:
     # launch takes).
     prefill_max_tiles: int = 0
     mixed_prefill_max_tiles: int = 0
+    mixed_prefill_workgroups: int = 0
     mixed_split_reason: str | None = None
 
     @property
@@ -114,6 +117,12 @@ _DECODE_WAVES_PER_CU = 5
 _MIXED_DECODE_WAVES_PER_CU = 6
 
 
+def _num_cus(device: torch.device | None) -> int:
+    if device is not None and device.type == "cuda":
+        return torch.cuda.get_device_properties(device).multi_processor_count
+    return 256
+
+
 def resident_decode_waves(device: torch.device | None = None, mixed: bool = False,
                           override: int | None = None) -> int:
     """Decode wavefronts per launch: CUs x 5 (x 6 in a MIXED launch); 1280 / 1536 on MI355X.
@@ -121,10 +130,7 @@ def resident_decode_waves(device: torch.device | None = None, mixed: bool = Fals
     ``override`` (a backend's ``decode_waves_override``) replaces the count."""
     if override:
         return max(1, int(override))
-    per_cu = _MIXED_DECODE_WAVES_PER_CU if mixed else _DECODE_WAVES_PER_CU
-    if device is not None and device.type == "cuda":
-        return torch.cuda.get_device_properties(device).multi_processor_count * per_cu
-    return 256 * per_cu
+    return _num_cus(device) * (_MIXED_DECODE_WAVES_PER_CU if mixed else _DECODE_WAVES_PER_CU)
 
 
 def _plan_counts(block_counts) -> np.ndarray:
@@ -238,10 +244,7 @@ def listed_decode_groups(num_kv_heads: int, device: torch.device | None = None,
     count the workgroups share.
     """
     per_group = num_kv_heads if num_kv_heads in (1, 2, 4, 8) else 1
-    cus = 256
-    if device is not None and device.type == "cuda":
-        cus = torch.cuda.get_device_properties(device).multi_processor_count
-    waves = max(1, int(override)) if override else cus * _LISTED_WAVES_PER_CU
+    waves = max(1, int(override)) if override else _num_cus(device) * _LISTED_WAVES_PER_CU
     return max(1, waves // num_kv_heads), per_group
 
 
@@ -655,6 +658,7 @@ class MI355XAttentionBackendMixin:
         num_decode_waves = 0
         num_part_slots = 0
         waves_per_group = 1
+        mixed_prefill_workgroups = 0
         # A MIXED batch runs as one launch when it fits that launch's limits;
         # split_reason says why not.
         mixed = bool(common.num_prefill_seqs and common.num_decode_seqs)
@@ -663,13 +667,27 @@ class MI355XAttentionBackendMixin:
         if common.num_decode_seqs:
             decode_counts = counts[common.num_prefill_seqs:]
             wave_extra = None
-            if one_launch:
+            if one_launch and self.decode_waves_override is None and self.decode_schedule_override != "claims":
+                cus = _num_cus(block_tables.device)
+                mixed_prefill_workgroups = ops.mixed_prefill_workgroups(
+                    counts[:common.num_prefill_seqs], common.num_prefill_tokens, int(decode_counts.sum()),
+                    self.num_q_heads, self.num_kv_heads, cus)
+            if mixed_prefill_workgroups:
+                # Decode ranges for the CUs that the prefill tiles leave.
+                waves = max(1, cus - mixed_prefill_workgroups) * _LISTED_WAVES_PER_CU
+                groups, waves_per_group = listed_decode_groups(self.num_kv_heads, override=waves)
+                items, wave_extra, num_decode_waves, num_part_slots, merges = plan_decode_listed(
+                    decode_counts, common.num_prefill_seqs, common.num_prefill_tokens, self.num_kv_heads, groups
+                )
+            elif one_launch:
                 items, num_decode_waves, num_part_slots, _ = plan_decode_claims(
                     decode_counts, common.num_prefill_seqs, common.num_prefill_tokens, self.num_kv_heads,
                     resident_decode_waves(block_tables.device, mixed=True, override=self.decode_waves_override),
                 )
-                # Its split-K arrival counters cover a bounded number of
-                # (partial slot, KV head) pairs.
+                # Its launch merges split segments itself, and its split-K
+                # arrival counters cover a bounded number of (partial slot,
+                # KV head) pairs.
+                merges = np.zeros((0, ops.DECODE_ITEM_INTS), np.int32)
                 if num_part_slots * self.num_kv_heads > ops.MIXED_ARRIVAL_COUNTERS:
                     one_launch = False
                     split_reason = (f"one MIXED launch merges at most {ops.MIXED_ARRIVAL_COUNTERS} split-K "
@@ -692,9 +710,6 @@ class MI355XAttentionBackendMixin:
                         self.num_kv_heads,
                         resident_decode_waves(block_tables.device, override=self.decode_waves_override),
                     )
-            else:
-                # The single MIXED launch merges split segments itself.
-                merges = np.zeros((0, ops.DECODE_ITEM_INTS), np.int32)
             num_decode_items = items.shape[0]
             num_decode_merges = merges.shape[0]
             # Pieces, merge entries and piece-list offsets share one
@@ -736,6 +751,7 @@ class MI355XAttentionBackendMixin:
             decode_host_plan=decode_host_plan,
             prefill_max_tiles=prefill_max_tiles,
             mixed_prefill_max_tiles=mixed_prefill_max_tiles,
+            mixed_prefill_workgroups=mixed_prefill_workgroups,
             mixed_split_reason=split_reason if mixed and not one_launch else None,
         )
 
@@ -906,8 +922,8 @@ class MI355XAttentionBackendMixin:
             raise RuntimeError(f"invalid planned MI355X route: {route!r}")
         if plan.batch_type is not expected:
             raise ValueError("MI355X route does not match the planned BatchType")
-        # The metadata fixes how a MIXED batch runs: a single launch's decode
-        # plan has no merge list, a split plan's has.
+        # The metadata fixes how a MIXED batch runs: the decode pieces of a
+        # single launch are cut for the CUs its prefill tiles leave.
         if expected is Batch.MIXED and (route is Route.MIXED_UNIFIED) != (metadata.mixed_prefill_max_tiles > 0):
             raise ValueError("MI355X MIXED route does not match the planned metadata")
         if not has_k_cache:
@@ -1175,6 +1191,30 @@ class MI355XAttentionBackendMixin:
         group = self.num_q_heads // self.num_kv_heads
         ws_bytes = ops.decode_workspace_bytes(metadata.num_decode_part_slots, self.num_kv_heads, group)
         workspace = self._get_workspace(ws_bytes, q.device)
+        if metadata.mixed_prefill_workgroups:
+            # The tile plan serves every layer of the step, as in _run_prefill.
+            # A captured launch plans inside the graph, in a workspace of the
+            # graph's own: replays see the lengths and page tables of their
+            # time and leave the eager steps' plan alone.
+            capturing = torch.cuda.is_current_stream_capturing()
+            if capturing:
+                nbytes = ops.prefill_workspace_bytes(metadata.prefill_max_tiles)
+                prefill_workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+            else:
+                prefill_workspace = self._get_prefill_workspace(metadata.prefill_max_tiles, q.device)
+            ops.paged_mixed_run(
+                q, k_cache, v_cache,
+                metadata.block_tables, metadata.seq_lens, metadata.query_start_loc,
+                common.num_prefill_seqs, metadata.prefill_max_tiles, metadata.mixed_prefill_workgroups,
+                prefill_workspace,
+                metadata.decode_items, metadata.num_decode_items, metadata.num_decode_waves,
+                metadata.decode_wave_extra, metadata.decode_merges, metadata.num_decode_merges,
+                metadata.num_decode_part_slots, output, workspace, self.softmax_scale,
+                planned=not capturing and self._prefill_planned_for is metadata,
+            )
+            if not capturing:
+                self._prefill_planned_for = metadata
+            return
         ops.paged_mixed(
             q,
             k_cache,

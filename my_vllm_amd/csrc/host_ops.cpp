@@ -333,27 +333,44 @@ PyObject* paged_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // (q, k_cache, v_cache, block_tables, seq_lens, query_start_loc, num_seqs,
 //  max_tiles, items | None, num_items, num_waves, num_part_slots, out,
-//  workspace, scale)
+//  workspace, scale[, prefill_workgroups, prefill_workspace, planned,
+//  wave_extra, merges, num_merges])
 PyObject* paged_mixed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     Paged p;
     int64_t seqs, tiles, items_n, waves, slots_n;
     double scale;
-    if (n != 15 || !p.read(a[0], a[1], a[2], a[3], a[4], a[12])) return none();
+    if ((n != 15 && n != 21) || !p.read(a[0], a[1], a[2], a[3], a[4], a[12])) return none();
     const Tensor *qsl = plain(a[5]), *items = a[8] == Py_None ? nullptr : plain(a[8]), *ws = plain(a[13]);
     if (!p.ints(qsl) || (a[8] != Py_None && !p.ints(items)) || !p.bytes(ws) || !as_int(a[6], &seqs) ||
         !as_int(a[7], &tiles) || !as_int(a[9], &items_n) || !as_int(a[10], &waves) || !as_int(a[11], &slots_n) ||
         !as_float(a[14], &scale))
       return none();
     const Tensor &q = *p.q, &kc = *p.kc, &out = *p.out;
-    const int status = mva_paged_mixed(
-        ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0), kc.stride(1),
-        (const int32_t*)ptr(*p.bt), p.bt->stride(0), (const int32_t*)ptr(*p.sl), (const int32_t*)ptr(*qsl), seqs, tiles,
-        (const int32_t*)ptr_or_null(items), items_n, waves, slots_n, ptr(out), out.stride(0), out.stride(1), ptr(*ws),
-        nbytes(ws), (int)q.size(1), (int)kc.size(2), (int)q.size(2), (int)kc.size(1), (float)scale, p.code,
-        stream_of(q));
+    int status;
+    if (n == 15) {
+      status = mva_paged_mixed(
+          ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0), kc.stride(1),
+          (const int32_t*)ptr(*p.bt), p.bt->stride(0), (const int32_t*)ptr(*p.sl), (const int32_t*)ptr(*qsl), seqs,
+          tiles, (const int32_t*)ptr_or_null(items), items_n, waves, slots_n, ptr(out), out.stride(0), out.stride(1),
+          ptr(*ws), nbytes(ws), (int)q.size(1), (int)kc.size(2), (int)q.size(2), (int)kc.size(1), (float)scale, p.code,
+          stream_of(q));
+    } else {
+      const Tensor *pws = plain(a[16]), *extra = plain(a[18]), *merges = plain(a[19]);
+      int64_t workgroups, merges_n;
+      if (!items || !p.bytes(pws) || !p.ints(extra) || !p.ints(merges) || !as_int(a[15], &workgroups) ||
+          !PyBool_Check(a[17]) || !as_int(a[20], &merges_n))
+        return none();
+      status = mva_paged_mixed_run(
+          ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0), kc.stride(1),
+          (const int32_t*)ptr(*p.bt), p.bt->stride(0), (const int32_t*)ptr(*p.sl), (const int32_t*)ptr(*qsl), seqs,
+          tiles, workgroups, ptr(*pws), nbytes(pws), a[17] == Py_True, (const int32_t*)ptr(*items), items_n, waves,
+          (const int32_t*)ptr(*extra), (const int32_t*)ptr(*merges), merges_n, slots_n, ptr(out), out.stride(0),
+          out.stride(1), ptr(*ws), nbytes(ws), (int)q.size(1), (int)kc.size(2), (int)q.size(2), (int)kc.size(1),
+          (float)scale, p.code, stream_of(q));
+    }
     Py_INCREF(Py_True);
-    return launched("mva_paged_mixed", status, Py_True);
+    return launched(n == 15 ? "mva_paged_mixed" : "mva_paged_mixed_run", status, Py_True);
   });
 }
 

@@ -1,8 +1,12 @@
-// C-ABI entry points of the ragged causal prefill kernel and of the
-// single-launch MIXED kernel (prefill tiles + decode items in one grid).
+// C-ABI entry points of the ragged causal prefill kernel and of the MIXED
+// kernels (prefill tiles + decode items in one grid).
 #include "mva_capi.h"
 #include "paged_prefill.h"
 #include "paged_prefill_pingpong.h"
+
+#include <algorithm>
+#include <functional>
+#include <vector>
 
 namespace mva {
 
@@ -16,8 +20,13 @@ int fill_decode_params(DecodeParams& p, const void* q, int64_t q_token_stride, i
                        int num_q_heads, int num_kv_heads, int head_dim, int page_size,
                        float softmax_scale);
 int32_t* decode_arrival_counters(void* workspace);
+int launch_decode_merge(const DecodeParams& p, const int32_t* merges, int64_t num_merges, int64_t num_part_slots,
+                        int dtype, hipStream_t stream);
 
 namespace {
+
+// Decode wavefronts in a workgroup of paged_mixed_split_cus_kernel.
+constexpr int kMixedDecodeWaves = kPrefillPPThreads / 64;
 
 // Piece list and arrival counters, before the partials, in words.
 constexpr int64_t kPrefillSplitMetaInts = kPrefillPieceSlots * (kPrefillPieceInts + 1);
@@ -290,6 +299,27 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(const int32_t* __res
   if (tid < kPrefillPlanMaxHeads) plan[kPrefillPlanLineInts * (1 + tid)] = 0;  // claim counters
 }
 
+// The last workgroup out zeroes the claim counters and the exit count, so
+// the plan serves the next launch as it is.  Every claim and counter read
+// of a workgroup has returned (its result decided the exit) before thread 0
+// counts the workgroup out, and workgroups of any head claim from every
+// head's counter, so only the grid's last exit may clear them.
+// (The grid size comes from the plan header, which keeps the dispatch
+// packet's registers out of the tile loop.)  Every thread of the workgroup
+// calls it.
+__device__ __attribute__((always_inline)) inline void leave_prefill_plan(int32_t* plan) {
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  int gone = 0;
+  if (threadIdx.x == 0)
+    gone = __hip_atomic_fetch_add(plan + kPrefillPlanExitInt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  gone = __builtin_amdgcn_readfirstlane(gone);
+  if (gone != plan[kPrefillPlanGridInt] - 1) return;
+  for (int hh = threadIdx.x; hh < kPrefillPlanMaxHeads; hh += 64)
+    __hip_atomic_store(plan + kPrefillPlanLineInts * (1 + hh), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) __hip_atomic_store(plan + kPrefillPlanExitInt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Persistent prefill: workgroup b serves KV head b % num_kv_heads (so head
 // h stays on XCD h when the head count divides 8).  The workgroups of a head
 // take tiles of the plan in order from that head's claim counter, one claim
@@ -306,25 +336,7 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_stream_kernel
     prefill_items_pingpong<T, 0, false>(p, plan, h, 0, (lds_u8*)tiles, (lds_i32*)nextq);
   else
     prefill_items_pingpong<T, 1, false>(p, plan, h, 0, (lds_u8*)tiles, (lds_i32*)nextq);
-  // The last workgroup out zeroes the claim counters and the exit count, so
-  // the plan serves the next launch as it is.  Every claim and counter read
-  // of a workgroup has returned (its result decided the exit) before thread 0
-  // counts the workgroup out, and workgroups of any head claim from every
-  // head's counter, so only the grid's last exit may clear them.
-  // (The grid size comes from the plan header, which keeps the dispatch
-  // packet's registers out of the tile loop.)
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    int gone = 0;
-    if (threadIdx.x == 0)
-      gone = __hip_atomic_fetch_add(plan + kPrefillPlanExitInt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    gone = __builtin_amdgcn_readfirstlane(gone);
-    if (gone == plan[kPrefillPlanGridInt] - 1) {
-      for (int hh = threadIdx.x; hh < kPrefillPlanMaxHeads; hh += 64)
-        __hip_atomic_store(plan + kPrefillPlanLineInts * (1 + hh), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (threadIdx.x == 0) __hip_atomic_store(plan + kPrefillPlanExitInt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
+  leave_prefill_plan(plan);
 }
 
 // The fixed form, for a batch of at most one tile per workgroup of a head: no
@@ -341,6 +353,56 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_fixed_kernel(
   else
     prefill_items_pingpong<T, 1, true>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
 }
+
+// A MIXED step on CUs of two kinds.  Workgroups of 512 threads, one per CU
+// (128 KB of LDS): the first `n_prefill` (a whole number per KV head) run the
+// prefill plan as the prefill-only kernels do, the rest run eight decode
+// wavefronts each, as the piece-list decode kernel does.  With kFixed the
+// plan has at most one item per prefill workgroup of a head; otherwise tiles
+// are claimed, and a decode workgroup whose pieces are done joins in.
+//
+// The two parts have different bounds (the matrix cores and HBM), so they are
+// best run side by side; sharing every CU between decode wavefronts and a
+// four-wave prefill core (paged_mixed_kernel) costs each part the other's
+// registers, LDS and issue slots: it time-slices more than it overlaps, with
+// prefill tiles half as large, none cut, at the end of a wave of work.  On
+// CUs of their own each part runs its own kernel's schedule.  What bounds it:
+// a CU of decode wavefronts has 64 KB in flight, 38 GB/s, so the CUs left to
+// decode set its time until HBM does (5.8 TB/s), and the prefill CUs slow
+// down beside it (power and L2).  Against paged_mixed_kernel, microseconds of
+// a step: 300 tokens over 1936 and 20 decodes of 2250 (32 / 8 heads, fp16)
+// 69 -> 47, 2 chunks over 4k and 64 decodes of 2700 211 -> 187, 4 chunks of a
+// budget of 8192 and 256 decodes of 4391 965 -> 945, 1 decode of 12695 beside
+// 109 prompt tokens (64 / 8 heads) 168 -> 20.  Split-K decode segments are
+// merged by the merge kernel that follows: merging inside the launch cost 5
+// to 17 us more (the merges run one after another on the last wavefronts).
+template <typename T, bool kFixed>
+__global__ __launch_bounds__(kPrefillPPThreads) void paged_mixed_split_cus_kernel(PrefillParams pp,
+                                                                                  int32_t* __restrict__ plan,
+                                                                                  DecodeParams dp,
+                                                                                  uint32_t n_prefill) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kMixedDecodeWaves * kDecodeWaveLdsBytes];
+  __shared__ int nextq[8];
+  __shared__ int progress[kMixedDecodeWaves];
+  if (blockIdx.x >= n_prefill) {
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wave = (int)(blockIdx.x - n_prefill) * kMixedDecodeWaves + w;
+    if ((threadIdx.x & 63) == 0) progress[w] = 0x3fffffff;
+    if (wave < dp.num_waves) decode_wave<T>(dp, wave, (lds_u8*)lds + w * kDecodeWaveLdsBytes, progress);
+    if constexpr (kFixed) return;
+    __builtin_amdgcn_s_setprio(0);
+    __syncthreads();  // the LDS of all eight is free
+  }
+  const int h = (int)(blockIdx.x % (uint32_t)pp.num_kv_heads);
+  const int rank = (int)(blockIdx.x / (uint32_t)pp.num_kv_heads);
+  if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) == 0)
+    prefill_items_pingpong<T, 0, kFixed>(pp, plan, h, rank, (lds_u8*)lds, (lds_i32*)nextq);
+  else
+    prefill_items_pingpong<T, 1, kFixed>(pp, plan, h, rank, (lds_u8*)lds, (lds_i32*)nextq);
+  if constexpr (!kFixed) leave_prefill_plan(plan);
+}
+
+static_assert(kMixedDecodeWaves * kDecodeWaveLdsBytes >= kPrefillPPLdsBytes, "prefill tiles fit the decode buffers");
 
 int device_cu_count() {
   static int counts[64] = {};
@@ -586,6 +648,38 @@ extern "C" int64_t mva_prefill_workspace_bytes(int64_t max_tiles) {
 
 namespace {
 
+using namespace mva;
+
+const char kBadTileCapacity[] = "paged attention: invalid tile capacity";
+
+// Plans a batch for `per_head` prefill workgroups per KV head in a launch of
+// `grid` workgroups that count themselves out of the plan.
+int launch_prefill_plan(const PrefillParams& p, int64_t num_seqs, int64_t max_tiles, int32_t* plan,
+                        int64_t workspace_bytes, int64_t per_head, int64_t grid, hipStream_t s) {
+  // The last three tiles per workgroup of a head go largest first.
+  const int64_t last = 3 * (per_head < max_tiles ? per_head : max_tiles);
+  const int tail = (int)(last < 1024 ? last : 1024);
+  // A batch of at most one tile per workgroup may be split, where there is
+  // room for partials.
+  const bool split = max_tiles <= per_head && max_tiles <= kPrefillPieceSlots &&
+                     workspace_bytes >= prefill_split_bytes(max_tiles);
+  hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(1024), 0, s, p.query_start_loc, p.seq_lens, p.block_tables,
+                     p.bt_stride, p.num_pages, (int)num_seqs, p.tile_tokens, p.num_kv_heads, plan, (int)max_tiles, tail,
+                     (int)grid, (int)per_head, split ? (int)prefill_piece_list(max_tiles) : 0);
+  return check_launch("paged_prefill plan");
+}
+
+// The checks of a prefill plan's tile capacity, workspace and head count.
+int check_prefill_plan(int64_t max_tiles, const void* workspace, int64_t workspace_bytes, int num_kv_heads) {
+  if (mva_prefill_workspace_bytes(max_tiles) < 0) return set_error(kBadTileCapacity);
+  // The plan itself must fit; without room for partials no tile is split.
+  if (workspace == nullptr || workspace_bytes < prefill_plan_bytes(max_tiles))
+    return set_error("paged attention: prefill workspace too small for max_tiles");
+  if (((uintptr_t)workspace) % 16) return set_error("paged attention: prefill workspace must be 16-byte aligned");
+  if (num_kv_heads > kPrefillPlanMaxHeads) return set_error("paged attention: at most 127 KV heads");
+  return 0;
+}
+
 // Plans (plan_it) and/or streams (run_it) a prefill batch: the shared body
 // of mva_paged_prefill, mva_paged_prefill_plan and mva_paged_prefill_run.
 int prefill_launch(const void* q, int64_t q_token_stride, int64_t q_head_stride, const void* k_cache,
@@ -595,7 +689,6 @@ int prefill_launch(const void* q, int64_t q_token_stride, int64_t q_head_stride,
                    int64_t workspace_bytes, void* out, int64_t out_token_stride, int64_t out_head_stride,
                    int num_q_heads, int num_kv_heads, int head_dim, int page_size, float softmax_scale, int dtype,
                    void* stream, bool plan_it, bool run_it) {
-  using namespace mva;
   PrefillParams p;
   int rc = fill_prefill_params(p, q, q_token_stride, q_head_stride, k_cache, v_cache, num_pages, page_stride,
                                token_stride, block_tables, block_table_stride, seq_lens, query_start_loc,
@@ -603,16 +696,12 @@ int prefill_launch(const void* q, int64_t q_token_stride, int64_t q_head_stride,
                                num_kv_heads, head_dim, page_size, softmax_scale);
   if (rc) return rc;
   if (dtype != kBF16 && dtype != kF16) return set_error("paged attention: dtype must be bf16 or fp16");
-  if (mva_prefill_workspace_bytes(max_tiles) < 0) return set_error("paged attention: invalid tile capacity");
-  // The plan itself must fit; without room for partials no tile is split.
-  const int64_t need = prefill_plan_bytes(max_tiles);
+  if (mva_prefill_workspace_bytes(max_tiles) < 0) return set_error(kBadTileCapacity);
   if (num_seqs == 0 || max_tiles == 0) return 0;
-  if (workspace == nullptr || workspace_bytes < need)
-    return set_error("paged attention: prefill workspace too small for max_tiles");
-  if (((uintptr_t)workspace) % 16) return set_error("paged attention: prefill workspace must be 16-byte aligned");
+  rc = check_prefill_plan(max_tiles, workspace, workspace_bytes, num_kv_heads);
+  if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   int32_t* plan = (int32_t*)workspace;
-  if (num_kv_heads > kPrefillPlanMaxHeads) return set_error("paged attention: at most 127 KV heads");
   p.tile_tokens = kPrefillPPRows / p.group;
   // Persistent grid: one workgroup per CU (96 KB of LDS and two waves per
   // SIMD each), a whole number per KV head, also where the tiles are fewer:
@@ -622,15 +711,7 @@ int prefill_launch(const void* q, int64_t q_token_stride, int64_t q_head_stride,
   // A batch of at most one tile per workgroup runs the fixed form.
   const bool fixed = max_tiles <= per_head;
   if (plan_it) {
-    // The last three tiles per workgroup of a head go largest first.
-    const int64_t last = 3 * (per_head < max_tiles ? per_head : max_tiles);
-    const int tail = (int)(last < 1024 ? last : 1024);
-    const bool split = fixed && max_tiles <= kPrefillPieceSlots && workspace_bytes >= prefill_split_bytes(max_tiles);
-    hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(1024), 0, s, query_start_loc, seq_lens, block_tables,
-                       block_table_stride, num_pages, (int)num_seqs, p.tile_tokens, num_kv_heads, plan,
-                       (int)max_tiles, tail, (int)(per_head * num_kv_heads), (int)per_head,
-                       split ? (int)prefill_piece_list(max_tiles) : 0);
-    rc = check_launch("paged_prefill plan");
+    rc = launch_prefill_plan(p, num_seqs, max_tiles, plan, workspace_bytes, per_head, per_head * num_kv_heads, s);
     if (rc) return rc;
   }
   if (!run_it) return 0;
@@ -750,4 +831,182 @@ extern "C" int mva_paged_mixed(const void* q, int64_t q_token_stride, int64_t q_
     hipLaunchKernelGGL(paged_mixed_kernel<_Float16>, grid, dim3(256), 0, s, pp, dp, np, nd);
   else return set_error("paged attention: dtype must be bf16 or fp16");
   return check_launch("paged_mixed");
+}
+
+// Host estimate of the CUs a MIXED launch gives its prefill part (see
+// mva_mixed_prefill_workgroups), in microseconds fitted to sweeps of the
+// split on one MI355X: a prefill workgroup takes 1.7 per 64 keys of a 256-row
+// tile and as much as 2.5 of them per tile or piece; a CU of decode
+// wavefronts streams 1 MB in 26.3 beside 0.045 per MB of the launch, and all
+// of them together no faster than 0.172 per MB (5.8 TB/s).
+namespace {
+
+constexpr double kTileUs = 1.7;
+constexpr double kItemTiles = 2.5;
+constexpr double kPrefillStartUs = 4.0;
+constexpr double kStreamUs = 5.0;  // claims, and decode workgroups joining in at the end
+constexpr double kDecodeStartUs = 6.0, kDecodeUsPerMB = 0.045, kDecodeUsPerMBCu = 26.3, kDecodeMinUsPerMB = 0.172;
+constexpr double kLittleDecode = 0.25;
+constexpr int64_t kSortTiles = 4096;  // batches of more tiles are taken as even
+
+struct PrefillEstimate {
+  int64_t tiles = 0;          // query tiles of one KV head
+  double work = 0;            // 64-key tiles of all of them
+  std::vector<int> keys;      // 64-key tiles of each, longest first (empty beyond kSortTiles)
+};
+
+// The batch's query tiles from its page and token counts: queries are spread
+// evenly over the sequences (their lengths are on the device), none having
+// more queries than keys.
+PrefillEstimate estimate_prefill(const int64_t* pages, int64_t n, int64_t tokens, int tile_tokens) {
+  PrefillEstimate e;
+  double share = (double)tokens / (double)n, held = 0;
+  int64_t longer = 0;
+  for (int64_t s = 0; s < n; ++s) {
+    const double kv = (double)pages[s] * kPageSize;
+    if (kv < share) held += kv;
+    else ++longer;
+  }
+  if (longer > 0) share = ((double)tokens - held) / (double)longer;
+  for (int64_t s = 0; s < n; ++s) {
+    const double kv = (double)pages[s] * kPageSize, q = kv < share ? kv : share;
+    const int64_t count = (int64_t)((q + tile_tokens - 1) / tile_tokens);
+    for (int64_t t = 0; t < count; ++t) {
+      const double end = kv - q + ((t + 1) * tile_tokens < q ? (double)((t + 1) * tile_tokens) : q);
+      const int keys = (int)((end + kPrefillKeys - 1) / kPrefillKeys);
+      e.work += keys;
+      if (++e.tiles <= kSortTiles) e.keys.push_back(keys);
+    }
+  }
+  if (e.tiles > kSortTiles) e.keys.clear();
+  std::sort(e.keys.begin(), e.keys.end(), std::greater<int>());
+  return e;
+}
+
+// Time of the prefill part on per_head workgroups per KV head.
+double prefill_part_us(const PrefillEstimate& e, int64_t per_head, int64_t max_tiles, int num_kv_heads) {
+  if (max_tiles > per_head) {
+    // j + 1 of the j * per_head + 1 longest tiles share a workgroup.
+    double len = e.work / (double)per_head + kItemTiles * ((double)e.tiles / (double)per_head);
+    for (int64_t j = 0; j * per_head < (int64_t)e.keys.size(); ++j) {
+      const double together = (double)(j + 1) * (e.keys[j * per_head] + kItemTiles);
+      if (together > len) len = together;
+    }
+    return kPrefillStartUs + kTileUs * len;
+  }
+  // plan_pieces' choice.
+  int64_t limit = kPrefillPieceSlots / num_kv_heads;
+  limit = per_head < limit ? per_head : limit;
+  const int longest = e.keys.empty() ? 0 : e.keys[0];
+  double best = longest;
+  for (int k = 2; k <= kPrefillMaxPieces; ++k) {
+    const int len = longest > k ? (longest + k - 1) / k : 1;
+    int64_t count = 0;
+    for (int keys : e.keys) count += (keys + len - 1) / len;
+    const double t = len + 2.5 + 0.75 * k;
+    if (count <= limit && t < best) best = t;
+  }
+  return kPrefillStartUs + kTileUs * (best + kItemTiles);
+}
+
+}  // namespace
+
+extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, int64_t num_prefill_seqs,
+                                                int64_t num_prefill_tokens, int64_t decode_pages, int num_q_heads,
+                                                int num_kv_heads, int64_t num_cus) {
+  if (num_prefill_seqs < 0 || num_prefill_tokens < 0 || decode_pages < 0 || num_kv_heads <= 0 || num_q_heads <= 0 ||
+      num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > 16 || (num_prefill_seqs > 0 && prefill_pages == nullptr))
+    return -1;
+  if (num_prefill_seqs == 0 || num_prefill_tokens == 0) return 0;
+  const int tile_tokens = kPrefillPPRows / (num_q_heads / num_kv_heads);
+  const int64_t max_tiles = num_prefill_tokens / tile_tokens + num_prefill_seqs;
+  const PrefillEstimate e = estimate_prefill(prefill_pages, num_prefill_seqs, num_prefill_tokens, tile_tokens);
+  const double mb = (double)decode_pages * kPageSize * num_kv_heads * kHeadDim * 2 * 2 * 1e-6;
+  int64_t best = 1;
+  double best_us = 0;
+  for (int64_t p = 1; p == 1 || p * num_kv_heads < num_cus; ++p) {
+    const int64_t left = num_cus - p * num_kv_heads;
+    double d = kDecodeUsPerMB + kDecodeUsPerMBCu / (double)(left > 0 ? left : 1);
+    d = kDecodeStartUs + mb * (d > kDecodeMinUsPerMB ? d : kDecodeMinUsPerMB);
+    const double f = prefill_part_us(e, p, max_tiles, num_kv_heads);
+    const double us = (d > f ? d : f) + (max_tiles > p ? kStreamUs : 0.0);
+    if (p == 1 || us < best_us) best = p, best_us = us;
+  }
+  // Little decode beside more tiles than workgroups: the 128-row tiles of
+  // mva_paged_mixed, two to a CU, balance better.  32 / 8 heads, 4 chunks of
+  // 512 tokens over up to 8k and 4 decodes 213 against 272 us; 64 / 8 heads,
+  // 4 prompts of 350-614 tokens and 13 decodes 40 against 43 us, 4 chunks of
+  // 280 over 7k and 157 decodes of 372 357 against 366 us.
+  if (max_tiles > best && kDecodeStartUs + mb * kDecodeMinUsPerMB < kLittleDecode * best_us) return 0;
+  return best * num_kv_heads;
+}
+
+extern "C" int mva_paged_mixed_run(const void* q, int64_t q_token_stride, int64_t q_head_stride,
+                                   const void* k_cache, const void* v_cache, int64_t num_pages,
+                                   int64_t page_stride, int64_t token_stride, const int32_t* block_tables,
+                                   int64_t block_table_stride, const int32_t* seq_lens,
+                                   const int32_t* query_start_loc, int64_t num_prefill_seqs, int64_t max_prefill_tiles,
+                                   int64_t prefill_workgroups, void* prefill_workspace,
+                                   int64_t prefill_workspace_bytes, int planned, const int32_t* decode_items,
+                                   int64_t num_decode_items, int64_t num_decode_waves, const int32_t* wave_extra,
+                                   const int32_t* merges, int64_t num_merges, int64_t num_part_slots, void* out,
+                                   int64_t out_token_stride, int64_t out_head_stride, void* workspace,
+                                   int64_t workspace_bytes, int num_q_heads, int num_kv_heads, int head_dim,
+                                   int page_size, float softmax_scale, int dtype, void* stream) {
+  PrefillParams pp;
+  int rc = fill_prefill_params(pp, q, q_token_stride, q_head_stride, k_cache, v_cache, num_pages, page_stride,
+                               token_stride, block_tables, block_table_stride, seq_lens, query_start_loc,
+                               num_prefill_seqs, out, out_token_stride, out_head_stride, num_q_heads, num_kv_heads,
+                               head_dim, page_size, softmax_scale);
+  if (rc) return rc;
+  if (dtype != kBF16 && dtype != kF16) return set_error("paged attention: dtype must be bf16 or fp16");
+  if (num_decode_items > 0 && wave_extra == nullptr)
+    return set_error("paged attention: a planned MIXED launch needs piece lists (wave_extra)");
+  DecodeParams dp;
+  rc = fill_decode_params(dp, q, q_token_stride, q_head_stride, k_cache, v_cache, num_pages, page_stride,
+                          token_stride, block_tables, block_table_stride, seq_lens, decode_items, num_decode_items,
+                          num_decode_waves, wave_extra, merges, num_merges, num_part_slots, out, out_token_stride,
+                          out_head_stride, workspace, workspace_bytes, num_q_heads, num_kv_heads, head_dim, page_size,
+                          softmax_scale);
+  if (rc) return rc;
+  const bool prefill = num_prefill_seqs > 0 && max_prefill_tiles > 0;
+  hipStream_t s = (hipStream_t)stream;
+  int64_t per_head = 0;
+  if (prefill) {
+    rc = check_prefill_plan(max_prefill_tiles, prefill_workspace, prefill_workspace_bytes, num_kv_heads);
+    if (rc) return rc;
+    if (prefill_workgroups <= 0 || prefill_workgroups % num_kv_heads)
+      return set_error("paged attention: prefill_workgroups must be a positive multiple of num_kv_heads");
+    per_head = prefill_workgroups / num_kv_heads;
+  } else if (num_prefill_seqs > 0 && max_prefill_tiles < 0) {
+    return set_error(kBadTileCapacity);
+  }
+  const int64_t n_decode_wgs =
+      num_decode_items > 0 ? (num_decode_waves + kMixedDecodeWaves - 1) / kMixedDecodeWaves : 0;
+  const int64_t grid = per_head * num_kv_heads + n_decode_wgs;
+  if (prefill_workgroups > 0x7fffff00LL || grid > 0x7fffff00LL) return set_error("paged attention: too many work items");
+  if (grid == 0) return 0;
+  if (num_decode_items == 0) dp.num_waves = 0;
+  // Without prefill sequences there is no plan: the fixed form ends after decode.
+  const bool fixed = !prefill || max_prefill_tiles <= per_head;
+  pp.tile_tokens = kPrefillPPRows / pp.group;
+  int32_t* plan = (int32_t*)prefill_workspace;
+  if (prefill && !planned) {
+    rc = launch_prefill_plan(pp, num_prefill_seqs, max_prefill_tiles, plan, prefill_workspace_bytes, per_head, grid, s);
+    if (rc) return rc;
+  }
+  const uint32_t np = (uint32_t)(per_head * num_kv_heads);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kPrefillPPThreads), 0, s, pp, plan, dp, np);
+  };
+  if (dtype == kBF16) {
+    if (fixed) launch(paged_mixed_split_cus_kernel<__bf16, true>);
+    else launch(paged_mixed_split_cus_kernel<__bf16, false>);
+  } else {
+    if (fixed) launch(paged_mixed_split_cus_kernel<_Float16, true>);
+    else launch(paged_mixed_split_cus_kernel<_Float16, false>);
+  }
+  rc = check_launch("paged_mixed");
+  if (rc) return rc;
+  return launch_decode_merge(dp, merges, num_merges, num_part_slots, dtype, s);
 }

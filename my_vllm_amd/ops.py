@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import functools
 
+import numpy as np
 import torch
 
 from . import _native
@@ -26,8 +27,8 @@ DECODE_ITEM_INTS = 8
 MAX_CHUNK_PAGES = 128
 # Query rows per prefill workgroup (kPrefillRows): G heads x 128 // G tokens.
 PREFILL_ROWS = 128
-# Query rows per tile of mva_paged_prefill's kernel (the MIXED kernel's
-# prefill tiles have PREFILL_ROWS).
+# Query rows per tile of the planned prefill (mva_paged_prefill,
+# mva_paged_mixed_run; mva_paged_mixed's tiles have PREFILL_ROWS).
 PREFILL_STREAM_ROWS = 256
 # Device-built prefill tile list: header ints (tile count + per-head claim
 # counters) and ints per tile record (kPrefillPlanHeaderInts / ItemInts).
@@ -792,6 +793,78 @@ def paged_mixed(
         query_start_loc.data_ptr(), int(num_prefill_seqs), int(max_prefill_tiles),
         decode_items.data_ptr() if decode_items is not None else 0, num_decode_items, num_decode_waves,
         num_part_slots,
+        out.data_ptr(), out.stride(0), out.stride(1),
+        workspace.data_ptr(), workspace.numel() * workspace.element_size(),
+        *_tail_args(q, k_cache, softmax_scale),
+    )
+
+
+def mixed_prefill_workgroups(prefill_pages, num_prefill_tokens: int, decode_pages: int, num_q_heads: int,
+                             num_kv_heads: int, num_cus: int) -> int:
+    """CUs :func:`paged_mixed_run` should give a step's prefill part
+    (``mva_mixed_prefill_workgroups``): ``prefill_pages`` holds the pages of
+    each prefill sequence, ``decode_pages`` those of all decode sequences; 0
+    where :func:`paged_mixed` is faster."""
+    pages = np.ascontiguousarray(prefill_pages, dtype=np.int64).reshape(-1)
+    count = int(_native.query("mva_mixed_prefill_workgroups", pages.ctypes.data, pages.size, int(num_prefill_tokens),
+                              int(decode_pages), int(num_q_heads), int(num_kv_heads), int(num_cus)))
+    if count < 0:
+        raise ValueError("invalid MIXED batch")
+    return count
+
+
+def paged_mixed_run(
+    q: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    block_tables: torch.Tensor,
+    seq_lens: torch.Tensor,
+    query_start_loc: torch.Tensor,
+    num_prefill_seqs: int,
+    max_prefill_tiles: int,
+    prefill_workgroups: int,
+    prefill_workspace: torch.Tensor,
+    decode_items: torch.Tensor,
+    num_decode_items: int,
+    num_decode_waves: int,
+    wave_extra: torch.Tensor,
+    merges: torch.Tensor,
+    num_merges: int,
+    num_part_slots: int,
+    out: torch.Tensor,
+    workspace: torch.Tensor,
+    softmax_scale: float,
+    *,
+    validate: bool = True,
+    planned: bool = False,
+) -> None:
+    """A MIXED step as prefill workgroups beside decode workgroups, then the
+    decode merges: prefill tiles write ``out[:P]``, decode pieces ``out[P:]``.
+
+    ``prefill_workgroups`` comes from :func:`mixed_prefill_workgroups`;
+    ``max_prefill_tiles`` and ``prefill_workspace`` are those of
+    :func:`paged_prefill` (:func:`prefill_max_tiles`), the decode arguments
+    those of :func:`paged_decode` with piece lists, ``workspace`` the decode
+    workspace.  ``planned=True`` runs the tile plan that an earlier call for
+    the same batch metadata left in ``prefill_workspace``.
+    """
+    if _native.host_ops().paged_mixed(q, k_cache, v_cache, block_tables, seq_lens, query_start_loc, num_prefill_seqs,
+                                      max_prefill_tiles, decode_items, num_decode_items, num_decode_waves,
+                                      num_part_slots, out, workspace, softmax_scale, prefill_workgroups,
+                                      prefill_workspace, planned, wave_extra, merges, num_merges):
+        return
+    if validate:
+        _check_paged(q, out, k_cache, v_cache,
+                     (("block_tables", block_tables), ("seq_lens", seq_lens), ("query_start_loc", query_start_loc),
+                      ("decode_items", decode_items), ("wave_extra", wave_extra), ("merges", merges)),
+                     (("workspace", workspace), ("prefill_workspace", prefill_workspace)))
+    _native.call(
+        "mva_paged_mixed_run",
+        *_paged_args(q, k_cache, v_cache, block_tables, seq_lens),
+        query_start_loc.data_ptr(), int(num_prefill_seqs), int(max_prefill_tiles), int(prefill_workgroups),
+        prefill_workspace.data_ptr(), prefill_workspace.numel() * prefill_workspace.element_size(), int(planned),
+        decode_items.data_ptr(), num_decode_items, num_decode_waves, wave_extra.data_ptr(),
+        merges.data_ptr(), num_merges, num_part_slots,
         out.data_ptr(), out.stride(0), out.stride(1),
         workspace.data_ptr(), workspace.numel() * workspace.element_size(),
         *_tail_args(q, k_cache, softmax_scale),

@@ -280,3 +280,73 @@ def test_mixed_output_only_8_byte_aligned_matches_aligned(gpu):
         outs.append(out.clone())
     assert torch.equal(outs[0], outs[1])
     assert_attention_close(outs[0], expected(batch))
+
+
+@pytest.mark.parametrize("hq,hkv,dtype", [(32, 8, torch.bfloat16), (16, 4, torch.float16), (3, 1, torch.bfloat16),
+                                          (64, 64, torch.bfloat16), (48, 16, torch.float16), (16, 1, torch.bfloat16)])
+@pytest.mark.parametrize("per_head", [1, 2, 3, 1000])
+@pytest.mark.parametrize("q,kv", [
+    ([1, 1], [1, 1]), ([1, 1, 1, 1], [70, 16, 17, 700]), ([300, 1], [300, 40]),
+    ([37, 700, 1, 1, 1], [300, 1300, 2100, 31, 257]), ([64, 65, 15, 16, 17, 1], [64, 65, 400, 16, 900, 1])])
+def test_planned_mixed_matches_the_unplanned_launch(gpu, monkeypatch, hq, hkv, dtype, per_head, q, kv):
+    # Prefill on CUs of its own, at the smallest and largest shares of the
+    # CUs: one claimed tile after another with decode workgroups joining in
+    # (more tiles than workgroups), or at most one item a workgroup, pieces of
+    # long tiles among them.  Planned on the first launch, streamed on the
+    # second; rows agree with the launch that plans nothing.
+    from my_vllm_amd import ops
+    from my_vllm_amd.attention_backend import MI355XAttentionBackend
+    from tests.test_gpu_prefill import to_device
+
+    prefills = sum(1 for n in q if n > 1) or len(q) - 1
+    batch = make_paged_batch(171, q, kv, prefills, hq, hkv)
+    common, qd, kc, vc = to_device(batch, gpu)
+    qd, kc, vc = (t.to(dtype) for t in (qd, kc, vc))
+    backend = MI355XAttentionBackend(hq, hkv, 128, 16, dtype)
+    empty = qd.new_empty((0, hkv, 128))
+    share = min(per_head, max(1, (torch.cuda.get_device_properties(0).multi_processor_count - 1) // hkv)) * hkv
+    monkeypatch.setattr(ops, "mixed_prefill_workgroups", lambda *a: share)
+    plan = backend.build_plan(common)
+    assert plan.route is AttentionRoute.MIXED_UNIFIED and plan.metadata.mixed_prefill_workgroups == share
+    first = backend.forward(qd, empty, empty, kc, vc, plan).clone()
+    again = backend.forward(qd, empty, empty, kc, vc, plan).clone()
+    assert torch.equal(first, again)
+    backend.decode_schedule_override = "claims"
+    other = backend.build_plan(common)
+    assert other.metadata.mixed_prefill_workgroups == 0
+    assert_attention_close(first, backend.forward(qd, empty, empty, kc, vc, other).float())
+
+
+def test_captured_planned_mixed_follows_lengths_and_pages(gpu):
+    # A captured step plans inside its graph: replays read the lengths and
+    # page tables of their time, and eager steps between them keep their plan.
+    from my_vllm_amd.attention_backend import MI355XAttentionBackend
+    from tests.test_gpu_prefill import to_device
+
+    backend = MI355XAttentionBackend(32, 8, 128, 16, torch.bfloat16)
+    batch = make_paged_batch(173, [90, 200, 1, 1], [400, 200, 900, 1200], 2, 32, 8)
+    eager = make_paged_batch(174, [40, 1, 1], [500, 77, 600], 1, 32, 8)
+    common, q, kc, vc = to_device(batch, gpu)
+    empty = q.new_empty((0, 8, 128))
+    plan = backend.build_plan(common)
+    assert plan.metadata.mixed_prefill_workgroups > 0
+    backend.forward(q, empty, empty, kc, vc, plan)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = backend.forward(q, empty, empty, kc, vc, plan)
+    tables = common.block_tables.clone()
+    e_common, eq, ekc, evc = to_device(eager, gpu)
+    e_plan = backend.build_plan(e_common)
+    want = expected(eager)
+    other = MI355XAttentionBackend(32, 8, 128, 16, torch.bfloat16)
+    for step in range(3):
+        # The first prefill sequence takes pages of the first decode one, in
+        # another order each step.
+        pages = (400 + 15) // 16
+        common.block_tables[0, :pages] = tables[2, :pages].roll(step)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.clone()
+        assert torch.equal(got, other.forward(q, empty, empty, kc, vc, other.build_plan(common)))
+        assert_attention_close(backend.forward(eq, empty, empty, ekc, evc, e_plan), want)

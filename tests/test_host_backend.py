@@ -491,6 +491,23 @@ def test_mixed_route_must_match_its_metadata():
         backend.forward(q, None, None, cache, cache, forced)
 
 
+@pytest.mark.parametrize("hq,hkv", [(8, 1), (16, 8), (64, 8), (48, 16), (64, 64), (6, 3)])
+@pytest.mark.parametrize("pages,tokens,decode", [((1,), 1, 1), ((19,), 300, 2800), ((4, 900, 3), 700, 1),
+                                                 ((64,) * 40, 40000, 100000), ((2,) * 600, 900, 7)])
+def test_mixed_prefill_workgroups_leave_cus_for_decode(hq, hkv, pages, tokens, decode):
+    count = ops.mixed_prefill_workgroups(pages, tokens, decode, hq, hkv, 256)
+    assert count % hkv == 0 and 0 <= count < 256
+    # Never the launch without a plan where every tile has a workgroup.
+    if tokens // (ops.PREFILL_STREAM_ROWS // (hq // hkv)) + len(pages) <= 1:
+        assert count > 0
+    # More decode never takes CUs away from it.
+    more = ops.mixed_prefill_workgroups(pages, tokens, 1000 * decode, hq, hkv, 256)
+    assert more <= count or count == 0
+    assert ops.mixed_prefill_workgroups((), 0, decode, hq, hkv, 256) == 0
+    with pytest.raises(ValueError):
+        ops.mixed_prefill_workgroups(pages, tokens, decode, hq, hkv + hq, 256)
+
+
 @pytest.mark.parametrize("seed", range(5))
 def test_decode_merge_list_names_every_split_segment_once(seed):
     rng = np.random.default_rng(300 + seed)
