@@ -558,31 +558,37 @@ constexpr int kPrefillPlanItemInts = 16;
 constexpr int kPrefillPlanDroppedInt = 1;
 constexpr int kPrefillPlanExitInt = 16;
 constexpr int kPrefillPlanGridInt = 17;
-// Batches of at most one item per workgroup of a head (the fixed form of the
-// launch): words 18 .. 21 = {pieces, word offsets into the plan buffer of the
-// piece list and the arrival counters, the partials' offset in
-// kPrefillPartUnit bytes}.  pieces > 0: the items are the pieces of the piece
-// list; 0: the tiles.
+// Words 18 .. 21 = {pieces, word offsets into the plan buffer of the piece list
+// and the arrival counters, the partials' offset in kPrefillPartUnit bytes}.
+// pieces > 0: the items of the plan are the pieces of the piece list, 0: the
+// tiles.
 constexpr int kPrefillPlanPiecesInt = 18;
 constexpr int kPrefillPlanPieceListInt = 19;
 constexpr int kPrefillPlanArriveInt = 20;
 constexpr int kPrefillPlanPartInt = 21;
+// Word 22: workgroups per KV head among which the items, longest first, are
+// dealt out in turns, or 0 where they are claimed.
+constexpr int kPrefillPlanTurnInt = 22;
 constexpr int kPrefillPlanLineInts = 32;
 constexpr int kPrefillPlanMaxHeads = 127;
 constexpr int kPrefillPlanHeaderInts = kPrefillPlanLineInts * (1 + kPrefillPlanMaxHeads);
-// A split-K piece: a tile record whose key counts, positions and pages are
-// those of the piece's keys, then {first page of the piece in the sequence,
-// pieces of the tile, the tile's first piece}.  Piece i of KV head h has
-// partial slot i * Hkv + h, and the tile's arrival counter is number
-// (first piece) * Hkv + h.
+// A piece: a tile record whose key counts, positions and pages are those of
+// the piece's keys, then {first page of the piece in the sequence, pieces of
+// the tile, slot of the tile's first piece, number of the piece in the tile}.
+// A tile of one piece has no slot.  Piece c of a tile with first slot s has,
+// for KV head h, partial (s + c) * Hkv + h and arrival counter s * Hkv + h.
 constexpr int kPrefillPieceInts = 32;
 constexpr int kPrefillPieceFirstPage = 16;
 constexpr int kPrefillPieceCount = 17;
 constexpr int kPrefillPieceFirst = 18;
+constexpr int kPrefillPieceOwn = 19;
 // A tile is cut into at most this many pieces (one workgroup reads all of a
-// tile's partials), and a plan has at most this many (piece, KV head) pairs.
+// tile's partials); a plan has at most kPrefillPieceSlots (slot, KV head)
+// pairs, and only plans of at most kPrefillCutTiles tiles are cut.
 constexpr int kPrefillMaxPieces = 8;
 constexpr int kPrefillPieceSlots = 256;
+constexpr int kPrefillCutTiles = 256;
+constexpr int kPrefillMaxItems = kPrefillCutTiles + kPrefillPieceSlots;
 // One partial: 64 floats of O, m and l of each of 512 threads.
 constexpr int kPrefillPartBytes = 512 * (64 + 2) * 4;
 constexpr int kPrefillPartUnit = 256;

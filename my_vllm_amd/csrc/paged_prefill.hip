@@ -29,7 +29,7 @@ namespace {
 constexpr int kMixedDecodeWaves = kPrefillPPThreads / 64;
 
 // Piece list and arrival counters, before the partials, in words.
-constexpr int64_t kPrefillSplitMetaInts = kPrefillPieceSlots * (kPrefillPieceInts + 1);
+constexpr int64_t kPrefillSplitMetaInts = kPrefillMaxItems * kPrefillPieceInts + kPrefillPieceSlots;
 static_assert(kPrefillSplitMetaInts * 4 % kPrefillPartUnit == 0, "partials stay aligned");
 // Word offset of the piece list of a plan of at most max_tiles tiles, and the
 // bytes of such a plan with its split-K area.
@@ -44,82 +44,147 @@ int64_t prefill_split_bytes(int64_t max_tiles) {
   return (prefill_piece_list(max_tiles) + kPrefillSplitMetaInts) * 4 + (int64_t)kPrefillPieceSlots * kPrefillPartBytes;
 }
 
-// Split-K pieces of the n planned tiles, for a batch whose tiles leave most
-// workgroups idle: returns their number, or 0 when whole tiles are as good.
-// A launch of few tiles lasts as long as its longest one (1.5 to 1.85 us per
-// 64 keys), so tiles longer than L key tiles are cut into near-equal pieces of
-// at most L.  L is ceil(longest / k) for the k in 1 .. kPrefillMaxPieces with
-// the smallest L + 2.5 + 0.75 k (key tiles; a split costs writing the partials
-// and one workgroup reading k of them: 4.7 and 5.3 us at k = 4 with all 256
-// workgroups busy), among those whose pieces fit one per workgroup.  All 1024 threads call it; nt, first and best are LDS
-// arrays of at least 1024 ints.  piece_list <= 0: no room for partials.
-__device__ int plan_pieces(int32_t* __restrict__ plan, int n, int per_head, int num_kv_heads,
+// Cuts the n planned tiles into split-K pieces where whole tiles would leave
+// workgroups idle; returns the number of items of the piece list (whole tiles
+// among them), or 0 when whole tiles are as good.  Tiles from number `start`
+// on that have more than L key tiles (64 keys, 1.5 to 1.85 us) are cut into
+// near-equal pieces of at most L; of 16 candidates the one with the lowest
+// estimate, in key tiles, is taken:
+//  * fixed (one item per workgroup; start 0, L = ceil(longest / k), k = 1 .. 8):
+//    L and, for a split, 2.5 + 0.75 k (writing the partials and one workgroup
+//    reading k of them: 4.7 and 5.3 us at k = 4 with all 256 workgroups busy);
+//  * claimed items, longest first.  An item costs 2.5 besides its keys, a
+//    split tile 3 and each of its pieces 2.75.  Long tiles cut (start 0, L =
+//    longest / (1 + c / 2), c = 0 .. 7): the largest of the work per workgroup
+//    and j + 1 times the length that more than j * per_head items have (whole
+//    tiles: exactly, otherwise of 3/4 and 1/2 of L).  Or the tiles past one or two whole rounds cut (start = per_head or twice
+//    that, where all tiles are sorted): the largest of the whole rounds and
+//    the work per workgroup and half a piece.  Plus 5, and a gain under a tenth
+//    is left.
+// Measured, whole and claimed / cut and in turns: 32 / 8 heads, a prompt of 2048
+// tokens (32 tiles of 1 to 32 for 32 workgroups a head) 59.6 / 52.8 us, 4
+// chunks of 512 over up to 8k 172 / 124, 4 of 560 over 4k 233 / 187; 64 / 8
+// heads, 4 of 280 over 7k 362 / 259; 16 / 8 heads, 6000 tokens 202 / 161.
+// All 1024 threads call it; nt, first, best and len are LDS arrays of at least
+// kPrefillMaxItems, 2 * kPrefillCutTiles + 2, 64 and kPrefillMaxItems ints.
+// piece_list <= 0: no room for partials.  The first `sorted` tiles or fewer
+// are longest first.
+__device__ int plan_pieces(int32_t* __restrict__ plan, int n, bool fixed, int per_head, int num_kv_heads,
                            const int32_t* __restrict__ block_tables, int64_t bt_stride, int64_t num_pages,
-                           int piece_list, int* nt, int* first, int* best) {
+                           int piece_list, int sorted, int* nt, int* first, int* best, int* len_of) {
   const int tid = threadIdx.x;
-  const int limit = min(per_head, kPrefillPieceSlots / num_kv_heads);
-  if (piece_list <= 0 || n == 0 || n > limit) return 0;  // limit <= kPrefillPieceSlots
+  const int slots = kPrefillPieceSlots / num_kv_heads;
+  if (piece_list <= 0 || n == 0 || n > (fixed ? min(per_head, slots) : kPrefillCutTiles)) return 0;
   const int32_t* tiles = plan + kPrefillPlanHeaderInts;
   __syncthreads();
   if (tid < n) nt[tid] = tiles[tid * kPrefillPlanItemInts + 5];
   __syncthreads();
-  // Wave k - 1 counts the pieces at k and prices them.
-  const int lane = tid & 63, k = (tid >> 6) + 1;
-  if (k <= kPrefillMaxPieces) {
-    int longest = 0;
-    for (int i = lane; i < n; i += 64) longest = max(longest, nt[i]);
+  // Wave c prices candidate c.
+  const int lane = tid & 63, c = tid >> 6;
+  auto wave_sum = [](int v) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
-    const int len = max((longest + k - 1) / k, 1);
-    int count = 0;
-    for (int i = lane; i < n; i += 64) count += (nt[i] + len - 1) / len;
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return v;
+  };
+  int longest = 0;
+  for (int i = lane; i < n; i += 64) longest = max(longest, nt[i]);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) count += __shfl_xor(count, off);
-    if (lane == 0) {
-      best[2 * k] = count > limit ? 0x7fffffff : k == 1 ? 4 * len : 4 * len + 10 + 3 * k;
-      best[2 * k + 1] = len;
-    }
+  for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
+  const int k = c + 1;
+  // Claimed items: candidates 0 .. 7 cut long tiles, 8 .. 15 the tiles past
+  // one (8 .. 11) or two (12 .. 15) rounds into 2, 4, 6 or 8.
+  const bool late = !fixed && c >= 8;
+  const int start = late ? per_head * (1 + ((c - 8) >> 2)) : 0;
+  int len = fixed ? (longest + k - 1) / k : (2 * longest + 1 + c) / (2 + c);
+  if (late) len = start < n ? (nt[start] + 2 * (c & 3) + 1) / (2 * (c & 3) + 2) : longest;
+  len = max(len, 1);
+  int items = 0, split = 0, work = 0, most = 0, half = 0, rounds = 0;
+  for (int i = lane; i < n; i += 64) {
+    const int cuts = i < start ? 1 : (nt[i] + len - 1) / len;
+    items += cuts;
+    split += cuts > 1 ? cuts : 0;
+    work += 4 * nt[i] + 10 * cuts + (cuts > 1 ? 12 + 11 * cuts : 0);
+    const int each = nt[i] / cuts;
+    most += 4 * each >= 3 * len ? cuts : 0;
+    half += 2 * each >= len ? cuts : 0;
+    if ((c == 0 || i < start) && i % per_head == 0) rounds = max(rounds, (i / per_head + 1) * (4 * nt[i] + 10));
+  }
+  items = wave_sum(items), split = wave_sum(split), work = wave_sum(work), most = wave_sum(most), half = wave_sum(half);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) rounds = max(rounds, __shfl_xor(rounds, off));
+  int price = 0x7fffffff;
+  if (fixed) {
+    if (k <= kPrefillMaxPieces && items <= min(per_head, slots)) price = k == 1 ? 4 * len : 4 * len + 10 + 3 * k;
+  } else if (late) {
+    if (n <= sorted && split > 0 && split <= slots) price = max(rounds, work / per_head + 2 * len) + 20;
+  } else if (split <= slots && (c == 0 || split > 0)) {
+    price = max(max(4 * len + 10, work / per_head),
+                max(((most - 1) / per_head + 1) * (3 * len + 10), ((half - 1) / per_head + 1) * (2 * len + 10)));
+    price += split > 0 ? 20 : 0;
+    if (c == 0 && n <= sorted) price = max(price, rounds);
+  }
+  if (lane == 0) {
+    best[3 * c] = price;
+    best[3 * c + 1] = len;
+    best[3 * c + 2] = start;
   }
   __syncthreads();
-  int pick = 1;
-  for (int c = 2; c <= kPrefillMaxPieces; ++c)
-    if (best[2 * c] < best[2 * pick]) pick = c;
-  if (pick == 1) return 0;
-  const int len = best[2 * pick + 1];
-  // First piece of each tile (n <= 256: wave 0 scans 64 tiles at a time).
+  int pick = 0;
+  for (int i = 1; i < 16; ++i)
+    if (best[3 * i] < best[3 * pick]) pick = i;
+  if (pick == 0 || (!fixed && 10 * (best[3 * pick] / 9) > best[0])) return 0;
+  const int cut = best[3 * pick + 1], from = best[3 * pick + 2];
+  // First item and first slot of each tile (wave 0 scans 64 tiles at a time;
+  // items in the low half, slots in the high half).
+  int* const slot_of = first + kPrefillCutTiles + 1;
   if (tid < 64) {
     int carry = 0;
-    for (int c = 0; c < n; c += 64) {
-      const int v = c + lane < n ? (nt[c + lane] + len - 1) / len : 0;
+    for (int i0 = 0; i0 < n; i0 += 64) {
+      const int i = i0 + lane;
+      const int cuts = i >= n ? 0 : i < from ? 1 : (nt[i] + cut - 1) / cut;
+      const int v = cuts + (cuts > 1 ? cuts << 16 : 0);
       int incl = v;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
         const int up = __shfl_up(incl, off);
         if (lane >= off) incl += up;
       }
-      if (c + lane < n) first[c + lane] = carry + incl - v;
+      if (i < n) {
+        first[i] = (carry + incl - v) & 0xffff;
+        slot_of[i] = (carry + incl - v) >> 16;
+      }
       carry += __shfl(incl, 63);
     }
-    if (lane == 0) first[n] = carry;
+    if (lane == 0) first[n] = carry & 0xffff;
   }
   __syncthreads();
-  const int total = first[n];
-  for (int i = tid; i < kPrefillPieceSlots; i += 1024) plan[piece_list + kPrefillPieceSlots * kPrefillPieceInts + i] = 0;
-  for (int i = tid; i < total; i += 1024) {
-    int lo = 0, hi = n - 1;  // last tile whose first piece is <= i
+  const int total = first[n];  // <= n + slots <= kPrefillMaxItems
+  for (int i = tid; i < kPrefillPieceSlots; i += 1024) plan[piece_list + kPrefillMaxItems * kPrefillPieceInts + i] = 0;
+  int lo = 0, cuts = 1, own = 0, a = 0, b = 0;
+  if (tid < total) {
+    int hi = n - 1;  // last tile whose first item is <= tid
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
-      if (first[mid] <= i) lo = mid;
+      if (first[mid] <= tid) lo = mid;
       else hi = mid - 1;
     }
-    const int cuts = first[lo + 1] - first[lo];
-    const int c = i - first[lo];
-    const int a = (int)((int64_t)c * nt[lo] / cuts), b = (int)((int64_t)(c + 1) * nt[lo] / cuts);
+    cuts = first[lo + 1] - first[lo];
+    own = tid - first[lo];
+    a = own * nt[lo] / cuts, b = (own + 1) * nt[lo] / cuts;
+    len_of[tid] = b - a;
+  }
+  __syncthreads();
+  if (tid < total) {
+    int at = tid;
+    if (!fixed) {  // longest first, ties in tile order
+      at = 0;
+      for (int o = 0; o < total; ++o) at += len_of[o] > b - a || (len_of[o] == b - a && o < tid);
+    }
     const int32_t* t = tiles + lo * kPrefillPlanItemInts;
     const int pages_per_tile = kPrefillKeys / kPageSize;
     const int npages = min(t[7] - a * pages_per_tile, (b - a) * pages_per_tile);
     const int32_t* bt = block_tables + (int64_t)t[0] * bt_stride + a * pages_per_tile;
-    int32_t* d = plan + piece_list + (int64_t)i * kPrefillPieceInts;
+    int32_t* d = plan + piece_list + (int64_t)at * kPrefillPieceInts;
     d[0] = t[0];
     d[1] = t[1];
     d[2] = t[2];
@@ -135,9 +200,27 @@ __device__ int plan_pieces(int32_t* __restrict__ plan, int n, int per_head, int 
     }
     d[kPrefillPieceFirstPage] = a * pages_per_tile;
     d[kPrefillPieceCount] = cuts;
-    d[kPrefillPieceFirst] = first[lo];
+    d[kPrefillPieceFirst] = cuts > 1 ? slot_of[lo] : 0;
+    d[kPrefillPieceOwn] = own;
   }
   return total;
+}
+
+// How a launch takes its items: claims; claims or turns, whole tiles or pieces
+// (kPieces); one item a workgroup.
+enum class PlanForm { kClaims, kTurns, kFixed };
+// Rounds of items dealt out in turns at most.  One prompt, 32 / 8 heads,
+// claimed / in turns: 3000 tokens (47 tiles for 32 workgroups a head) 114 / 95
+// us, 4096 (64) 165 / 135, 6000 (94) 287 / 281; 8 sequences of 300-600 over up
+// to 2k (59) 73 / 60; 64 / 8 heads, 2048 tokens (64) 90 / 72, 6000 (188) 533 /
+// 519.  At 7 rounds of 16 sequences claims were 2% faster: workgroups of a
+// faster XCD take more, and one sequence's pages are read together.
+constexpr int kPrefillTurns = 6;
+
+// The form of a plan of at most max_tiles tiles, on per_head workgroups a head.
+PlanForm plan_form(int64_t max_tiles, int64_t per_head) {
+  if (max_tiles <= per_head) return PlanForm::kFixed;
+  return max_tiles <= kPrefillTurns * per_head ? PlanForm::kTurns : PlanForm::kClaims;
 }
 
 // Exact tile list of a prefill batch, built on the device from
@@ -159,7 +242,7 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(const int32_t* __res
                                                             int64_t bt_stride, int64_t num_pages, int num_seqs,
                                                             int tile_tokens, int num_kv_heads,
                                                             int32_t* __restrict__ plan, int capacity, int tail,
-                                                            int grid, int per_head, int piece_list) {
+                                                            int grid, PlanForm form, int per_head, int piece_list) {
   // Sequences in plan order (rank -> sequence) and the first tile of each
   // rank; beyond kPrefillPlanSortMax sequences, all keep batch order and are
   // planned in passes of kPrefillPlanSortMax.
@@ -284,14 +367,17 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(const int32_t* __res
       }
     }
   }
-  const int pieces = plan_pieces(plan, min(carry, capacity), per_head, num_kv_heads, block_tables, bt_stride,
-                                 num_pages, piece_list, scan, first_tile, order);
+  const int n = min(carry, capacity);
+  const int pieces = plan_pieces(plan, n, form == PlanForm::kFixed, per_head, num_kv_heads, block_tables, bt_stride,
+                                 num_pages, piece_list, tail, scan, first_tile, order, kv_of);
   if (tid == 0) {
     plan[kPrefillPlanPiecesInt] = pieces;
     plan[kPrefillPlanPieceListInt] = piece_list;
-    plan[kPrefillPlanArriveInt] = piece_list + kPrefillPieceSlots * kPrefillPieceInts;
+    plan[kPrefillPlanArriveInt] = piece_list + kPrefillMaxItems * kPrefillPieceInts;
     plan[kPrefillPlanPartInt] = (int)((piece_list + kPrefillSplitMetaInts) / (kPrefillPartUnit / 4));
-    plan[0] = min(carry, capacity);
+    // All tiles are longest first where the sorted tail holds them.
+    plan[kPrefillPlanTurnInt] = form == PlanForm::kTurns && (pieces > 0 || n <= tail) ? per_head : 0;
+    plan[0] = n;
     plan[kPrefillPlanDroppedInt] = max(carry - capacity, 0);
     plan[kPrefillPlanExitInt] = 0;
     plan[kPrefillPlanGridInt] = grid;
@@ -307,7 +393,9 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(const int32_t* __res
 // (The grid size comes from the plan header, which keeps the dispatch
 // packet's registers out of the tile loop.)  Every thread of the workgroup
 // calls it.
+template <bool kPieces>
 __device__ __attribute__((always_inline)) inline void leave_prefill_plan(int32_t* plan) {
+  if (kPieces && sload(plan, kPrefillPlanTurnInt) > 0) return;  // nothing was claimed
   __syncthreads();
   if (threadIdx.x >= 64) return;
   int gone = 0;
@@ -326,17 +414,18 @@ __device__ __attribute__((always_inline)) inline void leave_prefill_plan(int32_t
 // ahead (prefill_items_pingpong), so the grid never waits on dispatch and
 // faster CUs simply run more tiles; once their head's queue is exhausted
 // they take the remaining tiles of the other heads.
-template <typename T>
+template <typename T, bool kPieces>
 __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_stream_kernel(PrefillParams p,
                                                                                  int32_t* __restrict__ plan) {
   __shared__ __attribute__((aligned(16))) uint8_t tiles[kPrefillPPLdsBytes];
-  __shared__ int nextq[4];
+  __shared__ int nextq[8];
   const int h = (int)(blockIdx.x % (uint32_t)p.num_kv_heads);
+  const int rank = kPieces ? (int)(blockIdx.x / (uint32_t)p.num_kv_heads) : 0;
   if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) == 0)
-    prefill_items_pingpong<T, 0, false>(p, plan, h, 0, (lds_u8*)tiles, (lds_i32*)nextq);
+    prefill_items_pingpong<T, 0, false, kPieces>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
   else
-    prefill_items_pingpong<T, 1, false>(p, plan, h, 0, (lds_u8*)tiles, (lds_i32*)nextq);
-  leave_prefill_plan(plan);
+    prefill_items_pingpong<T, 1, false, kPieces>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
+  leave_prefill_plan<kPieces>(plan);
 }
 
 // The fixed form, for a batch of at most one tile per workgroup of a head: no
@@ -349,9 +438,9 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_fixed_kernel(
   const int h = (int)(blockIdx.x % (uint32_t)p.num_kv_heads);
   const int rank = (int)(blockIdx.x / (uint32_t)p.num_kv_heads);
   if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) == 0)
-    prefill_items_pingpong<T, 0, true>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
+    prefill_items_pingpong<T, 0, true, true>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
   else
-    prefill_items_pingpong<T, 1, true>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
+    prefill_items_pingpong<T, 1, true, true>(p, plan, h, rank, (lds_u8*)tiles, (lds_i32*)nextq);
 }
 
 // A MIXED step on CUs of two kinds.  Workgroups of 512 threads, one per CU
@@ -396,10 +485,10 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_mixed_split_cus_kerne
   const int h = (int)(blockIdx.x % (uint32_t)pp.num_kv_heads);
   const int rank = (int)(blockIdx.x / (uint32_t)pp.num_kv_heads);
   if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) == 0)
-    prefill_items_pingpong<T, 0, kFixed>(pp, plan, h, rank, (lds_u8*)lds, (lds_i32*)nextq);
+    prefill_items_pingpong<T, 0, kFixed, true>(pp, plan, h, rank, (lds_u8*)lds, (lds_i32*)nextq);
   else
-    prefill_items_pingpong<T, 1, kFixed>(pp, plan, h, rank, (lds_u8*)lds, (lds_i32*)nextq);
-  if constexpr (!kFixed) leave_prefill_plan(plan);
+    prefill_items_pingpong<T, 1, kFixed, true>(pp, plan, h, rank, (lds_u8*)lds, (lds_i32*)nextq);
+  if constexpr (!kFixed) leave_prefill_plan<true>(plan);
 }
 
 static_assert(kMixedDecodeWaves * kDecodeWaveLdsBytes >= kPrefillPPLdsBytes, "prefill tiles fit the decode buffers");
@@ -642,7 +731,7 @@ extern "C" int mva_prefill_tile_tokens(int num_q_heads, int num_kv_heads) {
 extern "C" int64_t mva_prefill_workspace_bytes(int64_t max_tiles) {
   if (max_tiles < 0 || max_tiles > 0x7fffffffLL / mva::kPrefillPlanItemInts) return -1;
   // Up to this many tiles a plan may be cut into split-K pieces.
-  if (max_tiles <= mva::kPrefillPieceSlots) return mva::prefill_split_bytes(max_tiles);
+  if (max_tiles <= mva::kPrefillCutTiles) return mva::prefill_split_bytes(max_tiles);
   return mva::prefill_plan_bytes(max_tiles);
 }
 
@@ -656,16 +745,18 @@ const char kBadTileCapacity[] = "paged attention: invalid tile capacity";
 // `grid` workgroups that count themselves out of the plan.
 int launch_prefill_plan(const PrefillParams& p, int64_t num_seqs, int64_t max_tiles, int32_t* plan,
                         int64_t workspace_bytes, int64_t per_head, int64_t grid, hipStream_t s) {
-  // The last three tiles per workgroup of a head go largest first.
-  const int64_t last = 3 * (per_head < max_tiles ? per_head : max_tiles);
+  const PlanForm form = plan_form(max_tiles, per_head);
+  // All tiles of a plan dealt out in turns go largest first, otherwise the
+  // last three per workgroup of a head.
+  const int64_t last =
+      form == PlanForm::kTurns ? max_tiles : 3 * (per_head < max_tiles ? per_head : max_tiles);
   const int tail = (int)(last < 1024 ? last : 1024);
-  // A batch of at most one tile per workgroup may be split, where there is
-  // room for partials.
-  const bool split = max_tiles <= per_head && max_tiles <= kPrefillPieceSlots &&
+  // Tiles may be cut where there is room for partials.
+  const bool split = form != PlanForm::kClaims && max_tiles <= kPrefillCutTiles &&
                      workspace_bytes >= prefill_split_bytes(max_tiles);
   hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(1024), 0, s, p.query_start_loc, p.seq_lens, p.block_tables,
                      p.bt_stride, p.num_pages, (int)num_seqs, p.tile_tokens, p.num_kv_heads, plan, (int)max_tiles, tail,
-                     (int)grid, (int)per_head, split ? (int)prefill_piece_list(max_tiles) : 0);
+                     (int)grid, form, (int)per_head, split ? (int)prefill_piece_list(max_tiles) : 0);
   return check_launch("paged_prefill plan");
 }
 
@@ -708,25 +799,29 @@ int prefill_launch(const void* q, int64_t q_token_stride, int64_t q_head_stride,
   // they may be planned as pieces.
   int64_t per_head = (int64_t)device_cu_count() / num_kv_heads;
   per_head = per_head < 1 ? 1 : per_head;
-  // A batch of at most one tile per workgroup runs the fixed form.
-  const bool fixed = max_tiles <= per_head;
+  const PlanForm form = plan_form(max_tiles, per_head);
   if (plan_it) {
     rc = launch_prefill_plan(p, num_seqs, max_tiles, plan, workspace_bytes, per_head, per_head * num_kv_heads, s);
     if (rc) return rc;
   }
   if (!run_it) return 0;
   const dim3 grid((uint32_t)(per_head * num_kv_heads));
-  if (fixed) {
+  if (form == PlanForm::kFixed) {
     if (dtype == kBF16)
       hipLaunchKernelGGL(paged_prefill_fixed_kernel<__bf16>, grid, dim3(kPrefillPPThreads), 0, s, p, plan);
     else
       hipLaunchKernelGGL(paged_prefill_fixed_kernel<_Float16>, grid, dim3(kPrefillPPThreads), 0, s, p, plan);
     return check_launch("paged_prefill");
   }
-  if (dtype == kBF16)
-    hipLaunchKernelGGL(paged_prefill_stream_kernel<__bf16>, grid, dim3(kPrefillPPThreads), 0, s, p, plan);
-  else
-    hipLaunchKernelGGL(paged_prefill_stream_kernel<_Float16>, grid, dim3(kPrefillPPThreads), 0, s, p, plan);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kPrefillPPThreads), 0, s, p, plan); };
+  const bool pieces = form == PlanForm::kTurns;
+  if (dtype == kBF16) {
+    if (pieces) launch(paged_prefill_stream_kernel<__bf16, true>);
+    else launch(paged_prefill_stream_kernel<__bf16, false>);
+  } else {
+    if (pieces) launch(paged_prefill_stream_kernel<_Float16, true>);
+    else launch(paged_prefill_stream_kernel<_Float16, false>);
+  }
   return check_launch("paged_prefill");
 }
 
@@ -843,10 +938,11 @@ namespace {
 
 constexpr double kTileUs = 1.7;
 constexpr double kItemTiles = 2.5;
+constexpr double kCutTiles = 16.0;
 constexpr double kPrefillStartUs = 4.0;
 constexpr double kStreamUs = 5.0;  // claims, and decode workgroups joining in at the end
 constexpr double kDecodeStartUs = 6.0, kDecodeUsPerMB = 0.045, kDecodeUsPerMBCu = 26.3, kDecodeMinUsPerMB = 0.172;
-constexpr double kLittleDecode = 0.25;
+constexpr double kLittleDecode = 0.25, kShortTile = 8.0;
 constexpr int64_t kSortTiles = 4096;  // batches of more tiles are taken as even
 
 struct PrefillEstimate {
@@ -892,6 +988,9 @@ double prefill_part_us(const PrefillEstimate& e, int64_t per_head, int64_t max_t
       const double together = (double)(j + 1) * (e.keys[j * per_head] + kItemTiles);
       if (together > len) len = together;
     }
+    // Pieces in turns.
+    const double cut = e.work / (double)per_head + kItemTiles * ((double)e.tiles / (double)per_head) + kCutTiles;
+    if (plan_form(max_tiles, per_head) == PlanForm::kTurns && max_tiles <= kPrefillCutTiles && cut < len) len = cut;
     return kPrefillStartUs + kTileUs * len;
   }
   // plan_pieces' choice.
@@ -932,12 +1031,15 @@ extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, in
     const double us = (d > f ? d : f) + (max_tiles > p ? kStreamUs : 0.0);
     if (p == 1 || us < best_us) best = p, best_us = us;
   }
-  // Little decode beside more tiles than workgroups: the 128-row tiles of
-  // mva_paged_mixed, two to a CU, balance better.  32 / 8 heads, 4 chunks of
-  // 512 tokens over up to 8k and 4 decodes 213 against 272 us; 64 / 8 heads,
-  // 4 prompts of 350-614 tokens and 13 decodes 40 against 43 us, 4 chunks of
-  // 280 over 7k and 157 decodes of 372 357 against 366 us.
-  if (max_tiles > best && kDecodeStartUs + mb * kDecodeMinUsPerMB < kLittleDecode * best_us) return 0;
+  // Little decode beside many short tiles: the 128-row tiles of
+  // mva_paged_mixed, two to a CU, start sooner.  64 / 8 heads, 13 decodes of
+  // 176 and 4 prompts of 426-604 tokens 38.9 against 41.1 us; longer tiles or
+  // more decode run better on CUs of their own (32 / 8 heads, 4 chunks of 512
+  // over up to 8k and 4 decodes 218 / 204 us, a 2048-token prompt and 10
+  // decodes 66 / 60, 4 such prompts and 3 decodes 142 / 134).
+  if (max_tiles > best && e.work < kShortTile * (double)e.tiles &&
+      kDecodeStartUs + mb * kDecodeMinUsPerMB < kLittleDecode * best_us)
+    return 0;
   return best * num_kv_heads;
 }
 

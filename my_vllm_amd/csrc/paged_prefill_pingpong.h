@@ -42,11 +42,11 @@ struct StreamWork {
   int t0, q0, q_len, kv, ntiles, full_tiles, npages, pg0, pg1;
 };
 
-// Item `idx` of the plan's tile list (kFixed: of its piece list, when it has
+// Item `idx` of the plan's tile list (kPieces: of its piece list, when it has
 // one) with the page ids of page slot `slot` (0..3) of its 64-key tiles 0 and 1.
-template <bool kFixed>
+template <bool kPieces>
 __device__ inline StreamWork plan_work_slot(const PrefillParams& p, const int32_t* plan, int idx, int slot) {
-  const bool pieces = kFixed && sload(plan, kPrefillPlanPiecesInt) > 0;
+  const bool pieces = kPieces && sload(plan, kPrefillPlanPiecesInt) > 0;
   const int32_t* rec = pieces ? plan + sload(plan, kPrefillPlanPieceListInt) + (int64_t)idx * kPrefillPieceInts
                               : plan + kPrefillPlanHeaderInts + (int64_t)idx * kPrefillPlanItemInts;
   const i32x16 d = *(const_i32x16*)rec;
@@ -99,7 +99,7 @@ __device__ __attribute__((always_inline)) inline bool settle_piece(int32_t* plan
   char* const part = (char*)plan + (int64_t)sload(plan, kPrefillPlanPartInt) * kPrefillPartUnit;
   auto slot = [&](int piece) { return part + ((int64_t)piece * num_heads + head) * kPrefillPartBytes; };
   {
-    char* const mine = slot(idx);
+    char* const mine = slot(first + sload(rec, kPrefillPieceOwn));
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const f32x4 v = {o[j >> 2][4 * (j & 3)], o[j >> 2][4 * (j & 3) + 1], o[j >> 2][4 * (j & 3) + 2],
@@ -162,9 +162,18 @@ __device__ __attribute__((always_inline)) inline bool settle_piece(int32_t* plan
 // starts next; word 4 serves settle_piece.  `rank` is the workgroup's number
 // among those of head h0.
 //
-// kFixed: the launch has at least one workgroup per item of a head, workgroup
+// kPieces: the plan may hold split-K pieces.  kFixed: the launch has at least
+// one workgroup per item of a head, workgroup
 // `rank` of a head runs item `rank` of the piece or tile list and nothing
 // else, and what follows about claims and successors does not apply.
+//
+// Turns (kPieces, when the plan says so): of the items, longest first, the
+// workgroups of a head take one each in order, then one each in the opposite
+// order, and so on; workgroup `rank` knows its items without a claim.  A few
+// rounds are dealt out so (kPrefillTurns): a claim is made one item ahead,
+// when every workgroup of a short launch still runs its first item, so claims
+// pair the first workgroups to ask, not those with the shortest items, with
+// the next ones.
 //
 // Claims: a workgroup of KV head h0 claims from h0's counter.  Once that
 // queue is exhausted it reads every head's counter (one per lane of wave 0)
@@ -196,7 +205,7 @@ __device__ __attribute__((always_inline)) inline bool settle_piece(int32_t* plan
 // known: no plan read, query load, copy wait or claim sits between items.
 // Only when A has a single tile does group 1 copy V(B, 0) at B's start
 // (it is first read at B's phase 2, after the wait that ends phase 1).
-template <typename T, int kGrp, bool kFixed>
+template <typename T, int kGrp, bool kFixed, bool kPieces>
 __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(const PrefillParams& p, int32_t* plan,
                                                                              int h0, int rank, lds_u8* tiles, lds_i32* nextq) {
   typedef typename Elem<T>::v8 V8;
@@ -208,9 +217,10 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
   const int hi = lane >> 5;
   const int G = p.group;
   const int BMT = p.tile_tokens;  // 256 / G
-  const int n_pieces = kFixed ? sload(plan, kPrefillPlanPiecesInt) : 0;
+  const int n_pieces = kPieces ? sload(plan, kPrefillPlanPiecesInt) : 0;
   const int n_items = n_pieces > 0 ? n_pieces : sload(plan, 0);
   const int H = p.num_kv_heads;
+  const int turn = kPieces && !kFixed ? sload(plan, kPrefillPlanTurnInt) : 0;
   auto claim = [&](int head) {
     return __hip_atomic_fetch_add(plan + kPrefillPlanLineInts * (1 + head), 1, __ATOMIC_RELAXED,
                                   __HIP_MEMORY_SCOPE_AGENT);
@@ -338,7 +348,9 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
   int claim_head = h0;  // wave 0: the head claimed from last
   int claim_ret = 0;    // thread 0: the latest claim
   int idx = rank, cur_h = h0;
-  if constexpr (!kFixed) {
+  int after = 2 * turn - 1;  // turns: sum of this item's number and the next one's
+  if (turn > 0 && rank >= turn) return;
+  if (!kFixed && turn == 0) {
     if (w == 0) {
       int r = 0;
       if (lane == 0) r = claim(h0);
@@ -353,11 +365,11 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     cur_h = __builtin_amdgcn_readfirstlane(nextq[3]);
   }
   if (idx >= n_items) return;  // uniform: nothing for this workgroup
-  StreamWork cur = plan_work_slot<kFixed>(p, plan, idx, slot);
+  StreamWork cur = plan_work_slot<kPieces>(p, plan, idx, slot);
   // The page of the item's tile 2, which the item's first copies need; for
   // later items it is loaded during the item before (see below).
   int pg2_next = page_of_item(cur, 2);
-  if constexpr (!kFixed) {
+  if (!kFixed && turn == 0) {
     if (tid == 0) claim_ret = claim(claim_head);
   }
   load_q(cur, cur_h);
@@ -368,7 +380,7 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     copy_page(0, cur.pg0, cur_h);
   }
   __builtin_amdgcn_s_waitcnt(kVmcnt0);
-  if constexpr (!kFixed) {
+  if (!kFixed && turn == 0) {
     if (w == 0) {
       const int r = claim_on(claim_ret, claim_head);
       if (lane == 0) {
@@ -384,8 +396,8 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
   const std::true_type yes;
   const std::false_type no;
   while (true) {
-    const int nidx = kFixed ? n_items : __builtin_amdgcn_readfirstlane(nextq[1]);
-    const int nh = kFixed ? cur_h : __builtin_amdgcn_readfirstlane(nextq[2]);  // B's KV head
+    const int nidx = kFixed ? n_items : turn > 0 ? after - idx : __builtin_amdgcn_readfirstlane(nextq[1]);
+    const int nh = kFixed || turn > 0 ? cur_h : __builtin_amdgcn_readfirstlane(nextq[2]);  // B's KV head
     const bool has_next = !kFixed && nidx < n_items;
     const int n = cur.ntiles;
     const int full_tiles = cur.full_tiles;
@@ -397,7 +409,7 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     StreamWork nx;  // B's record, loaded at this item's first S phase
     nx.ntiles = 0;
     auto load_next = [&]() __attribute__((always_inline)) {
-      if (has_next) nx = plan_work_slot<kFixed>(p, plan, nidx, slot);
+      if (has_next) nx = plan_work_slot<kPieces>(p, plan, nidx, slot);
     };
     if constexpr (kGrp == 1) {
       if (!v0_done) copy_page(G0, cur.pg0, cur_h);
@@ -639,7 +651,7 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     if constexpr (kGrp == 0) {
       if (has_next) {
         load_q(nx, nh);
-        if (tid == 0) claim_ret = claim(claim_head);
+        if (tid == 0 && turn == 0) claim_ret = claim(claim_head);
       }
       issue(n);
       phase_m(n, no, yes);
@@ -647,7 +659,7 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
       // B's tile-2 page, loaded while this group waits for group 1's M(n).
       if (has_next) pg2_next = page_of_item(nx, 2);
       __builtin_amdgcn_s_waitcnt(kVmcnt0);
-      if (w == 0 && has_next) {
+      if (w == 0 && has_next && turn == 0) {
         const int r = claim_on(claim_ret, claim_head);
         if (lane == 0) {
           nextq[1] = r;
@@ -671,7 +683,7 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     // workgroup that finishes it.
     float l_tot = pair_sum(l);
     bool done = true;
-    if constexpr (kFixed) {
+    if constexpr (kPieces) {
       if (n_pieces > 0) done = settle_piece(plan, idx, cur_h, H, o, m, l_tot, nextq + 4);
     }
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
@@ -710,6 +722,10 @@ __device__ __attribute__((always_inline)) inline void prefill_items_pingpong(con
     v0_done = n >= 2;
     cur = nx;
     cur_h = nh;
+    if constexpr (kPieces) {
+      idx = nidx;
+      after += 2 * turn;
+    }
   }
 }
 

@@ -476,3 +476,47 @@ def test_split_key_ranges(gpu, hq, hkv, dtype, q, kv):
     # The merge takes a tile's pieces in key order, whichever ends last.
     assert all(torch.equal(out, outs[0]) for out in outs[:4])
     assert torch.equal(outs[4], outs[5])
+
+
+# Between one and six tiles per workgroup of a head they are dealt out in
+# turns, longest first, whole or cut (word 22 of the plan: the workgroups of a
+# head); beyond that they are claimed (0).  16 heads leave 16 workgroups a head.
+@pytest.mark.parametrize("q,kv,turns,cut", [
+    ([64, 512, 31], [64 * 60, 512, 31 + 64], True, True),      # a few long tiles
+    ([32 * 17], [32 * 17 + 64 * 40 - 5], True, True),          # one tile past a round
+    ([32 * 32 + 1], [32 * 32 + 1 + 64 * 64], True, True),      # past two rounds
+    ([32 * 40], [32 * 40], True, None),                        # whole tiles of 1 .. 20
+    ([5] * 96, [5 + 16 * i for i in range(96)], True, None),   # the most in turns
+    ([5] * 97, [5 + 16 * i for i in range(97)], False, False),  # claimed
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tiles_in_turns(gpu, q, kv, turns, cut, dtype):
+    hq, hkv = 128, 16
+    per_head = torch.cuda.get_device_properties(gpu).multi_processor_count // hkv
+    if per_head != 16:
+        pytest.skip("sizes are those of 256 CUs")
+    batch = make_paged_batch(229, q, kv, len(q), hq, hkv, dtype=dtype)
+    common, qd, kc, vc = to_device(batch, gpu)
+    n_tiles = sum(-(-n // 32) for n in q)
+    full = ops.prefill_workspace_bytes(n_tiles)
+    plan_only = 4 * (ops.PREFILL_PLAN_HEADER_INTS + n_tiles * ops.PREFILL_PLAN_ITEM_INTS)
+    outs = []
+    for nbytes in (full, plan_only):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
+        for planned in (False, True, True):
+            out = torch.full_like(qd, float("nan"))
+            ops.paged_prefill(qd, kc, vc, common.block_tables, common.seq_lens, common.query_start_loc, len(q),
+                              n_tiles, ws, out, 128 ** -0.5, planned=planned)
+            outs.append(out)
+        words = ws[:96].view(torch.int32).tolist()
+        assert words[0] == n_tiles and words[22] == (per_head if turns else 0)
+        if nbytes == plan_only:
+            assert words[18] == 0
+        elif cut is not None:
+            assert (words[18] > n_tiles) == cut
+    # Whole tiles against the oracle (the largest case would take it minutes),
+    # cut ones against whole ones.
+    want = expected(batch) if sum(q) * max(kv) < 3_000_000 else outs[3].float()
+    for i, out in enumerate(outs):
+        assert torch.equal(out, outs[i // 3 * 3])
+        assert_attention_close(out, want)
