@@ -211,6 +211,7 @@ def make_decode_plan(
 # Workgroups of a piece-list decode launch fill 8 wave slots per CU (the
 # kernel's occupancy is 2 wavefronts per SIMD).
 _LISTED_WAVES_PER_CU = 8
+_MAX_RANGES_PER_SEQ = 512
 # Piece lists (an equal share of pages per wavefront, no claims) at every
 # size when a workgroup holds all 8 KV heads of its range (one CU streams
 # every head of the same pages): measured as fast as claims or faster from
@@ -246,6 +247,31 @@ def listed_decode_groups(num_kv_heads: int, device: torch.device | None = None,
     per_group = num_kv_heads if num_kv_heads in (1, 2, 4, 8) else 1
     waves = max(1, int(override)) if override else _num_cus(device) * _LISTED_WAVES_PER_CU
     return max(1, waves // num_kv_heads), per_group
+
+
+def decode_ranges(total_pages: int, num_seqs: int, num_kv_heads: int,
+                  device: torch.device | None = None) -> tuple[int, int]:
+    """:func:`listed_decode_groups` for a decode batch of its own launch, with
+    fewer ranges where those are faster.
+
+    With one or two KV heads a batch is cut into 2048 or 1024 ranges: many
+    split-K chunks a sequence, and a merge takes 256 of them a memory round
+    trip.  Beyond 512 ranges a sequence more are slower (call, K/V not in any
+    cache, microseconds: 1 sequence of 32000 tokens at 8 / 1 heads, 2000 / 512
+    ranges 25.8 / 16.2, at 16 / 2, 1024 / 512 23.0 / 19.5; 16000 at 8 / 1, 1000 /
+    512 16.8 / 13.8).  And where a range holds two pages or more, six (two KV
+    heads) or four (one) wavefronts per CU read as fast as eight and leave
+    fewer chunks: 16 / 2 heads, 4 of 28000-32000 35.8 / 32.6, 37 of 300-6000
+    35.6 / 34.1; 8 / 1, 2 of 30000 22.8 / 19.4, 64 of 128-2048 20.5 / 19.3, but
+    128 of 100-300 (1.6 pages a range) at 16 / 2 18.7 / 19.4.  At 16 / 4 heads
+    four and eight are level (37 of 300-6000 54.3 / 54.6).
+    """
+    groups, waves_per_group = listed_decode_groups(num_kv_heads, device)
+    if num_kv_heads <= 2:
+        if total_pages >= 2 * groups:
+            groups = groups // 2 if num_kv_heads == 1 else groups * 3 // 4
+        groups = min(groups, _MAX_RANGES_PER_SEQ * num_seqs)
+    return groups, waves_per_group
 
 
 def plan_decode_listed(
@@ -697,8 +723,12 @@ class MI355XAttentionBackendMixin:
                 schedule = decode_schedule(int(decode_counts.sum()), self.num_kv_heads,
                                            forced=self.decode_schedule_override)
                 if schedule == "listed":
-                    groups, waves_per_group = listed_decode_groups(self.num_kv_heads, block_tables.device,
-                                                                   override=self.decode_waves_override)
+                    if self.decode_waves_override:
+                        groups, waves_per_group = listed_decode_groups(self.num_kv_heads, block_tables.device,
+                                                                       override=self.decode_waves_override)
+                    else:
+                        groups, waves_per_group = decode_ranges(int(decode_counts.sum()), len(decode_counts),
+                                                                self.num_kv_heads, block_tables.device)
                     items, wave_extra, num_decode_waves, num_part_slots, merges = plan_decode_listed(
                         decode_counts, common.num_prefill_seqs, common.num_prefill_tokens, self.num_kv_heads, groups
                     )

@@ -18,8 +18,10 @@ from my_vllm_amd.attention_backend import (
     MI355XAttentionBackend,
     MI355XAttentionMetadata,
     MI355XSplitAttentionBackend,
+    decode_ranges,
     decode_schedule,
     integrate,
+    listed_decode_groups,
     make_decode_plan,
     make_decode_plan_listed,
 )
@@ -506,6 +508,18 @@ def test_mixed_prefill_workgroups_leave_cus_for_decode(hq, hkv, pages, tokens, d
     assert ops.mixed_prefill_workgroups((), 0, decode, hq, hkv, 256) == 0
     with pytest.raises(ValueError):
         ops.mixed_prefill_workgroups(pages, tokens, decode, hq, hkv + hq, 256)
+
+
+@pytest.mark.parametrize("hkv", [1, 2, 3, 4, 8, 16])
+@pytest.mark.parametrize("pages,seqs", [(1, 1), (511, 1), (513, 1), (1791, 2), (1792, 2), (2000, 1), (60000, 300)])
+def test_decode_ranges_stay_within_the_full_launch(hkv, pages, seqs):
+    most, per_group = listed_decode_groups(hkv)
+    groups, per = decode_ranges(pages, seqs, hkv)
+    assert per == per_group and most // 4 <= groups <= most
+    if hkv > 2:
+        assert groups == most
+    else:
+        assert groups <= 512 * seqs and (pages >= 2 * most or groups == min(most, 512 * seqs))
 
 
 @pytest.mark.parametrize("seed", range(5))
