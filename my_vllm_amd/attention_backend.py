@@ -262,7 +262,7 @@ def decode_ranges(total_pages: int, num_seqs: int, num_kv_heads: int,
     512 16.8 / 13.8).  And where a range holds two pages or more, six (two KV
     heads) or four (one) wavefronts per CU read as fast as eight and leave
     fewer chunks: 16 / 2 heads, 4 of 28000-32000 35.8 / 32.6, 37 of 300-6000
-    35.6 / 34.1; 8 / 1, 2 of 30000 22.8 / 19.4, 64 of 128-2048 20.5 / 19.3, but
+    35.6 / 34.1; 8 / 1, 4 of 30000 26.0 / 24.4, 64 of 128-2048 20.5 / 19.3, but
     128 of 100-300 (1.6 pages a range) at 16 / 2 18.7 / 19.4.  At 16 / 4 heads
     four and eight are level (37 of 300-6000 54.3 / 54.6).
     """

@@ -460,8 +460,8 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_fixed_kernel(
 // decode set its time until HBM does (5.8 TB/s), and the prefill CUs slow
 // down beside it (power and L2).  Against paged_mixed_kernel, microseconds of
 // a step: 300 tokens over 1936 and 20 decodes of 2250 (32 / 8 heads, fp16)
-// 69 -> 47, 2 chunks over 4k and 64 decodes of 2700 211 -> 187, 4 chunks of a
-// budget of 8192 and 256 decodes of 4391 965 -> 945, 1 decode of 12695 beside
+// 69 -> 47, 2 chunks over 4k and 64 decodes of 2700 211 -> 176, 4 chunks of a
+// budget of 8192 and 256 decodes of 4391 974 -> 914, 1 decode of 12695 beside
 // 109 prompt tokens (64 / 8 heads) 168 -> 20.  Split-K decode segments are
 // merged by the merge kernel that follows: merging inside the launch cost 5
 // to 17 us more (the merges run one after another on the last wavefronts).
