@@ -1,9 +1,9 @@
 """MIXED batches: single-launch (MIXED_UNIFIED) and split (MIXED_SPLIT) routes.
 
-Both routes run the same prefill code, so the prefill rows must be bitwise
-identical; the split route's decode half runs the piece-list schedule (a
-different split-K partition than the single launch's claims), so decode
-rows agree within the attention tolerance.  Both are checked against the
+Both routes run the same prefill arithmetic, so the prefill rows must be
+bitwise identical where neither cuts a tile; their decode halves are cut
+differently (ranges for all CUs, ranges for the CUs that prefill leaves, or
+claims), so decode rows agree within the attention tolerance.  Both are checked against the
 fp32 oracle (2e-2 / 1e-2).
 The split route writes ``out[:P]`` and ``out[P:]`` of one buffer without
 concatenation.  GQA ratios 1, 3 and 8 and fp16 run on both routes.
