@@ -56,10 +56,31 @@ void* ptr(const Tensor& t) { return t.data_ptr(); }
 
 PyObject* none() { Py_RETURN_NONE; }
 
+// The status of `launch`, run without the GIL, as a ctypes call runs it: a
+// launch that waits for room in a full queue stops no other Python thread, and
+// none that a host callback in the queue waits for.  The arguments are read
+// before it is released.
+template <typename... P, typename... A>
+int unlocked(int (*launch)(P...), A... args) {
+  struct Released {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  return launch(args...);
+}
+
+// `result` (a new reference) when the launch went out, else its error.
 PyObject* launched(const char* name, int status, PyObject* result) {
   if (status == 0) return result;
   Py_XDECREF(result);
   return PyErr_Format(PyExc_RuntimeError, "%s failed (%d): %s", name, status, mva_last_error());
+}
+PyObject* launched(const char* name, int status) {
+  Py_INCREF(Py_True);
+  return launched(name, status, Py_True);
+}
+PyObject* launched(const char* name, int status, const Tensor& out) {
+  return launched(name, status, status == 0 ? THPVariable_Wrap(out) : nullptr);
 }
 
 // Integer and float arguments; false (no Python error left) when one is not.
@@ -113,9 +134,9 @@ PyObject* silu_and_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
     c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
     shape.back() = width / 2;
     const Tensor out = at::empty(shape, x->options().requires_grad(false));
-    return launched("mva_silu_and_mul",
-                    mva_silu_and_mul(ptr(*x), ptr(out), x->numel() / width, width / 2, code, stream_of(*x)),
-                    THPVariable_Wrap(out));
+    void* const stream = stream_of(*x);
+    const int status = unlocked(mva_silu_and_mul, ptr(*x), ptr(out), x->numel() / width, width / 2, code, stream);
+    return launched("mva_silu_and_mul", status, out);
   });
 }
 
@@ -137,10 +158,11 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t row_stride = heads ? x->stride(1) : x->size(0) > 1 ? x->stride(0) : hidden;
     const int64_t group_stride = heads ? x->stride(0) : row_stride;
     const Tensor out = at::empty(x->sizes(), x->options().requires_grad(false));
-    return launched("mva_rms_norm",
-                    mva_rms_norm(ptr(*x), group_stride, row_stride, ptr(*w), ptr(out), per_group * hidden, hidden,
-                                 rows, per_group, hidden, (float)eps, code, wcode, stream_of(*x)),
-                    THPVariable_Wrap(out));
+    void* const stream = stream_of(*x);
+    const int status = unlocked(
+        mva_rms_norm, ptr(*x), group_stride, row_stride, ptr(*w), ptr(out), per_group * hidden, hidden, rows,
+        per_group, hidden, (float)eps, code, wcode, stream);
+    return launched("mva_rms_norm", status, out);
   });
 }
 
@@ -163,9 +185,10 @@ PyObject* fused_add_rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const auto options = x->options().requires_grad(false);
     const Tensor out = inplace ? *x : at::empty(x->sizes(), options);
     const Tensor res = inplace ? *r : at::empty(x->sizes(), options);
-    const int status = mva_fused_add_rms_norm(ptr(*x), xs, ptr(*r), rs, ptr(*w), ptr(out), inplace ? xs : hidden,
-                                              ptr(res), inplace ? rs : hidden, rows, hidden, (float)eps, code, wcode,
-                                              stream_of(*x));
+    void* const stream = stream_of(*x);
+    const int status = unlocked(
+        mva_fused_add_rms_norm, ptr(*x), xs, ptr(*r), rs, ptr(*w), ptr(out), inplace ? xs : hidden, ptr(res),
+        inplace ? rs : hidden, rows, hidden, (float)eps, code, wcode, stream);
     if (status != 0) return launched("mva_fused_add_rms_norm", status, nullptr);
     if (inplace) return PyTuple_Pack(2, a[0], a[1]);
     PyObject* pair = PyTuple_New(2);
@@ -225,14 +248,14 @@ PyObject* qk_norm_rope_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
           c->size(2) != k->size(1) || c->size(3) != kHeadDim || !c->is_contiguous())
         return none();
     if (kc->sizes() != vc->sizes() || !slot_list(*slots, *q, tokens)) return none();
-    const int status = mva_qk_norm_rope_store(
-        ptr(*q), ptr(*qo), q->stride(0), q->stride(1), (int)q->size(1), ptr(*k), ptr(*ko), k->stride(0), k->stride(1),
-        ptr(*v), v->stride(0), v->stride(1), (int)k->size(1), (const int64_t*)ptr(*pos), (const float*)ptr(*table),
-        table->size(0), kHeadDim, norm ? ptr(*wq) : nullptr, norm ? ptr(*wk) : nullptr, wcode, (float)eps, ptr(*kc),
-        ptr(*vc), kc->size(0) * kc->size(1), ptr(*slots), slots->scalar_type() == at::kLong, tokens, kHeadDim, code,
-        stream_of(*q));
-    Py_INCREF(Py_True);
-    return launched("mva_qk_norm_rope_store", status, Py_True);
+    void* const stream = stream_of(*q);
+    const int status = unlocked(
+        mva_qk_norm_rope_store, ptr(*q), ptr(*qo), q->stride(0), q->stride(1), (int)q->size(1), ptr(*k), ptr(*ko),
+        k->stride(0), k->stride(1), ptr(*v), v->stride(0), v->stride(1), (int)k->size(1), (const int64_t*)ptr(*pos),
+        (const float*)ptr(*table), table->size(0), kHeadDim, norm ? ptr(*wq) : nullptr, norm ? ptr(*wk) : nullptr,
+        wcode, (float)eps, ptr(*kc), ptr(*vc), kc->size(0) * kc->size(1), ptr(*slots),
+        slots->scalar_type() == at::kLong, tokens, kHeadDim, code, stream);
+    return launched("mva_qk_norm_rope_store", status);
   });
 }
 
@@ -260,7 +283,7 @@ struct Paged {
 };
 
 int64_t nbytes(const Tensor* t) { return t ? t->numel() * (int64_t)t->element_size() : 0; }
-void* ptr_or_null(const Tensor* t) { return t ? ptr(*t) : nullptr; }
+const int32_t* words(const Tensor* t) { return t ? (const int32_t*)ptr(*t) : nullptr; }
 
 // (q, k_cache, v_cache, block_tables, seq_lens, items, num_items, num_waves,
 //  merges | None, num_merges, num_part_slots, out, workspace, scale,
@@ -281,12 +304,11 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* const stream = stream_of(q);
     int status;
     if (n == 16) {
-      status = mva_paged_decode(
-          ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0), kc.stride(1),
-          (const int32_t*)ptr(*p.bt), p.bt->stride(0), (const int32_t*)ptr(*p.sl), (const int32_t*)ptr(*items), items_n,
-          waves, (const int32_t*)ptr_or_null(extra), (int)per_group, (const int32_t*)ptr_or_null(merges), merges_n,
-          slots_n, ptr(out), out.stride(0), out.stride(1), ptr(*ws), nbytes(ws), (int)q.size(1), (int)kc.size(2),
-          (int)q.size(2), (int)kc.size(1), (float)scale, p.code, stream);
+      status = unlocked(
+          mva_paged_decode, ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0),
+          kc.stride(1), words(p.bt), p.bt->stride(0), words(p.sl), words(items), items_n, waves, words(extra),
+          (int)per_group, words(merges), merges_n, slots_n, ptr(out), out.stride(0), out.stride(1), ptr(*ws),
+          nbytes(ws), (int)q.size(1), (int)kc.size(2), (int)q.size(2), (int)kc.size(1), (float)scale, p.code, stream);
     } else {
       const Tensor *k = plain(a[16]), *v = plain(a[17]), *slots = plain(a[18]);
       if (!extra || !k || !v || !slots || k->sizes() != v->sizes() || k->dim() != 3 || k->size(1) != kc.size(2) ||
@@ -294,16 +316,15 @@ PyObject* paged_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
           k->device() != q.device() || v->device() != q.device() || k->stride(2) != 1 || v->stride(2) != 1 ||
           !slot_list(*slots, q, k->size(0)))
         return none();
-      status = mva_paged_decode_store(
-          ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0), kc.stride(1),
-          (const int32_t*)ptr(*p.bt), p.bt->stride(0), (const int32_t*)ptr(*p.sl), (const int32_t*)ptr(*items), items_n,
-          waves, (const int32_t*)ptr(*extra), (int)per_group, (const int32_t*)ptr_or_null(merges), merges_n, slots_n,
-          ptr(out), out.stride(0), out.stride(1), ptr(*ws), nbytes(ws), ptr(*k), k->stride(0), k->stride(1), ptr(*v),
-          v->stride(0), v->stride(1), ptr(*slots), slots->scalar_type() == at::kLong, k->size(0), (int)q.size(1),
-          (int)kc.size(2), (int)q.size(2), (int)kc.size(1), (float)scale, p.code, stream);
+      status = unlocked(
+          mva_paged_decode_store, ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0),
+          kc.stride(1), words(p.bt), p.bt->stride(0), words(p.sl), words(items), items_n, waves, words(extra),
+          (int)per_group, words(merges), merges_n, slots_n, ptr(out), out.stride(0), out.stride(1), ptr(*ws),
+          nbytes(ws), ptr(*k), k->stride(0), k->stride(1), ptr(*v), v->stride(0), v->stride(1), ptr(*slots),
+          slots->scalar_type() == at::kLong, k->size(0), (int)q.size(1), (int)kc.size(2), (int)q.size(2),
+          (int)kc.size(1), (float)scale, p.code, stream);
     }
-    Py_INCREF(Py_True);
-    return launched(n == 16 ? "mva_paged_decode" : "mva_paged_decode_store", status, Py_True);
+    return launched(n == 16 ? "mva_paged_decode" : "mva_paged_decode_store", status);
   });
 }
 
@@ -321,13 +342,13 @@ PyObject* paged_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return none();
     const bool planned = a[11] == Py_True;
     const Tensor &q = *p.q, &kc = *p.kc, &out = *p.out;
-    const int status = (planned ? mva_paged_prefill_run : mva_paged_prefill)(
-        ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0), kc.stride(1),
-        (const int32_t*)ptr(*p.bt), p.bt->stride(0), (const int32_t*)ptr(*p.sl), (const int32_t*)ptr(*qsl), seqs, tiles,
+    void* const stream = stream_of(q);
+    const int status = unlocked(
+        planned ? mva_paged_prefill_run : mva_paged_prefill, ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc),
+        kc.size(0), kc.stride(0), kc.stride(1), words(p.bt), p.bt->stride(0), words(p.sl), words(qsl), seqs, tiles,
         ptr(*ws), nbytes(ws), ptr(out), out.stride(0), out.stride(1), (int)q.size(1), (int)kc.size(2), (int)q.size(2),
-        (int)kc.size(1), (float)scale, p.code, stream_of(q));
-    Py_INCREF(Py_True);
-    return launched(planned ? "mva_paged_prefill_run" : "mva_paged_prefill", status, Py_True);
+        (int)kc.size(1), (float)scale, p.code, stream);
+    return launched(planned ? "mva_paged_prefill_run" : "mva_paged_prefill", status);
   });
 }
 
@@ -347,30 +368,28 @@ PyObject* paged_mixed(PyObject*, PyObject* const* a, Py_ssize_t n) {
         !as_float(a[14], &scale))
       return none();
     const Tensor &q = *p.q, &kc = *p.kc, &out = *p.out;
+    void* const stream = stream_of(q);
     int status;
     if (n == 15) {
-      status = mva_paged_mixed(
-          ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0), kc.stride(1),
-          (const int32_t*)ptr(*p.bt), p.bt->stride(0), (const int32_t*)ptr(*p.sl), (const int32_t*)ptr(*qsl), seqs,
-          tiles, (const int32_t*)ptr_or_null(items), items_n, waves, slots_n, ptr(out), out.stride(0), out.stride(1),
-          ptr(*ws), nbytes(ws), (int)q.size(1), (int)kc.size(2), (int)q.size(2), (int)kc.size(1), (float)scale, p.code,
-          stream_of(q));
+      status = unlocked(
+          mva_paged_mixed, ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0),
+          kc.stride(1), words(p.bt), p.bt->stride(0), words(p.sl), words(qsl), seqs, tiles, words(items), items_n,
+          waves, slots_n, ptr(out), out.stride(0), out.stride(1), ptr(*ws), nbytes(ws), (int)q.size(1),
+          (int)kc.size(2), (int)q.size(2), (int)kc.size(1), (float)scale, p.code, stream);
     } else {
       const Tensor *pws = plain(a[16]), *extra = plain(a[18]), *merges = plain(a[19]);
       int64_t workgroups, merges_n;
       if (!items || !p.bytes(pws) || !p.ints(extra) || !p.ints(merges) || !as_int(a[15], &workgroups) ||
           !PyBool_Check(a[17]) || !as_int(a[20], &merges_n))
         return none();
-      status = mva_paged_mixed_run(
-          ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0), kc.stride(1),
-          (const int32_t*)ptr(*p.bt), p.bt->stride(0), (const int32_t*)ptr(*p.sl), (const int32_t*)ptr(*qsl), seqs,
-          tiles, workgroups, ptr(*pws), nbytes(pws), a[17] == Py_True, (const int32_t*)ptr(*items), items_n, waves,
-          (const int32_t*)ptr(*extra), (const int32_t*)ptr(*merges), merges_n, slots_n, ptr(out), out.stride(0),
-          out.stride(1), ptr(*ws), nbytes(ws), (int)q.size(1), (int)kc.size(2), (int)q.size(2), (int)kc.size(1),
-          (float)scale, p.code, stream_of(q));
+      status = unlocked(
+          mva_paged_mixed_run, ptr(q), q.stride(0), q.stride(1), ptr(kc), ptr(*p.vc), kc.size(0), kc.stride(0),
+          kc.stride(1), words(p.bt), p.bt->stride(0), words(p.sl), words(qsl), seqs, tiles, workgroups, ptr(*pws),
+          nbytes(pws), a[17] == Py_True, words(items), items_n, waves, words(extra), words(merges), merges_n, slots_n,
+          ptr(out), out.stride(0), out.stride(1), ptr(*ws), nbytes(ws), (int)q.size(1), (int)kc.size(2),
+          (int)q.size(2), (int)kc.size(1), (float)scale, p.code, stream);
     }
-    Py_INCREF(Py_True);
-    return launched(n == 15 ? "mva_paged_mixed" : "mva_paged_mixed_run", status, Py_True);
+    return launched(n == 15 ? "mva_paged_mixed" : "mva_paged_mixed_run", status);
   });
 }
 
