@@ -281,8 +281,11 @@ def host_ops() -> ModuleType:
 
 
 def native_available() -> bool:
+    """Whether both parts of the native code load: the library, and the module
+    that launches through it."""
     try:
         load_library()
+        host_ops()
     except RuntimeError:
         return False
     return True

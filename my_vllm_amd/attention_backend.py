@@ -580,7 +580,8 @@ class MI355XAttentionBackendMixin:
         if not arch.startswith("gfx950"):
             return f"a gfx950 (MI355X) device is required, found {arch or 'unknown'}"
         if not _native.native_available():
-            return f"native library unavailable ({_native.LIB_PATH}); run `python -m my_vllm_amd.build`"
+            return (f"native library unavailable ({_native.LIB_PATH} and {_native.HOST_PATH.name}); "
+                    "run `python -m my_vllm_amd.build`")
         return None
 
     @property

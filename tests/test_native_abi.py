@@ -130,3 +130,18 @@ def test_stale_library_without_a_new_entry_point_asks_for_a_rebuild(monkeypatch)
     with pytest.raises(RuntimeError, match="rebuild"):
         _native.load_library()
     assert _native.native_available() is False
+
+
+def test_missing_or_stale_host_module_makes_the_native_code_unavailable(monkeypatch, tmp_path):
+    # Every operator launches through the module, so without it (or with one
+    # of another revision or Python) the platform check must say no.
+    monkeypatch.setattr(_native, "_host", None)
+    assert _native.native_available() is True
+    for content in (None, b"not a module"):
+        monkeypatch.setattr(_native, "_host", None)
+        monkeypatch.setattr(_native, "HOST_PATH", tmp_path / "mva_host.so")
+        if content is not None:
+            _native.HOST_PATH.write_bytes(content)
+        with pytest.raises(RuntimeError, match="my_vllm_amd.build"):
+            _native.host_ops()
+        assert _native.native_available() is False
