@@ -24,6 +24,7 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC_DIR = PACKAGE_DIR / "csrc"
 LIB_DIR = PACKAGE_DIR / "lib"
 LIB_PATH = LIB_DIR / "libmy_vllm_amd.so"
+HOST_PATH = LIB_DIR / "mva_host.so"
 BUILD_DIR = PACKAGE_DIR / "_build"
 
 OFFLOAD_ARCH = "gfx950"
@@ -69,36 +70,36 @@ def _compile(hipcc: str, source: Path, obj: Path) -> None:
         )
 
 
-def _build_host_module() -> None:
+def _build_host_module(target: Path) -> None:
     """Compile ``csrc/host_ops.cpp`` (host code only) against torch's headers
-    into ``lib/mva_host.so``, bound to the library beside it."""
+    into ``target``, bound to the library beside it."""
     import torch
 
     from . import _native
 
     root = Path(torch.__file__).resolve().parent
-    target = _native.HOST_PATH
-    fd, tmp = tempfile.mkstemp(prefix=".mva_host.", suffix=".so.tmp", dir=LIB_DIR)
-    os.close(fd)
     cmd = [
         os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++") or "g++",
         "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
         "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-DMVA_HOST_ABI_VERSION={_native.ABI_VERSION}",
         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
         f"-I{root / 'include'}", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
-        str(CSRC_DIR / "host_ops.cpp"), "-o", tmp,
+        str(CSRC_DIR / "host_ops.cpp"), "-o", str(target),
         f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
-        f"-L{LIB_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN",
+        f"-L{target.parent}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN",
     ]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
-        os.unlink(tmp)
         raise RuntimeError(f"{cmd[0]} failed for host_ops.cpp:\n{proc.stdout}\n{proc.stderr}")
-    os.replace(tmp, target)
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile all kernels for gfx950 and link the shared library; return its path."""
+    """Compile all kernels for gfx950 and link the shared library; return its path.
+
+    The library and the host module over it are put in place together, once
+    both are built: a build that fails leaves the earlier pair.  They are
+    written by the compilers themselves, so that their modes follow the umask
+    and another user's processes can load them."""
     hipcc = _hipcc()
     sources = sorted(CSRC_DIR.glob("*.hip"))
     if not sources:
@@ -109,15 +110,15 @@ def build(verbose: bool = False) -> Path:
     jobs = max(1, min(len(sources), int(os.environ.get("MAX_JOBS", "8"))))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         list(pool.map(lambda pair: _compile(hipcc, *pair), zip(sources, objects)))
-    fd, tmp = tempfile.mkstemp(prefix=".libmy_vllm_amd.", suffix=".so.tmp", dir=LIB_DIR)
-    os.close(fd)
-    cmd = [hipcc, f"--offload-arch={OFFLOAD_ARCH}", "-shared", "-fPIC", "-o", tmp, *map(str, objects)]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        os.unlink(tmp)
-        raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
-    os.replace(tmp, LIB_PATH)
-    _build_host_module()
+    with tempfile.TemporaryDirectory(prefix=".build.", dir=LIB_DIR) as tmp:
+        library, host = Path(tmp) / LIB_PATH.name, Path(tmp) / HOST_PATH.name
+        cmd = [hipcc, f"--offload-arch={OFFLOAD_ARCH}", "-shared", "-fPIC", "-o", str(library), *map(str, objects)]
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
+        _build_host_module(host)
+        os.replace(library, LIB_PATH)
+        os.replace(host, HOST_PATH)
     if verbose:
         print(f"built {LIB_PATH} from {len(sources)} sources", file=sys.stderr)
     return LIB_PATH

@@ -14,10 +14,10 @@ def pytest_configure(config):
 
 
 def pytest_sessionstart(session):
-    """Build the C-ABI library when a checkout has none yet (it is not committed)."""
+    """Build the native code when a checkout has none yet (it is not committed)."""
     from my_vllm_amd import _native
 
-    if not _native.LIB_PATH.exists():
+    if not (_native.LIB_PATH.exists() and _native.HOST_PATH.exists()):
         from my_vllm_amd import build
 
         build.build()

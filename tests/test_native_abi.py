@@ -6,6 +6,7 @@ validation that fails before any launch); nothing touches a GPU.
 
 import ctypes
 import re
+import types
 from pathlib import Path
 
 import pytest
@@ -145,3 +146,38 @@ def test_missing_or_stale_host_module_makes_the_native_code_unavailable(monkeypa
         with pytest.raises(RuntimeError, match="my_vllm_amd.build"):
             _native.host_ops()
         assert _native.native_available() is False
+
+
+def test_a_failed_build_leaves_the_earlier_pair(monkeypatch, tmp_path):
+    from my_vllm_amd import build
+
+    failing = []
+
+    def run(cmd, **_):
+        target = Path(cmd[cmd.index("-o") + 1])
+        target.write_text("new")
+        return types.SimpleNamespace(returncode=int(target.name in failing), stdout="", stderr="")
+
+    monkeypatch.setattr(build, "subprocess", types.SimpleNamespace(run=run))
+    monkeypatch.setattr(build, "_hipcc", lambda: "hipcc")
+    monkeypatch.setattr(build, "LIB_DIR", tmp_path)
+    monkeypatch.setattr(build, "BUILD_DIR", tmp_path / "objects")
+    pair = tmp_path / "libmy_vllm_amd.so", tmp_path / "mva_host.so"
+    monkeypatch.setattr(build, "LIB_PATH", pair[0])
+    monkeypatch.setattr(build, "HOST_PATH", pair[1])
+    for path in pair:
+        path.write_text("old")
+    for failing in (["mva_host.so"], ["libmy_vllm_amd.so"]):
+        with pytest.raises(RuntimeError, match="failed"):
+            build.build()
+        assert [path.read_text() for path in pair] == ["old", "old"]
+    failing = []
+    build.build()
+    assert [path.read_text() for path in pair] == ["new", "new"]
+    assert sorted(path.name for path in tmp_path.iterdir()) == ["libmy_vllm_amd.so", "mva_host.so", "objects"]
+
+
+def test_built_files_are_readable_alike():
+    # A module that only its builder can read fails in another user's process.
+    library, host = (path.stat().st_mode & 0o444 for path in (_native.LIB_PATH, _native.HOST_PATH))
+    assert library == host
