@@ -331,8 +331,12 @@ int mva_paged_decode_noalloc(const void* q, int64_t q_token_stride, int64_t q_he
  * mva_paged_prefill's tiles hold twice as many (256 query rows). */
 int mva_prefill_tile_tokens(int num_q_heads, int num_kv_heads);
 
-/* Bytes of the prefill workspace (the device-built tile list) for at most
- * max_tiles query tiles, or -1 for an invalid count. */
+/* Bytes of the prefill workspace for at most max_tiles query tiles, or -1 for
+ * an invalid count: the device-built tile list (16 KB and 64 bytes a tile),
+ * then the piece list, arrival counters and fp32 partials of tiles cut by
+ * keys (34.7 MB).  It never shrinks as max_tiles grows, so a workspace sized
+ * for the largest batch serves every smaller one.  A workspace that holds the
+ * tile list alone is taken too; no tile is cut then. */
 int64_t mva_prefill_workspace_bytes(int64_t max_tiles);
 
 /* Byte offset, inside a prefill workspace, of the int32 word where
@@ -350,7 +354,11 @@ int64_t mva_prefill_workspace_bytes(int64_t max_tiles);
  * (nothing is read back to the host): one query tile per
  * 2 * mva_prefill_tile_tokens() tokens x all query heads of a KV head (256
  * query rows), longest context first, written into `workspace`
- * (mva_prefill_workspace_bytes(max_tiles) bytes, 16-byte aligned).
+ * (mva_prefill_workspace_bytes(max_tiles) bytes, 16-byte aligned).  Where
+ * whole tiles would leave workgroups idle, tiles are cut by keys into pieces;
+ * each piece leaves an fp32 partial and the last piece of a tile to end merges
+ * them in key order, so a sequence's rows depend on the batch around it in
+ * their rounding, and on nothing else.
  * max_tiles must bound the tile count, e.g. num_prefill_tokens / tile_tokens
  * + num_seqs with tile_tokens = 2 * mva_prefill_tile_tokens(); tiles beyond
  * it are not run (their output rows keep what `out` held), and the launch

@@ -730,9 +730,10 @@ extern "C" int mva_prefill_tile_tokens(int num_q_heads, int num_kv_heads) {
 
 extern "C" int64_t mva_prefill_workspace_bytes(int64_t max_tiles) {
   if (max_tiles < 0 || max_tiles > 0x7fffffffLL / mva::kPrefillPlanItemInts) return -1;
-  // Up to this many tiles a plan may be cut into split-K pieces.
-  if (max_tiles <= mva::kPrefillCutTiles) return mva::prefill_split_bytes(max_tiles);
-  return mva::prefill_plan_bytes(max_tiles);
+  // The split-K area at every size, though only plans of at most
+  // kPrefillCutTiles tiles use it: a workspace sized for a program's largest
+  // batch, or by its memory probe, then serves every smaller one in full.
+  return mva::prefill_split_bytes(max_tiles);
 }
 
 namespace {

@@ -59,6 +59,17 @@ def test_host_queries():
     assert _native.query("mva_decode_workspace_bytes", -1, 8, 2) == -1
 
 
+def test_prefill_workspaces_grow_with_their_tiles():
+    # A workspace sized for the largest batch (or by a memory probe) serves
+    # every smaller one: the bytes never fall as the tiles grow, and hold at
+    # least the tile list.
+    counts = [0, 1, 2, 31, 32, 255, 256, 257, 300, 1000, 4096, 100000]
+    sizes = [_native.query("mva_prefill_workspace_bytes", n) for n in counts]
+    assert sizes == sorted(sizes)
+    assert all(size >= 4 * (32 * 128 + 16 * n) for size, n in zip(sizes, counts))
+    assert _native.query("mva_prefill_workspace_bytes", -1) == -1
+
+
 def test_invalid_arguments_fail_before_launch_with_a_message():
     lib = _native.load_library()
     with pytest.raises(RuntimeError, match="mva_silu_and_mul failed"):
