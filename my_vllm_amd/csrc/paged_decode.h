@@ -807,41 +807,31 @@ __device__ inline f32x4 part_load4(const float* a) {
   }
 }
 
-// Chunks one wavefront of a merge holds in flight at a time.
+// Chunks one wavefront of a merge holds in flight at a time, and wavefronts
+// of a wide merge.
 constexpr int kMergeRows = 32;
+constexpr int kWideMergeWaves = 8;
+// Floats of one merge of more than kMergeRows chunks in LDS: per wavefront of
+// the wide form a row of sums, the max and the weight sum.
+constexpr int kMergeLdsFloats = kWideMergeWaves * (kHeadDim + 2);
 
-// Split-K merge of one (split segment, query head g): d is a piece
-// descriptor {seq, -, -, -, n_chunks, part_base, q_row, kv_head} of a
-// segment cut into n_chunks > 1 pieces; writes
-//   o = sum_k w_k o_k / sum_k w_k,  w_k = 2^(lse_k - max_k lse_k)
-// over the segment's chunks k.  Runs in the kernel after the decode kernel
-// (kAgent false: the kernel boundary makes every partial visible) or inside
-// the launch after the segment's last arrival (kAgent true).
-//
-// A merge is a chain of memory latencies, not bandwidth: 512 bytes a chunk.
-// So a wavefront requests 32 chunks at once (16-byte loads, two rows per
-// instruction: lane half 0 the even rows, half 1 the odd) together with
-// their log-sum-exps, and kWaves wavefronts of a workgroup take 32 chunks
-// each of every 32 * kWaves, meeting in LDS (`red`, kWaves > 1 only).
-// Measured, decode call of one sequence at 32 / 8 heads (256 chunks a head):
-// 30001 tokens 49.8 -> 32.3 us, 8192 tokens 32.4 -> 15.0 us against one
-// wavefront walking the chunks 16 at a time, 8 bytes a lane; 64 sequences of
-// 512-1024 tokens (5 chunks) 49.2 -> 48.8 us.
-template <typename T, bool kAgent, int kWaves>
-__device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int wave, float* red) {
+// Sums over some chunks of a merge: the weighted rows (columns 4 * (lane % 32)
+// .. + 3), the weights, and the log-sum-exp they are relative to.
+struct MergeSums {
+  f32x4 acc;
+  float m, wsum;
+};
+
+// The sums of chunks base .. base + 31, base + step .. base + step + 31, ...
+// below n; slot(k) is chunk k's partial slot (lse index; o row = slot * D).
+template <bool kAgent, typename Slot>
+__device__ __attribute__((always_inline)) inline MergeSums merge_chunks(const DecodeParams& p, Slot slot, int n,
+                                                                        int base, int step) {
   const int lane = threadIdx.x & 63;
   const int half = lane >> 5, col = 4 * (lane & 31);
-  const int G = p.group;
-  const int Hkv = p.num_kv_heads;
-  const int n = d[4];
-  const int pbase = d[5];
-  const int64_t qrow = d[6];
-  const int h = d[7];
-  // Partial slot of chunk k (lse index; o row = slot * D).
-  auto slot = [&](int k) -> int64_t { return ((int64_t)(pbase + k) * Hkv + h) * G + g; };
   float m = -INFINITY, wsum = 0.f;
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int base = kMergeRows * wave; base < n; base += kMergeRows * kWaves) {
+  for (; base < n; base += step) {
     const int cnt = min(kMergeRows, n - base);
     f32x4 rows[kMergeRows / 2];
     // Row indices past the count are clamped (weight 0; the clamped rows are
@@ -879,39 +869,95 @@ __device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int 
   for (int off = 16; off > 0; off >>= 1) wsum += __shfl_xor(wsum, off);
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], 32);
-  if constexpr (kWaves > 1) {
-    if (n > kMergeRows) {  // the same for every wavefront of the workgroup
-      float* const max_of = red + kWaves * kHeadDim;
-      float* const sum_of = max_of + kWaves;
-      if (half == 0) *reinterpret_cast<f32x4*>(red + wave * kHeadDim + col) = acc;
-      if (lane == 0) {
-        max_of[wave] = m;
-        sum_of[wave] = wsum;
-      }
-      __syncthreads();
-      if (wave != 0) return;
-      float mx = max_of[0];
-#pragma unroll
-      for (int v = 1; v < kWaves; ++v) mx = fmaxf(mx, max_of[v]);
-      const float m_use = mx == -INFINITY ? 0.f : mx;
-      acc = f32x4{0.f, 0.f, 0.f, 0.f};
-      wsum = 0.f;
-#pragma unroll
-      for (int v = 0; v < kWaves; ++v) {
-        const float f = fast_exp2(max_of[v] - m_use);
-        acc += f * *reinterpret_cast<const f32x4*>(red + v * kHeadDim + col);
-        wsum += f * sum_of[v];
-      }
-    } else if (wave != 0) {
-      return;
-    }
+  return {acc, m, wsum};
+}
+
+// Part v of kWideMergeWaves of a merge into its LDS (`red`, kMergeLdsFloats),
+// and the parts' total.
+__device__ __attribute__((always_inline)) inline void put_merge_part(float* red, int v, const MergeSums& s) {
+  const int lane = threadIdx.x & 63;
+  if (lane < 32) *reinterpret_cast<f32x4*>(red + v * kHeadDim + 4 * lane) = s.acc;
+  if (lane == 0) {
+    red[kWideMergeWaves * kHeadDim + v] = s.m;
+    red[kWideMergeWaves * (kHeadDim + 1) + v] = s.wsum;
   }
-  const float winv = wsum > 0.f ? 1.0f / wsum : 0.f;
-  if (half == 0) {
+}
+__device__ __attribute__((always_inline)) inline MergeSums total_merge_parts(const float* red) {
+  const int col = 4 * (threadIdx.x & 31);
+  const float* const max_of = red + kWideMergeWaves * kHeadDim;
+  const float* const sum_of = max_of + kWideMergeWaves;
+  float mx = max_of[0];
+#pragma unroll
+  for (int v = 1; v < kWideMergeWaves; ++v) mx = fmaxf(mx, max_of[v]);
+  const float m_use = mx == -INFINITY ? 0.f : mx;
+  MergeSums s = {f32x4{0.f, 0.f, 0.f, 0.f}, mx, 0.f};
+#pragma unroll
+  for (int v = 0; v < kWideMergeWaves; ++v) {
+    const float f = fast_exp2(max_of[v] - m_use);
+    s.acc += f * *reinterpret_cast<const f32x4*>(red + v * kHeadDim + col);
+    s.wsum += f * sum_of[v];
+  }
+  return s;
+}
+
+// Split-K merge of one (split segment, query head g): d is a piece
+// descriptor {seq, -, -, -, n_chunks, part_base, q_row, kv_head} of a
+// segment cut into n_chunks > 1 pieces; writes
+//   o = sum_k w_k o_k / sum_k w_k,  w_k = 2^(lse_k - max_k lse_k)
+// over the segment's chunks k.  Runs in the kernel after the decode kernel
+// (kAgent false: the kernel boundary makes every partial visible) or inside
+// the launch after the segment's last arrival (kAgent true).
+//
+// A merge is a chain of memory latencies, not bandwidth: 512 bytes a chunk.
+// So a wavefront requests 32 chunks at once (16-byte loads, two rows per
+// instruction: lane half 0 the even rows, half 1 the odd) together with
+// their log-sum-exps, and kWaves wavefronts of a workgroup take 32 chunks
+// each of every 32 * kWaves, meeting in LDS (`red`).
+// Measured, decode call of one sequence at 32 / 8 heads (256 chunks a head):
+// 30001 tokens 49.8 -> 32.3 us, 8192 tokens 32.4 -> 15.0 us against one
+// wavefront walking the chunks 16 at a time, 8 bytes a lane; 64 sequences of
+// 512-1024 tokens (5 chunks) 49.2 -> 48.8 us.
+//
+// The merge kernel's one wavefront sums the same parts in the same order as
+// its eight do, so the result does not depend on which of the two a launch
+// takes: a captured launch decides by its capacities, an eager one by its
+// plan, and their bits are the same.  (Merges inside a launch walk the chunks
+// in one pass.)
+template <typename T, bool kAgent, int kWaves>
+__device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int wave, float* red) {
+  static_assert(kWaves == 1 || kWaves == kWideMergeWaves, "one wavefront, or one per part");
+  const int G = p.group;
+  const int Hkv = p.num_kv_heads;
+  const int n = d[4];
+  const int64_t pbase = d[5];
+  const int64_t qrow = d[6];
+  const int h = d[7];
+  auto slot = [&](int k) -> int64_t { return ((int64_t)(pbase + k) * Hkv + h) * G + g; };
+  MergeSums s;
+  if (kAgent || n <= kMergeRows) {  // the same for every wavefront of the workgroup
+    if (wave != 0) return;
+    s = merge_chunks<kAgent>(p, slot, n, 0, kMergeRows);
+  } else if constexpr (kWaves > 1) {
+    put_merge_part(red, wave, merge_chunks<kAgent>(p, slot, n, kMergeRows * wave, kMergeRows * kWideMergeWaves));
+    __syncthreads();
+    if (wave != 0) return;
+    s = total_merge_parts(red);
+  } else {
+#pragma unroll 1
+    for (int v = 0; v < kWideMergeWaves; ++v)
+      put_merge_part(red, v, merge_chunks<kAgent>(p, slot, n, kMergeRows * v, kMergeRows * kWideMergeWaves));
+    // The wavefront's own LDS writes, in order.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    s = total_merge_parts(red);
+  }
+  const int lane = threadIdx.x & 63;
+  const float winv = s.wsum > 0.f ? 1.0f / s.wsum : 0.f;
+  if (lane < 32) {
     typename Elem<T>::v4 y;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = (T)(acc[e] * winv);
-    T* op = (T*)p.out + qrow * p.out_tok_stride + (int64_t)(h * G + g) * p.out_head_stride + col;
+    for (int e = 0; e < 4; ++e) y[e] = (T)(s.acc[e] * winv);
+    T* op = (T*)p.out + qrow * p.out_tok_stride + (int64_t)(h * G + g) * p.out_head_stride + 4 * lane;
     *reinterpret_cast<typename Elem<T>::v4*>(op) = y;
   }
 }

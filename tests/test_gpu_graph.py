@@ -102,3 +102,32 @@ def test_decode_graph_state_rejects_plans_that_do_not_fit(gpu):
     assert backend.full_decode_graph_metadata_fits(state, backend.build_plan(_on(ok.common, gpu)))
     with pytest.raises(RuntimeError, match="planned before activation"):
         backend.activate_full_decode_graph(backend.create_full_decode_graph_state(4, 32, gpu))
+
+
+# Merges of more than 32 chunks where the captured launch, which decides by its
+# capacities, and the eager one, which decides by its plan, give a merge
+# another number of wavefronts: one long context among short ones (eager
+# eight, captured one), and 125 chunks among merges of eight (the other way).
+# fp16 and 16 query heads a KV head: many results, finely rounded.
+@pytest.mark.parametrize("hq,hkv,ctx", [(128, 8, [8192] * 2 + [16] * 38), (128, 8, [2000] + [128] * 16)])
+def test_merge_width_does_not_change_the_result(gpu, hq, hkv, ctx):
+    backend = MI355XAttentionBackend(hq, hkv, 128, 16, torch.float16)
+    b = make_paged_batch(41, [1] * len(ctx), ctx, 0, hq, hkv, dtype=torch.float16)
+    common = _on(b.common, gpu)
+    q, kc, vc = b.q.to(gpu), b.k_cache.to(gpu), b.v_cache.to(gpu)
+    empty = q.new_empty((0, hkv, 128))
+    plan = backend.build_plan(common)
+    m = plan.metadata
+    state = backend.create_full_decode_graph_state(len(ctx), len(ctx) * common.block_tables.size(1), gpu)
+    eager_wide = m.num_decode_part_slots * hkv > 16 * m.num_decode_merges
+    assert eager_wide != (state.part_slot_capacity * hkv > 16 * state.merge_capacity)
+    assert int(m.decode_merges[:, 4].max()) > 32
+    eager = backend.forward(q, empty, empty, kc, vc, plan).clone()
+    backend.plan_full_decode_graph(state, plan)
+    backend.activate_full_decode_graph(state)
+    try:
+        captured = backend.forward(q, empty, empty, kc, vc, plan).clone()
+    finally:
+        backend.deactivate_full_decode_graph()
+    assert torch.equal(captured, eager)
+    assert_attention_close(eager, paged_attention(b.q, b.k_cache, b.v_cache, b.common.block_tables, [1] * len(ctx), ctx))
