@@ -1107,7 +1107,10 @@ class MI355XAttentionBackendMixin:
             raise ValueError("attention plan does not fit full decode graph state")
         metadata = plan.metadata
         host = metadata.decode_host_plan
-        if host is None or host[3] != state.groups:
+        # The step's own plan, whose page ranges are at most those that the
+        # state's capacities are for (decode_ranges takes fewer at one or two
+        # KV heads): replays run what an eager launch runs.
+        if host is None or host[3] > state.groups:
             counts = np.diff(np.asarray(metadata.kv_indptr, dtype=np.int64))
             items, wave_extra, _, _, merges = plan_decode_listed(counts, 0, 0, self.num_kv_heads, state.groups)
         else:

@@ -131,3 +131,40 @@ def test_merge_width_does_not_change_the_result(gpu, hq, hkv, ctx):
         backend.deactivate_full_decode_graph()
     assert torch.equal(captured, eager)
     assert_attention_close(eager, paged_attention(b.q, b.k_cache, b.v_cache, b.common.block_tables, [1] * len(ctx), ctx))
+
+
+# At one and two KV heads a step of two pages a range or more, or of a few
+# long sequences, is cut into fewer ranges than a launch can hold: the graph
+# takes that plan as it is (no second one on the host), and its replay is the
+# eager launch bit for bit.  The last case stays under the bound.
+@pytest.mark.parametrize("hq,hkv,ctx", [(8, 1, [30000, 20000, 20000]), (16, 2, [9000] * 6 + [17]), (16, 2, [9000]),
+                                        (8, 1, [8300]), (16, 2, [700, 40])])
+def test_graph_takes_the_steps_own_plan(gpu, monkeypatch, hq, hkv, ctx):
+    import my_vllm_amd.attention_backend as ab
+
+    backend = MI355XAttentionBackend(hq, hkv, 128, 16, torch.float16)
+    b = make_paged_batch(43, [1] * len(ctx), ctx, 0, hq, hkv, dtype=torch.float16)
+    common = _on(b.common, gpu)
+    q, kc, vc = b.q.to(gpu), b.k_cache.to(gpu), b.v_cache.to(gpu)
+    empty = q.new_empty((0, hkv, 128))
+    plan = backend.build_plan(common)
+    state = backend.create_full_decode_graph_state(len(ctx), len(ctx) * common.block_tables.size(1), gpu)
+    eager = backend.forward(q, empty, empty, kc, vc, plan).clone()
+    with monkeypatch.context() as m:
+        m.setattr(ab, "plan_decode_listed", lambda *a: pytest.fail("planned twice"))
+        backend.plan_full_decode_graph(state, plan)
+    backend.activate_full_decode_graph(state)
+    try:
+        backend.forward(q, empty, empty, kc, vc, plan)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            backend.forward(q, empty, empty, kc, vc, plan)
+    finally:
+        backend.deactivate_full_decode_graph()
+    for _ in range(3):
+        state.output.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(state.output, eager)
+    assert_attention_close(eager, paged_attention(b.q, b.k_cache, b.v_cache, b.common.block_tables, [1] * len(ctx), ctx))
