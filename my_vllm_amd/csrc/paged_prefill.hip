@@ -947,9 +947,11 @@ constexpr double kLittleDecode = 0.25, kShortTile = 8.0;
 constexpr int64_t kSortTiles = 4096;  // batches of more tiles are taken as even
 
 struct PrefillEstimate {
-  int64_t tiles = 0;          // query tiles of one KV head
-  double work = 0;            // 64-key tiles of all of them
-  std::vector<int> keys;      // 64-key tiles of each, longest first (empty beyond kSortTiles)
+  int64_t tiles = 0;      // query tiles of one KV head
+  double work = 0;        // 64-key tiles of all of them
+  std::vector<int> keys;  // 64-key tiles of each, longest first (empty beyond kSortTiles)
+  // Pieces of all tiles when the longest is cut into k, once asked for.
+  int64_t pieces[kPrefillMaxPieces + 1] = {};
 };
 
 // The batch's query tiles from its page and token counts: queries are spread
@@ -980,8 +982,14 @@ PrefillEstimate estimate_prefill(const int64_t* pages, int64_t n, int64_t tokens
   return e;
 }
 
+// No prefill time on per_head workgroups per KV head is below this: the
+// tiles' work in equal parts.
+double least_prefill_us(const PrefillEstimate& e, int64_t per_head) {
+  return kPrefillStartUs + kTileUs * (e.work / (double)per_head);
+}
+
 // Time of the prefill part on per_head workgroups per KV head.
-double prefill_part_us(const PrefillEstimate& e, int64_t per_head, int64_t max_tiles, int num_kv_heads) {
+double prefill_part_us(PrefillEstimate& e, int64_t per_head, int64_t max_tiles, int num_kv_heads) {
   if (max_tiles > per_head) {
     // j + 1 of the j * per_head + 1 longest tiles share a workgroup.
     double len = e.work / (double)per_head + kItemTiles * ((double)e.tiles / (double)per_head);
@@ -1001,10 +1009,11 @@ double prefill_part_us(const PrefillEstimate& e, int64_t per_head, int64_t max_t
   double best = longest;
   for (int k = 2; k <= kPrefillMaxPieces; ++k) {
     const int len = longest > k ? (longest + k - 1) / k : 1;
-    int64_t count = 0;
-    for (int keys : e.keys) count += (keys + len - 1) / len;
     const double t = len + 2.5 + 0.75 * k;
-    if (count <= limit && t < best) best = t;
+    if (t >= best) continue;
+    if (e.pieces[k] == 0)
+      for (int keys : e.keys) e.pieces[k] += (keys + len - 1) / len;
+    if (e.pieces[k] <= limit) best = t;
   }
   return kPrefillStartUs + kTileUs * (best + kItemTiles);
 }
@@ -1020,17 +1029,36 @@ extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, in
   if (num_prefill_seqs == 0 || num_prefill_tokens == 0) return 0;
   const int tile_tokens = kPrefillPPRows / (num_q_heads / num_kv_heads);
   const int64_t max_tiles = num_prefill_tokens / tile_tokens + num_prefill_seqs;
-  const PrefillEstimate e = estimate_prefill(prefill_pages, num_prefill_seqs, num_prefill_tokens, tile_tokens);
+  PrefillEstimate e = estimate_prefill(prefill_pages, num_prefill_seqs, num_prefill_tokens, tile_tokens);
   const double mb = (double)decode_pages * kPageSize * num_kv_heads * kHeadDim * 2 * 2 * 1e-6;
-  int64_t best = 1;
-  double best_us = 0;
-  for (int64_t p = 1; p == 1 || p * num_kv_heads < num_cus; ++p) {
+  auto decode_us = [&](int64_t p) {
     const int64_t left = num_cus - p * num_kv_heads;
-    double d = kDecodeUsPerMB + kDecodeUsPerMBCu / (double)(left > 0 ? left : 1);
-    d = kDecodeStartUs + mb * (d > kDecodeMinUsPerMB ? d : kDecodeMinUsPerMB);
-    const double f = prefill_part_us(e, p, max_tiles, num_kv_heads);
-    const double us = (d > f ? d : f) + (max_tiles > p ? kStreamUs : 0.0);
-    if (p == 1 || us < best_us) best = p, best_us = us;
+    const double d = kDecodeUsPerMB + kDecodeUsPerMBCu / (double)(left > 0 ? left : 1);
+    return kDecodeStartUs + mb * (d > kDecodeMinUsPerMB ? d : kDecodeMinUsPerMB);
+  };
+  auto step_us = [&](int64_t p, double prefill_us) {
+    const double d = decode_us(p);
+    return (d > prefill_us ? d : prefill_us) + (max_tiles > p ? kStreamUs : 0.0);
+  };
+  // The fastest share, the smallest of equals.  Prices are lower the closer
+  // the two parts are, so the share where decode takes the least that prefill
+  // can is priced first, and most others fall to their lower bound: at one KV
+  // head, 255 shares, pricing each cost 15 to 250 us a step, now 4 to 6 (25 at
+  // 2500 tiles, most of it sorting them).
+  const int64_t shares = num_kv_heads < num_cus ? (num_cus - 1) / num_kv_heads : 1;
+  int64_t lo = 1, hi = shares;
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) / 2;
+    if (decode_us(mid) >= least_prefill_us(e, mid)) hi = mid;
+    else lo = mid + 1;
+  }
+  int64_t best = lo;
+  double best_us = step_us(lo, prefill_part_us(e, lo, max_tiles, num_kv_heads));
+  for (int64_t p = 1; p <= shares; ++p) {
+    if (decode_us(p) > best_us) break;  // and so for every larger share
+    if (p == lo || step_us(p, least_prefill_us(e, p)) > best_us) continue;
+    const double us = step_us(p, prefill_part_us(e, p, max_tiles, num_kv_heads));
+    if (us < best_us || (us == best_us && p < best)) best = p, best_us = us;
   }
   // Little decode beside many short tiles: the 128-row tiles of
   // mva_paged_mixed, two to a CU, start sooner.  64 / 8 heads, 13 decodes of

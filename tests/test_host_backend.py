@@ -7,6 +7,7 @@ through the ``require_device_metadata`` seam; nothing here calls a kernel.
 """
 
 import json
+import time
 from pathlib import Path
 
 import numpy as np
@@ -508,6 +509,19 @@ def test_mixed_prefill_workgroups_leave_cus_for_decode(hq, hkv, pages, tokens, d
     assert ops.mixed_prefill_workgroups((), 0, decode, hq, hkv, 256) == 0
     with pytest.raises(ValueError):
         ops.mixed_prefill_workgroups(pages, tokens, decode, hq, hkv + hq, 256)
+
+
+@pytest.mark.parametrize("hq,hkv,pages,tokens,decode", [(8, 1, (128, 503, 503, 503), 2150, 15000),
+                                                        (1, 1, (600,), 9000, 3000)])
+def test_mixed_share_is_priced_in_a_few_microseconds(hq, hkv, pages, tokens, decode):
+    # 255 shares at one KV head: pricing each took 120 to 190 us a step here,
+    # beside about 70 for the rest of a step's plan; now 6.
+    best = 1.0
+    for _ in range(100):
+        start = time.perf_counter()
+        ops.mixed_prefill_workgroups(pages, tokens, decode, hq, hkv, 256)
+        best = min(best, time.perf_counter() - start)
+    assert best < 60e-6
 
 
 @pytest.mark.parametrize("hkv", [1, 2, 3, 4, 8, 16])
