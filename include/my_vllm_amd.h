@@ -437,11 +437,22 @@ int mva_paged_mixed(const void* q, int64_t q_token_stride, int64_t q_head_stride
 
 /*
  * Workgroups (CUs) that mva_paged_mixed_run should give the prefill part of a
- * MIXED step: the multiple of num_kv_heads, below num_cus, whose estimated
- * prefill time and decode time on the CUs left are closest.  prefill_pages
- * holds the pages of each prefill sequence, decode_pages those of all decode
- * sequences.  0 without prefill tokens and where mva_paged_mixed is faster
- * (many prefill tiles, little decode), -1 for invalid arguments.  Host only.
+ * MIXED step, a multiple of num_kv_heads below num_cus, or 0 without prefill
+ * tokens and where mva_paged_mixed is estimated faster (small steps, and those
+ * whose query lengths may be so uneven that a share of CUs fits only some of
+ * what they can be); -1 for invalid arguments.  prefill_pages holds the pages
+ * of each prefill sequence, max_query_len bounds their queries (0: unknown),
+ * decode_pages and max_decode_pages are the decode sequences' total and
+ * largest.  Host only.
+ */
+int64_t mva_mixed_prefill_share(const int64_t* prefill_pages, int64_t num_prefill_seqs,
+                                int64_t num_prefill_tokens, int64_t max_query_len, int64_t decode_pages,
+                                int64_t max_decode_pages, int num_q_heads, int num_kv_heads, int64_t num_cus);
+
+/*
+ * The share alone, for queries spread evenly over the prefill sequences: the
+ * one with the lowest estimated time, and 0 without prefill tokens and for
+ * many short prefill tiles beside little decode.  Host only.
  */
 int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, int64_t num_prefill_seqs,
                                      int64_t num_prefill_tokens, int64_t decode_pages, int num_q_heads,

@@ -183,6 +183,7 @@ _SIGNATURES = {
             _i32, _i32, _i32, _i32, _f32, _i32, _c_void_p,
         ],
     ),
+    "mva_mixed_prefill_share": (_i64, [_c_void_p, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _i64]),
     "mva_mixed_prefill_workgroups": (_i64, [_c_void_p, _i64, _i64, _i64, _i32, _i32, _i64]),
     "mva_paged_mixed_run": (
         _i32,
@@ -203,7 +204,7 @@ _SIGNATURES = {
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 # The C ABI revision these signatures describe (mva_abi_version()).
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

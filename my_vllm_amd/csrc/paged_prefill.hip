@@ -5,6 +5,7 @@
 #include "paged_prefill_pingpong.h"
 
 #include <algorithm>
+#include <cmath>
 #include <functional>
 #include <vector>
 
@@ -929,36 +930,83 @@ extern "C" int mva_paged_mixed(const void* q, int64_t q_token_stride, int64_t q_
   return check_launch("paged_mixed");
 }
 
-// Host estimate of the CUs a MIXED launch gives its prefill part (see
-// mva_mixed_prefill_workgroups), in microseconds fitted to sweeps of the
-// split on one MI355X: a prefill workgroup takes 1.7 per 64 keys of a 256-row
-// tile and as much as 2.5 of them per tile or piece; a CU of decode
-// wavefronts streams 1 MB in 26.3 beside 0.045 per MB of the launch, and all
-// of them together no faster than 0.172 per MB (5.8 TB/s).
+// Host estimates for MIXED steps (see mva_mixed_prefill_share): the time of
+// mva_paged_mixed_run at a share of the CUs for its prefill part, and that of
+// mva_paged_mixed, in microseconds fitted to sweeps of the share over 730 drawn
+// steps on one MI355X (7000 timings; one prefill sequence or more, even and
+// skewed, 1 to 900 MB of decode K/V and more).  Of each timing over the
+// estimate, the 5th and 95th percentiles: decode part 0.90 and 1.09, fixed
+// prefill form 0.92 and 1.10, turns 0.88 and 1.20, mva_paged_mixed 0.84 and
+// 1.14 up to 30 us, 0.88 and 1.09 from 150 us on.  Tiles and pieces are counted
+// as plan_pieces counts them, but its prices are its own: the two need not
+// agree, and a share that is off costs time and nothing else.
 namespace {
 
-constexpr double kTileUs = 1.7;
-constexpr double kItemTiles = 2.5;
-constexpr double kCutTiles = 16.0;
-constexpr double kPrefillStartUs = 4.0;
-constexpr double kStreamUs = 5.0;  // claims, and decode workgroups joining in at the end
-constexpr double kDecodeStartUs = 6.0, kDecodeUsPerMB = 0.045, kDecodeUsPerMBCu = 26.3, kDecodeMinUsPerMB = 0.172;
-constexpr double kLittleDecode = 0.25, kShortTile = 8.0;
-constexpr int64_t kSortTiles = 4096;  // batches of more tiles are taken as even
+// Decode part: a CU of eight wavefronts streams 1 MB in 24.1 beside 0.0367 per
+// MB of the launch, and all of them together no faster than 0.1752 (5.7 TB/s).
+constexpr double kDecodeStartUs = 9.7, kDecodeUsPerMB = 0.0367, kDecodeUsPerMBCu = 24.1, kDecodeMinUsPerMB = 0.1752;
+// Prefill part, one item a workgroup: whole tiles, or tiles cut into k.
+constexpr double kWholeStartUs = 12.5, kWholeKeyUs = 1.37;
+constexpr double kCutStartUs = 17.0, kCutPieceUs = 0.95, kCutKeyUs = 1.41;
+// More tiles than workgroups: key tiles and items a workgroup, the tiles that
+// must share one, and what a cut plan in turns has on top.
+constexpr double kRoundsStartUs = 10.0, kRoundsKeyUs = 1.57, kRoundsItemUs = 4.7, kTogetherUs = 1.43;
+constexpr double kItemKeys = 2.5, kTurnsCutUs = 17.3;
+// mva_paged_mixed: the longest tile, the longest decode piece and its merge
+// (one pass of 32 chunks a query head after another), and the work of a CU,
+// in a root of squares.
+constexpr double kOneStartUs = 7.6, kOneKeyUs = 1.28, kOnePageUs = 0.9, kOneMergeUs = 0.58, kOnePassUs = 0.866,
+                 kOneChunkUs = 0.042, kOneWorkUs = 0.747, kOneTileUs = 5.6, kOneMBUs = 0.212;
+constexpr double kMixedWavesPerCu = 6.0, kPiecesPerWave = 1.5;  // of its decode plan (plan_decode_claims)
+constexpr int64_t kListTiles = 1024;  // batches of more tiles are taken as even
 
 struct PrefillEstimate {
-  int64_t tiles = 0;      // query tiles of one KV head
-  double work = 0;        // 64-key tiles of all of them
-  std::vector<int> keys;  // 64-key tiles of each, longest first (empty beyond kSortTiles)
+  int64_t tiles = 0, half_tiles = 0;  // query tiles of one KV head: 256 rows, 128 rows
+  double work = 0, half_work = 0;     // 64-key tiles of all of them
+  int longest = 0;
+  int spare = 0;          // pieces that a cut keeps free (the lengths are not known)
+  std::vector<int> keys;  // 64-key tiles of each 256-row tile, longest first (empty beyond kListTiles)
   // Pieces of all tiles when the longest is cut into k, once asked for.
   int64_t pieces[kPrefillMaxPieces + 1] = {};
 };
 
-// The batch's query tiles from its page and token counts: queries are spread
-// evenly over the sequences (their lengths are on the device), none having
-// more queries than keys.
-PrefillEstimate estimate_prefill(const int64_t* pages, int64_t n, int64_t tokens, int tile_tokens) {
+// 64-key tiles that query tile t of a sequence of q queries and kv keys sees.
+int key_tiles(int64_t kv, int64_t q, int64_t t, int64_t rows) {
+  const int64_t end = kv - q + ((t + 1) * rows < q ? (t + 1) * rows : q);
+  return (int)((end + kPrefillKeys - 1) / kPrefillKeys);
+}
+
+// Adds the query tiles of one sequence.
+void add_tiles(PrefillEstimate& e, int64_t kv, int64_t q, int64_t rows) {
+  auto sum = [&](int64_t height, int64_t& tiles, double& work) {
+    const int64_t n = (q + height - 1) / height;
+    tiles += n;
+    if (n > kListTiles) {
+      work += 0.5 * (double)n * ((double)key_tiles(kv, q, 0, height) + (double)key_tiles(kv, q, n - 1, height));
+      return;
+    }
+    for (int64_t t = 0; t < n; ++t) work += key_tiles(kv, q, t, height);
+  };
+  if (q <= 0) return;
+  sum(rows / 2, e.half_tiles, e.half_work);
+  sum(rows, e.tiles, e.work);
+  const int64_t n = (q + rows - 1) / rows;
+  e.longest = std::max(e.longest, key_tiles(kv, q, n - 1, rows));
+  if (e.tiles <= kListTiles)  // they are cleared where the batch has more
+    for (int64_t t = 0; t < n; ++t) e.keys.push_back(key_tiles(kv, q, t, rows));
+}
+
+PrefillEstimate estimate_prefill(const int64_t* pages, const std::vector<int64_t>& queries, int tile_tokens) {
   PrefillEstimate e;
+  for (size_t s = 0; s < queries.size(); ++s) add_tiles(e, pages[s] * kPageSize, queries[s], tile_tokens);
+  if (e.tiles > kListTiles) e.keys.clear();
+  std::sort(e.keys.begin(), e.keys.end(), std::greater<int>());
+  return e;
+}
+
+// Query lengths are on the device.  Without a bound on them they are taken as
+// evenly spread, no sequence having more queries than keys.
+std::vector<int64_t> even_queries(const int64_t* pages, int64_t n, int64_t tokens) {
   double share = (double)tokens / (double)n, held = 0;
   int64_t longer = 0;
   for (int64_t s = 0; s < n; ++s) {
@@ -967,98 +1015,106 @@ PrefillEstimate estimate_prefill(const int64_t* pages, int64_t n, int64_t tokens
     else ++longer;
   }
   if (longer > 0) share = ((double)tokens - held) / (double)longer;
-  for (int64_t s = 0; s < n; ++s) {
-    const double kv = (double)pages[s] * kPageSize, q = kv < share ? kv : share;
-    const int64_t count = (int64_t)((q + tile_tokens - 1) / tile_tokens);
-    for (int64_t t = 0; t < count; ++t) {
-      const double end = kv - q + ((t + 1) * tile_tokens < q ? (double)((t + 1) * tile_tokens) : q);
-      const int keys = (int)((end + kPrefillKeys - 1) / kPrefillKeys);
-      e.work += keys;
-      if (++e.tiles <= kSortTiles) e.keys.push_back(keys);
-    }
+  std::vector<int64_t> q(n);
+  for (int64_t s = 0; s < n; ++s) q[s] = std::min(pages[s] * kPageSize, (int64_t)(share + 0.999));
+  return q;
+}
+
+// With a bound, all the work that `tokens` queries of at most max_query a
+// sequence can be lies between two batches: the longest queries on the longest
+// contexts, or on the shortest.
+std::vector<int64_t> packed_queries(const int64_t* pages, int64_t n, int64_t tokens, int64_t max_query, bool longest) {
+  std::vector<int64_t> order(n), q(n);
+  for (int64_t s = 0; s < n; ++s) order[s] = s;
+  std::sort(order.begin(), order.end(), [&](int64_t a, int64_t b) {
+    return longest ? pages[a] > pages[b] : pages[a] < pages[b];
+  });
+  int64_t left = tokens;
+  for (int64_t s = 0; s < n; ++s) left -= q[s] = pages[s] > 0 && left > 0 ? 1 : 0;
+  for (int64_t s : order) {
+    const int64_t more = std::max<int64_t>(std::min(left, std::min(max_query, pages[s] * kPageSize) - q[s]), 0);
+    q[s] += more;
+    left -= more;
   }
-  if (e.tiles > kSortTiles) e.keys.clear();
-  std::sort(e.keys.begin(), e.keys.end(), std::greater<int>());
-  return e;
+  return q;
 }
 
 // No prefill time on per_head workgroups per KV head is below this: the
 // tiles' work in equal parts.
 double least_prefill_us(const PrefillEstimate& e, int64_t per_head) {
-  return kPrefillStartUs + kTileUs * (e.work / (double)per_head);
+  return kRoundsStartUs + kWholeKeyUs * (e.work / (double)per_head);
 }
 
 // Time of the prefill part on per_head workgroups per KV head.
 double prefill_part_us(PrefillEstimate& e, int64_t per_head, int64_t max_tiles, int num_kv_heads) {
   if (max_tiles > per_head) {
+    const double even = (kRoundsKeyUs * e.work + kRoundsItemUs * (double)e.tiles) / (double)per_head;
     // j + 1 of the j * per_head + 1 longest tiles share a workgroup.
-    double len = e.work / (double)per_head + kItemTiles * ((double)e.tiles / (double)per_head);
-    for (int64_t j = 0; j * per_head < (int64_t)e.keys.size(); ++j) {
-      const double together = (double)(j + 1) * (e.keys[j * per_head] + kItemTiles);
-      if (together > len) len = together;
-    }
+    double together = 0;
+    for (int64_t j = 0; j * per_head < (int64_t)e.keys.size(); ++j)
+      together = std::max(together, kTogetherUs * (double)(j + 1) * (e.keys[j * per_head] + kItemKeys));
     // Pieces in turns.
-    const double cut = e.work / (double)per_head + kItemTiles * ((double)e.tiles / (double)per_head) + kCutTiles;
-    if (plan_form(max_tiles, per_head) == PlanForm::kTurns && max_tiles <= kPrefillCutTiles && cut < len) len = cut;
-    return kPrefillStartUs + kTileUs * len;
+    if (plan_form(max_tiles, per_head) == PlanForm::kTurns && max_tiles <= kPrefillCutTiles)
+      together = std::min(together, even + kTurnsCutUs);
+    return kRoundsStartUs + std::max(even, together);
   }
-  // plan_pieces' choice.
-  int64_t limit = kPrefillPieceSlots / num_kv_heads;
-  limit = per_head < limit ? per_head : limit;
-  const int longest = e.keys.empty() ? 0 : e.keys[0];
-  double best = longest;
+  const int64_t limit = std::min<int64_t>(per_head, kPrefillPieceSlots / num_kv_heads);
+  double best = kWholeStartUs + kWholeKeyUs * e.longest;
   for (int k = 2; k <= kPrefillMaxPieces; ++k) {
-    const int len = longest > k ? (longest + k - 1) / k : 1;
-    const double t = len + 2.5 + 0.75 * k;
+    const int len = e.longest > k ? (e.longest + k - 1) / k : 1;
+    const double t = kCutStartUs + kCutPieceUs * k + kCutKeyUs * len;
     if (t >= best) continue;
     if (e.pieces[k] == 0)
       for (int keys : e.keys) e.pieces[k] += (keys + len - 1) / len;
-    if (e.pieces[k] <= limit) best = t;
+    if (e.pieces[k] + e.spare <= limit) best = t;
   }
-  return kPrefillStartUs + kTileUs * (best + kItemTiles);
+  return best;
 }
 
-}  // namespace
+// One MIXED step, and its time at a share of p workgroups per KV head.
+struct MixedStep {
+  double mb;  // decode K/V
+  int64_t max_tiles;
+  int num_kv_heads;
+  int64_t num_cus;
 
-extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, int64_t num_prefill_seqs,
-                                                int64_t num_prefill_tokens, int64_t decode_pages, int num_q_heads,
-                                                int num_kv_heads, int64_t num_cus) {
-  if (num_prefill_seqs < 0 || num_prefill_tokens < 0 || decode_pages < 0 || num_kv_heads <= 0 || num_q_heads <= 0 ||
-      num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > 16 || (num_prefill_seqs > 0 && prefill_pages == nullptr))
-    return -1;
-  if (num_prefill_seqs == 0 || num_prefill_tokens == 0) return 0;
-  const int tile_tokens = kPrefillPPRows / (num_q_heads / num_kv_heads);
-  const int64_t max_tiles = num_prefill_tokens / tile_tokens + num_prefill_seqs;
-  PrefillEstimate e = estimate_prefill(prefill_pages, num_prefill_seqs, num_prefill_tokens, tile_tokens);
-  const double mb = (double)decode_pages * kPageSize * num_kv_heads * kHeadDim * 2 * 2 * 1e-6;
-  auto decode_us = [&](int64_t p) {
+  double decode_us(int64_t p) const {
     const int64_t left = num_cus - p * num_kv_heads;
     const double d = kDecodeUsPerMB + kDecodeUsPerMBCu / (double)(left > 0 ? left : 1);
-    return kDecodeStartUs + mb * (d > kDecodeMinUsPerMB ? d : kDecodeMinUsPerMB);
-  };
-  auto step_us = [&](int64_t p, double prefill_us) {
-    const double d = decode_us(p);
-    return (d > prefill_us ? d : prefill_us) + (max_tiles > p ? kStreamUs : 0.0);
-  };
-  // The fastest share, the smallest of equals.  Prices are lower the closer
-  // the two parts are, so the share where decode takes the least that prefill
-  // can is priced first, and most others fall to their lower bound: at one KV
-  // head, 255 shares, pricing each cost 15 to 250 us a step, now 4 to 6 (25 at
-  // 2500 tiles, most of it sorting them).
-  const int64_t shares = num_kv_heads < num_cus ? (num_cus - 1) / num_kv_heads : 1;
-  int64_t lo = 1, hi = shares;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) / 2;
-    if (decode_us(mid) >= least_prefill_us(e, mid)) hi = mid;
-    else lo = mid + 1;
+    return kDecodeStartUs + mb * std::max(d, kDecodeMinUsPerMB);
   }
-  int64_t best = lo;
-  double best_us = step_us(lo, prefill_part_us(e, lo, max_tiles, num_kv_heads));
-  for (int64_t p = 1; p <= shares; ++p) {
-    if (decode_us(p) > best_us) break;  // and so for every larger share
-    if (p == lo || step_us(p, least_prefill_us(e, p)) > best_us) continue;
-    const double us = step_us(p, prefill_part_us(e, p, max_tiles, num_kv_heads));
-    if (us < best_us || (us == best_us && p < best)) best = p, best_us = us;
+  double us(PrefillEstimate& e, int64_t p) const {
+    return std::max(decode_us(p), prefill_part_us(e, p, max_tiles, num_kv_heads));
+  }
+  double least_us(const PrefillEstimate& e, int64_t p) const { return std::max(decode_us(p), least_prefill_us(e, p)); }
+  int64_t shares() const { return num_kv_heads < num_cus ? (num_cus - 1) / num_kv_heads : 1; }
+  // The smallest share at which decode takes the least that prefill can: both
+  // times are near their lowest there.
+  int64_t meet(const PrefillEstimate& e) const {
+    int64_t lo = 1, hi = shares();
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) / 2;
+      if (decode_us(mid) >= least_prefill_us(e, mid)) hi = mid;
+      else lo = mid + 1;
+    }
+    return lo;
+  }
+  // The lowest cost of any share, and the smallest share that has it.
+  // `start` is priced first, and most others fall to their lower bound: at one
+  // KV head, 255 shares, pricing each cost 15 to 250 us a step, now 4 to 12.
+  template <typename Cost, typename Least>
+  double lowest(int64_t start, Cost cost, Least least, int64_t* share) const {
+    double best = cost(start);
+    *share = start;
+    for (int64_t p = 1; p <= shares(); ++p) {
+      if (p == start || least(p) > best) continue;
+      const double c = cost(p);
+      if (c < best || (c == best && p < *share)) best = c, *share = p;
+    }
+    return best;
+  }
+  double fastest(PrefillEstimate& e, int64_t* share) const {
+    return lowest(meet(e), [&](int64_t p) { return us(e, p); }, [&](int64_t p) { return least_us(e, p); }, share);
   }
   // Little decode beside many short tiles: the 128-row tiles of
   // mva_paged_mixed, two to a CU, start sooner.  64 / 8 heads, 13 decodes of
@@ -1066,10 +1122,104 @@ extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, in
   // more decode run better on CUs of their own (32 / 8 heads, 4 chunks of 512
   // over up to 8k and 4 decodes 218 / 204 us, a 2048-token prompt and 10
   // decodes 66 / 60, 4 such prompts and 3 decodes 142 / 134).
-  if (max_tiles > best && e.work < kShortTile * (double)e.tiles &&
-      kDecodeStartUs + mb * kDecodeMinUsPerMB < kLittleDecode * best_us)
-    return 0;
-  return best * num_kv_heads;
+  bool short_tiles(const PrefillEstimate& e, int64_t share, double step_us) const {
+    return max_tiles > share && e.work < 8.0 * (double)e.tiles && mb * kDecodeMinUsPerMB < 0.1 * step_us;
+  }
+  // Time of mva_paged_mixed with its own decode plan.
+  double one_launch_us(const PrefillEstimate& e, int64_t decode_pages, int64_t max_decode_pages, int group) const {
+    const double per_cu = (double)num_kv_heads / (double)num_cus;
+    const double piece = std::min(
+        std::max((double)decode_pages * num_kv_heads / (kPiecesPerWave * kMixedWavesPerCu * (double)num_cus), 4.0), 128.0);
+    const double chunks = std::ceil((double)max_decode_pages / piece);
+    double decode = kOnePageUs * std::min(piece, (double)max_decode_pages);
+    if (chunks > 1)
+      decode += kOneMergeUs + group * (kOnePassUs * std::ceil(chunks / 32.0) + kOneChunkUs * chunks);
+    const double prefill = kOneKeyUs * e.longest;
+    const double work = per_cu * (kOneWorkUs * e.half_work + kOneTileUs * (double)e.half_tiles) + kOneMBUs * mb;
+    return kOneStartUs + std::sqrt(prefill * prefill + decode * decode + work * work);
+  }
+};
+
+bool mixed_step(MixedStep& m, const int64_t* pages, int64_t n, int64_t tokens, int64_t decode_pages, int num_q_heads,
+                int num_kv_heads, int64_t num_cus) {
+  if (n < 0 || tokens < 0 || decode_pages < 0 || num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads ||
+      num_q_heads / num_kv_heads > 16 || (n > 0 && pages == nullptr))
+    return false;
+  m.mb = (double)decode_pages * kPageSize * num_kv_heads * kHeadDim * 2 * 2 * 1e-6;
+  m.max_tiles = tokens / (kPrefillPPRows / (num_q_heads / num_kv_heads)) + n;
+  m.num_kv_heads = num_kv_heads;
+  m.num_cus = num_cus;
+  return true;
+}
+
+}  // namespace
+
+extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, int64_t num_prefill_seqs,
+                                                int64_t num_prefill_tokens, int64_t decode_pages, int num_q_heads,
+                                                int num_kv_heads, int64_t num_cus) {
+  MixedStep m;
+  if (!mixed_step(m, prefill_pages, num_prefill_seqs, num_prefill_tokens, decode_pages, num_q_heads, num_kv_heads,
+                  num_cus))
+    return -1;
+  if (num_prefill_seqs == 0 || num_prefill_tokens == 0) return 0;
+  PrefillEstimate e = estimate_prefill(prefill_pages, even_queries(prefill_pages, num_prefill_seqs, num_prefill_tokens),
+                                       kPrefillPPRows / (num_q_heads / num_kv_heads));
+  int64_t share;
+  const double us = m.fastest(e, &share);
+  return m.short_tiles(e, share, us) ? 0 : share * num_kv_heads;
+}
+
+// The query lengths lie between two batches (packed_queries).  The share is the
+// one that loses least, as a factor of the lowest time at any share: to half
+// over the worse of the two, to half over evenly spread queries between them.
+// Taken as evenly spread, a 2048-token prompt beside seven 8-token chunks over
+// 8000 (32 / 8 heads, 64 decodes of 2000) got 208 CUs for its prefill and 300
+// us, against 226 in mva_paged_mixed; the worse of the two alone gave the step
+// of a 8192-token budget 96 CUs (939 us) in place of 88 (922).  And a step whose
+// estimate is not below mva_paged_mixed's by kLaunchUs (its own launch of the
+// decode merges) and kMargin in either batch is left to that: steps of 15 to 25
+// us were 3 to 4 us slower on CUs of their own.  Over the drawn steps of the
+// fit, against mva_paged_mixed: 90 were slower by more than 3%, the worst by
+// 84%; now one, by 8%, and the mean time is lower too.
+extern "C" int64_t mva_mixed_prefill_share(const int64_t* prefill_pages, int64_t num_prefill_seqs,
+                                           int64_t num_prefill_tokens, int64_t max_query_len, int64_t decode_pages,
+                                           int64_t max_decode_pages, int num_q_heads, int num_kv_heads,
+                                           int64_t num_cus) {
+  constexpr double kMargin = 1.05, kLaunchUs = 3.0;
+  MixedStep m;
+  const int64_t n = num_prefill_seqs;
+  if (!mixed_step(m, prefill_pages, n, num_prefill_tokens, decode_pages, num_q_heads, num_kv_heads, num_cus) ||
+      max_query_len < 0 || max_decode_pages < 0 || max_decode_pages > decode_pages)
+    return -1;
+  if (n == 0 || num_prefill_tokens == 0) return 0;
+  const int group = num_q_heads / num_kv_heads;
+  // A bound that the tokens do not fit under bounds nothing.
+  if (max_query_len < (num_prefill_tokens + n - 1) / n) max_query_len = num_prefill_tokens;
+  PrefillEstimate e[3];
+  double best[3];
+  const int bounds = n > 1 ? 2 : 1;
+  int64_t share = 1;
+  auto estimate = [&](int b, const std::vector<int64_t>& queries) {
+    e[b] = estimate_prefill(prefill_pages, queries, kPrefillPPRows / group);
+    e[b].spare = n > 1 ? (int)std::min<int64_t>(n, kPrefillPieceSlots) : 0;
+    best[b] = m.fastest(e[b], &share);
+  };
+  for (int b = 0; b < bounds; ++b)
+    estimate(b, packed_queries(prefill_pages, n, num_prefill_tokens, max_query_len, b == 0));
+  if (bounds == 2) {
+    estimate(2, even_queries(prefill_pages, n, num_prefill_tokens));
+    auto lost = [&](auto us) { return us(2) / best[2] + std::max(us(0) / best[0], us(1) / best[1]); };
+    m.lowest(
+        share, [&](int64_t p) { return lost([&](int b) { return m.us(e[b], p); }); },
+        [&](int64_t p) { return lost([&](int b) { return m.least_us(e[b], p); }); }, &share);
+  }
+  for (int b = 0; b < bounds; ++b) {
+    const double us = m.us(e[b], share);
+    if (m.short_tiles(e[b], share, us) ||
+        m.one_launch_us(e[b], decode_pages, max_decode_pages, group) < kMargin * us + kLaunchUs)
+      return 0;
+  }
+  return share * num_kv_heads;
 }
 
 extern "C" int mva_paged_mixed_run(const void* q, int64_t q_token_stride, int64_t q_head_stride,

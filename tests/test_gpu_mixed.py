@@ -317,12 +317,15 @@ def test_planned_mixed_matches_the_unplanned_launch(gpu, monkeypatch, hq, hkv, d
     assert_attention_close(first, backend.forward(qd, empty, empty, kc, vc, other).float())
 
 
-def test_captured_planned_mixed_follows_lengths_and_pages(gpu):
+def test_captured_planned_mixed_follows_lengths_and_pages(gpu, monkeypatch):
     # A captured step plans inside its graph: replays read the lengths and
     # page tables of their time, and eager steps between them keep their plan.
+    # (So small a step is left to the launch without a plan; the share is set.)
+    from my_vllm_amd import ops
     from my_vllm_amd.attention_backend import MI355XAttentionBackend
     from tests.test_gpu_prefill import to_device
 
+    monkeypatch.setattr(ops, "mixed_prefill_workgroups", lambda *a: 48)
     backend = MI355XAttentionBackend(32, 8, 128, 16, torch.bfloat16)
     batch = make_paged_batch(173, [90, 200, 1, 1], [400, 200, 900, 1200], 2, 32, 8)
     eager = make_paged_batch(174, [40, 1, 1], [500, 77, 600], 1, 32, 8)
