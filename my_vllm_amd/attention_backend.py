@@ -536,6 +536,9 @@ class MI355XAttentionBackendMixin:
         # The metadata whose device tile plan the prefill workspace holds:
         # the first prefill launch of a step plans, the other layers reuse it.
         self._prefill_planned_for: MI355XAttentionMetadata | None = None
+        # The plan of a captured MIXED step: its capture and stream, metadata
+        # and workspace.
+        self._captured_plan: tuple[tuple[int, int], MI355XAttentionMetadata, torch.Tensor] | None = None
         self._staging = PinnedStaging()
         self._active_graph_state: MI355XFullDecodeGraphState | None = None
         # (key, value, slot_mapping) of the step while forward_with_kv_store
@@ -812,6 +815,7 @@ class MI355XAttentionBackendMixin:
             )
         plan = self.plan_type(batch_type, route, common, metadata)
         self._prefill_planned_for = None  # a new step plans its prefill tiles again
+        self._captured_plan = None
         self._planned_route = route.value
         self._route_counts[route.value] += 1
         return plan
@@ -839,6 +843,24 @@ class MI355XAttentionBackendMixin:
             self._prefill_workspace = ws
             self._prefill_planned_for = None
         return ws
+
+    def _get_captured_plan(self, metadata: MI355XAttentionMetadata, device: torch.device) -> tuple[torch.Tensor, bool]:
+        """(prefill workspace, whether it holds ``metadata``'s plan) for a launch
+        that is being captured.
+
+        A graph plans for itself, in a workspace of its own pool, so its replays
+        see the lengths and page tables of their time and leave the eager steps'
+        plan alone.  The first layer of a capture plans, the later ones on its
+        stream run that plan.  The workspace is held meanwhile: given back, the
+        pool would hand it to the next captured allocation."""
+        key = (_native.host_ops().capture_id(device.index), _native.stream_handle(device))
+        held = self._captured_plan
+        if key[0] and held is not None and held[0] == key and held[1] is metadata:
+            return held[2], True
+        nbytes = ops.prefill_workspace_bytes(metadata.prefill_max_tiles)
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        self._captured_plan = (key, metadata, workspace)
+        return workspace, False
 
     def _get_workspace(self, nbytes: int, device: torch.device) -> torch.Tensor | None:
         if nbytes <= 0:
@@ -1227,15 +1249,12 @@ class MI355XAttentionBackendMixin:
         workspace = self._get_workspace(ws_bytes, q.device)
         if metadata.mixed_prefill_workgroups:
             # The tile plan serves every layer of the step, as in _run_prefill.
-            # A captured launch plans inside the graph, in a workspace of the
-            # graph's own: replays see the lengths and page tables of their
-            # time and leave the eager steps' plan alone.
             capturing = torch.cuda.is_current_stream_capturing()
             if capturing:
-                nbytes = ops.prefill_workspace_bytes(metadata.prefill_max_tiles)
-                prefill_workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+                prefill_workspace, planned = self._get_captured_plan(metadata, q.device)
             else:
                 prefill_workspace = self._get_prefill_workspace(metadata.prefill_max_tiles, q.device)
+                planned = self._prefill_planned_for is metadata
             ops.paged_mixed_run(
                 q, k_cache, v_cache,
                 metadata.block_tables, metadata.seq_lens, metadata.query_start_loc,
@@ -1244,7 +1263,7 @@ class MI355XAttentionBackendMixin:
                 metadata.decode_items, metadata.num_decode_items, metadata.num_decode_waves,
                 metadata.decode_wave_extra, metadata.decode_merges, metadata.num_decode_merges,
                 metadata.num_decode_part_slots, output, workspace, self.softmax_scale,
-                planned=not capturing and self._prefill_planned_for is metadata,
+                planned=planned,
             )
             if not capturing:
                 self._prefill_planned_for = metadata

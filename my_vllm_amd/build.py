@@ -85,7 +85,7 @@ def _build_host_module(target: Path) -> None:
         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
         f"-I{root / 'include'}", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
         str(CSRC_DIR / "host_ops.cpp"), "-o", str(target),
-        f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+        f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-lamdhip64", "-ltorch_cpu", "-ltorch_python",
         f"-L{target.parent}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN",
     ]
     proc = subprocess.run(cmd, capture_output=True, text=True)

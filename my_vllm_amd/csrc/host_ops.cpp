@@ -5,8 +5,8 @@
 // Each function handles the common form of a call (plain strided GPU tensors
 // that pass every check) and returns None for anything else, having done
 // nothing; the caller in ops.py then runs its own checks, which raise the
-// precise error or take the general path.  So this file decides no error and
-// refuses nothing.
+// precise error or take the general path.  So these decide no error and refuse
+// nothing.
 //
 // Why: the same work in Python (tensor attribute reads, reshapes and a ctypes
 // call of 13 to 40 converted arguments) took about 18 us an operator, longer
@@ -415,10 +415,27 @@ PyObject* forward_inputs_ok(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// (device index): number of the graph capture that torch's current stream of
+// the device is in, or 0.
+PyObject* capture_id(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  int64_t device;
+  if (n != 1 || !as_int(a[0], &device)) return PyErr_Format(PyExc_TypeError, "capture_id takes a device index");
+  unsigned long long id = 0;
+  try {
+    hipStreamCaptureStatus status;
+    const hipStream_t stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess || status != hipStreamCaptureStatusActive) id = 0;
+  } catch (const std::exception& error) {
+    return PyErr_Format(PyExc_RuntimeError, "%s", error.what());
+  }
+  return PyLong_FromUnsignedLongLong(id);
+}
+
 #define MVA_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {MVA_METHOD(silu_and_mul),       MVA_METHOD(rms_norm),      MVA_METHOD(fused_add_rms_norm),
                           MVA_METHOD(qk_norm_rope_store), MVA_METHOD(paged_decode),  MVA_METHOD(paged_prefill),
-                          MVA_METHOD(paged_mixed),        MVA_METHOD(forward_inputs_ok), {nullptr, nullptr, 0, nullptr}};
+                          MVA_METHOD(paged_mixed),        MVA_METHOD(forward_inputs_ok), MVA_METHOD(capture_id),
+                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "mva_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

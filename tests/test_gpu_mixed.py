@@ -353,3 +353,52 @@ def test_captured_planned_mixed_follows_lengths_and_pages(gpu, monkeypatch):
         got = out.clone()
         assert torch.equal(got, other.forward(q, empty, empty, kc, vc, other.build_plan(common)))
         assert_attention_close(backend.forward(eq, empty, empty, ekc, evc, e_plan), want)
+
+
+def test_a_capture_plans_once_for_its_layers(gpu, monkeypatch):
+    # The first layer of a captured step plans on the device, the later ones run
+    # its plan; another capture of the same step, and another stream inside a
+    # capture, plan for themselves.  Replays follow the lengths of their time
+    # in every layer.
+    from my_vllm_amd import ops
+    from my_vllm_amd.attention_backend import MI355XAttentionBackend
+    from tests.test_gpu_prefill import to_device
+
+    monkeypatch.setattr(ops, "mixed_prefill_workgroups", lambda *a: 48)
+    planned, run = [], ops.paged_mixed_run
+    monkeypatch.setattr(ops, "paged_mixed_run", lambda *a, **k: (planned.append(k["planned"]), run(*a, **k)))
+    backend = MI355XAttentionBackend(32, 8, 128, 16, torch.bfloat16)
+    batch = make_paged_batch(177, [90, 200, 1, 1], [400, 200, 900, 1200], 2, 32, 8)
+    common, q, kc, vc = to_device(batch, gpu)
+    empty = q.new_empty((0, 8, 128))
+    plan = backend.build_plan(common)
+    layers = [(kc, vc), (vc, kc), (kc, kc)]
+    forward = lambda k, v: backend.forward(q, empty, empty, k, v, plan).clone()  # noqa: E731
+    forward(kc, vc)
+    torch.cuda.synchronize()
+    graphs = []
+    for side in (False, False, True):
+        planned.clear()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            outs = [forward(*layer) for layer in layers]
+            if side:
+                main, other = torch.cuda.current_stream(), torch.cuda.Stream()
+                other.wait_stream(main)
+                with torch.cuda.stream(other):
+                    outs.append(forward(*layers[0]))
+                main.wait_stream(other)
+        assert planned == [False, True, True] + [False] * side
+        graphs.append((graph, outs))
+    assert graphs[0][1][0].data_ptr() != graphs[1][1][0].data_ptr()
+    tables = common.block_tables.clone()
+    eager = MI355XAttentionBackend(32, 8, 128, 16, torch.bfloat16)
+    for step, kv in enumerate((400, 385, 393)):
+        common.seq_lens[0] = kv
+        common.block_tables[0, :25] = tables[2, :25].roll(step)
+        want = [eager.forward(q, empty, empty, k, v, eager.build_plan(common)).clone() for k, v in layers]
+        for graph, outs in graphs:
+            graph.replay()
+            torch.cuda.synchronize()
+            for i, out in enumerate(outs):
+                assert torch.equal(out, want[i % 3])
