@@ -95,7 +95,8 @@ int launch_decode_merge(const DecodeParams& p, const int32_t* merges, int64_t nu
   const int64_t late_rows = p.k_new != nullptr ? p.num_new : 0;
   if (num_merges == 0 && late_rows == 0) return 0;
   const int64_t waves = num_merges * p.group;
-  const bool wide = num_merges > 0 && num_part_slots * p.num_kv_heads > kWideMergeChunks * num_merges;
+  const bool wide = num_merges > 0 && num_part_slots * p.num_kv_heads > kWideMergeChunks * num_merges &&
+                    waves <= 0xffffffffLL / (64 * kWideMergeWaves);  // a launch has fewer than 2^32 threads
   const int64_t per_block = wide ? kWideMergeWaves : 4;
   const int64_t merge_blocks = wide ? waves : (waves + 3) / 4;
   const int64_t blocks = merge_blocks + (late_rows + per_block - 1) / per_block;

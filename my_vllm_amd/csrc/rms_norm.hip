@@ -17,6 +17,8 @@
 #include "mva_capi.h"
 #include "mva_common.h"
 
+#include <algorithm>
+
 namespace mva {
 namespace {
 
@@ -39,6 +41,7 @@ struct RmsArgs {
   int64_t rows_per_group;
   int64_t x_group_stride;
   int64_t out_group_stride;
+  int64_t first_row;  // of this launch (launch_rows)
 };
 
 // Rows and rows per group below 2^31 (the usual case) divide in 32 bits: a
@@ -91,7 +94,7 @@ __global__ __launch_bounds__(kWaves == 1 ? 256 : 64 * kWaves) void rms_norm_vec_
   __shared__ float part[kWaves];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t row = kWaves == 1 ? (int64_t)blockIdx.x * 4 + w : (int64_t)blockIdx.x;
+  const int64_t row = a.first_row + (kWaves == 1 ? (int64_t)blockIdx.x * 4 + w : (int64_t)blockIdx.x);
   if (row >= a.rows) return;
   const int j0 = kWaves == 1 ? lane : (int)threadIdx.x;
   const int nvec = a.hidden >> 3;
@@ -159,7 +162,7 @@ __global__ __launch_bounds__(kWaves == 1 ? 256 : 64 * kWaves) void rms_norm_vec_
 template <typename T, typename W, bool kAdd>
 __global__ __launch_bounds__(256) void rms_norm_scalar_kernel(RmsArgs a) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = a.first_row + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= a.rows) return;
   const T* xr = (const T*)a.x + row_offset(row, a.rows_per_group, a.x_group_stride, a.x_stride);
   const T* rr = kAdd ? (const T*)a.residual + row * a.res_stride : nullptr;
@@ -183,18 +186,26 @@ __global__ __launch_bounds__(256) void rms_norm_scalar_kernel(RmsArgs a) {
   }
 }
 
+// A launch of 2^32 threads or more runs some of its rows only (and reports
+// nothing), so more rows than that (8.4 million at 512 threads a row) take
+// several.
+void launch_rows(void (*kernel)(RmsArgs), RmsArgs a, int rows_per_block, int threads, hipStream_t s) {
+  const int64_t most = 0xffffffffLL / threads * rows_per_block;
+  for (a.first_row = 0; a.first_row < a.rows; a.first_row += most) {
+    const int64_t rows = std::min(most, a.rows - a.first_row);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)((rows + rows_per_block - 1) / rows_per_block)), dim3(threads), 0, s, a);
+  }
+}
+
 template <typename T, typename W, bool kAdd, int kWaves, int kChunks>
 void launch_vec(const RmsArgs& a, hipStream_t s) {
-  const uint32_t blocks = (uint32_t)(kWaves == 1 ? (a.rows + 3) / 4 : a.rows);
-  hipLaunchKernelGGL((rms_norm_vec_kernel<T, W, kWaves, kChunks, kAdd>), dim3(blocks),
-                     dim3(kWaves == 1 ? 256 : 64 * kWaves), 0, s, a);
+  launch_rows(rms_norm_vec_kernel<T, W, kWaves, kChunks, kAdd>, a, kWaves == 1 ? 4 : 1, kWaves == 1 ? 256 : 64 * kWaves,
+              s);
 }
 
 template <typename T, typename W, bool kAdd>
 int launch_rms(const RmsArgs& a, hipStream_t s) {
-  const int64_t blocks = (a.rows + 3) / 4;
-  if (blocks > 0x7fffffffLL) return set_error("rms_norm: too many rows");
-  const dim3 grid((uint32_t)blocks), block(256);
+  if ((a.rows + 3) / 4 > 0x7fffffffLL) return set_error("rms_norm: too many rows");
   uint64_t bits = (uint64_t)(uintptr_t)a.x | (uint64_t)(uintptr_t)a.out | (uint64_t)(uintptr_t)a.weight |
                   (uint64_t)(a.x_stride * (int64_t)sizeof(T)) | (uint64_t)(a.out_stride * (int64_t)sizeof(T)) |
                   (uint64_t)(a.x_group_stride * (int64_t)sizeof(T)) |
@@ -203,7 +214,7 @@ int launch_rms(const RmsArgs& a, hipStream_t s) {
     bits |= (uint64_t)(uintptr_t)a.residual | (uint64_t)(uintptr_t)a.residual_out |
             (uint64_t)(a.res_stride * (int64_t)sizeof(T)) | (uint64_t)(a.res_out_stride * (int64_t)sizeof(T));
   const int nvec = a.hidden / 8;
-  if (a.hidden % 8 == 0 && bits % 16 == 0 && nvec <= 64 * 16 && (nvec <= 64 || a.rows <= 0x7fffffffLL)) {
+  if (a.hidden % 8 == 0 && bits % 16 == 0 && nvec <= 64 * 16) {
     // One 16-byte chunk a lane up to 8 wavefronts a row, two beyond.  One
     // wavefront a row with 8 chunks a lane (hidden 4096) left 61 rows on 16 CUs
     // (6.2 us a launch) and read and wrote 4096 rows in two separate bursts (33 us):
@@ -215,7 +226,7 @@ int launch_rms(const RmsArgs& a, hipStream_t s) {
     else if (nvec <= 512) launch_vec<T, W, kAdd, 8, 1>(a, s);
     else launch_vec<T, W, kAdd, 8, 2>(a, s);
   } else {
-    hipLaunchKernelGGL((rms_norm_scalar_kernel<T, W, kAdd>), grid, block, 0, s, a);
+    launch_rows(rms_norm_scalar_kernel<T, W, kAdd>, a, 4, 256, s);
   }
   return check_launch("rms_norm");
 }

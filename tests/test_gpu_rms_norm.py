@@ -139,3 +139,19 @@ def test_wavefronts_per_row(gpu, hidden, inplace):
     assert torch.equal(res.cpu(), exp_res)
     assert_rms_matches(out, x.float() + r.float(), w, 1e-6)
     assert_rms_matches(ops.rms_norm(x.to(gpu), w.to(gpu), 1e-6), x.float(), w, 1e-6)
+
+
+# 2^32 threads a launch: 8388607 rows of 512 threads, 67108860 of 64 (narrow
+# rows, and rows of another width than a multiple of 8).  Rows overlap in memory
+# (eight elements apart), so the input is small; the outputs are 35, 1 and 1 GB.
+@pytest.mark.parametrize("hidden,most", [(2056, (2 ** 32 - 1) // 512), (8, (2 ** 32 - 1) // 256 * 4),
+                                         (7, (2 ** 32 - 1) // 256 * 4)])
+def test_more_rows_than_one_launch_holds(gpu, hidden, most):
+    rows = most + 70
+    flat = torch.randn(8 * rows + hidden, generator=torch.Generator(gpu).manual_seed(17), device=gpu,
+                       dtype=torch.bfloat16)
+    x = flat.as_strided((rows, hidden), (8, 1))
+    w = torch.randn(hidden, generator=torch.Generator().manual_seed(18)).bfloat16()
+    out = ops.rms_norm(x, w.to(gpu), 1e-6)
+    picked = torch.tensor([0, 1, most // 2, most - 1, most, most + 1, rows - 1], device=gpu)
+    assert_rms_matches(out[picked], x[picked].cpu().float(), w, 1e-6)
