@@ -1265,7 +1265,10 @@ extern "C" int mva_paged_mixed_run(const void* q, int64_t q_token_stride, int64_
   const int64_t n_decode_wgs =
       num_decode_items > 0 ? (num_decode_waves + kMixedDecodeWaves - 1) / kMixedDecodeWaves : 0;
   const int64_t grid = per_head * num_kv_heads + n_decode_wgs;
-  if (prefill_workgroups > 0x7fffff00LL || grid > 0x7fffff00LL) return set_error("paged attention: too many work items");
+  // A launch has fewer than 2^32 threads.
+  constexpr int64_t kMostWorkgroups = 0xffffffffLL / kPrefillPPThreads;
+  if (prefill_workgroups > kMostWorkgroups || grid > kMostWorkgroups)
+    return set_error("paged attention: too many work items");
   if (grid == 0) return 0;
   if (num_decode_items == 0) dp.num_waves = 0;
   // Without prefill sequences there is no plan: the fixed form ends after decode.

@@ -94,6 +94,12 @@ def test_invalid_arguments_fail_before_launch_with_a_message():
         _native.call("mva_paged_prefill_run", 0, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0, 1, 1, 0, 0, 0, 0, 0,
                      32, 8, 128, 16, 1.0, 0, 0)
 
+    # A launch has fewer than 2^32 threads; more workgroups of 512 would be
+    # left out of it without an error.  (Nothing reads the addresses.)
+    with pytest.raises(RuntimeError, match="too many work items"):
+        _native.call("mva_paged_mixed_run", 256, 128, 128, 256, 256, 1, 16384, 1024, 256, 1, 256, 256, 0, 0, 0, 0, 0,
+                     0, 256, 1 << 27, 1 << 27, 256, 0, 0, 0, 256, 128, 128, 256, 1 << 40, 8, 8, 128, 16, 1.0, 0, 0)
+
 
 def test_dtype_codes_match_the_header():
     header = (ROOT / "include" / "my_vllm_amd.h").read_text()
