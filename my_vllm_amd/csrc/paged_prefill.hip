@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <exception>
 #include <functional>
 #include <vector>
 
@@ -1145,6 +1146,8 @@ bool mixed_step(MixedStep& m, const int64_t* pages, int64_t n, int64_t tokens, i
   if (n < 0 || tokens < 0 || decode_pages < 0 || num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads ||
       num_q_heads / num_kv_heads > 16 || (n > 0 && pages == nullptr))
     return false;
+  for (int64_t s = 0; s < n; ++s)
+    if (pages[s] < 0 || pages[s] > 0x7fffffffLL) return false;
   m.mb = (double)decode_pages * kPageSize * num_kv_heads * kHeadDim * 2 * 2 * 1e-6;
   m.max_tiles = tokens / (kPrefillPPRows / (num_q_heads / num_kv_heads)) + n;
   m.num_kv_heads = num_kv_heads;
@@ -1156,7 +1159,7 @@ bool mixed_step(MixedStep& m, const int64_t* pages, int64_t n, int64_t tokens, i
 
 extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, int64_t num_prefill_seqs,
                                                 int64_t num_prefill_tokens, int64_t decode_pages, int num_q_heads,
-                                                int num_kv_heads, int64_t num_cus) {
+                                                int num_kv_heads, int64_t num_cus) try {
   MixedStep m;
   if (!mixed_step(m, prefill_pages, num_prefill_seqs, num_prefill_tokens, decode_pages, num_q_heads, num_kv_heads,
                   num_cus))
@@ -1167,6 +1170,8 @@ extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, in
   int64_t share;
   const double us = m.fastest(e, &share);
   return m.short_tiles(e, share, us) ? 0 : share * num_kv_heads;
+} catch (const std::exception&) {  // out of memory
+  return -1;
 }
 
 // The query lengths lie between two batches (packed_queries).  The share is the
@@ -1184,7 +1189,7 @@ extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, in
 extern "C" int64_t mva_mixed_prefill_share(const int64_t* prefill_pages, int64_t num_prefill_seqs,
                                            int64_t num_prefill_tokens, int64_t max_query_len, int64_t decode_pages,
                                            int64_t max_decode_pages, int num_q_heads, int num_kv_heads,
-                                           int64_t num_cus) {
+                                           int64_t num_cus) try {
   constexpr double kMargin = 1.05, kLaunchUs = 3.0;
   MixedStep m;
   const int64_t n = num_prefill_seqs;
@@ -1220,6 +1225,8 @@ extern "C" int64_t mva_mixed_prefill_share(const int64_t* prefill_pages, int64_t
       return 0;
   }
   return share * num_kv_heads;
+} catch (const std::exception&) {  // out of memory
+  return -1;
 }
 
 extern "C" int mva_paged_mixed_run(const void* q, int64_t q_token_stride, int64_t q_head_stride,

@@ -535,6 +535,13 @@ def test_mixed_step_gets_cus_of_its_own_where_that_is_faster(hq, hkv, kv, tokens
 
 def test_mixed_share_arguments():
     args = ([20, 4], 300, 50, 32, 8, 256)
+    for pages in ([20, -1], [1 << 31, 4]):
+        for more in ((), (200, 9)):
+            with pytest.raises(ValueError):
+                ops.mixed_prefill_workgroups(pages, *args[1:], *more)
+    # No walk over every tile of an absurd batch (the two would be 60 billion).
+    for more in ((), (10 ** 12, 9)):
+        assert ops.mixed_prefill_workgroups([(1 << 31) - 1] * 2, 10 ** 12, 50, 32, 8, 256, *more) >= 0
     assert ops.mixed_prefill_workgroups(*args, 0, 9) % 8 == 0  # no bound on the queries
     for longest, decode in ((-1, 9), (200, -1), (200, 51)):
         with pytest.raises(ValueError):
