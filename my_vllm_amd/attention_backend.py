@@ -536,9 +536,10 @@ class MI355XAttentionBackendMixin:
         # The metadata whose device tile plan the prefill workspace holds:
         # the first prefill launch of a step plans, the other layers reuse it.
         self._prefill_planned_for: MI355XAttentionMetadata | None = None
-        # The plan of a captured MIXED step: its capture and stream, metadata
-        # and workspace.
-        self._captured_plan: tuple[tuple[int, int], MI355XAttentionMetadata, torch.Tensor] | None = None
+        self._prefill_planned_versions: tuple | None = None
+        # The plan of a captured MIXED step: its capture, stream and tensor
+        # versions, metadata and workspace.
+        self._captured_plan: tuple[tuple, MI355XAttentionMetadata, torch.Tensor] | None = None
         self._staging = PinnedStaging()
         self._active_graph_state: MI355XFullDecodeGraphState | None = None
         # (key, value, slot_mapping) of the step while forward_with_kv_store
@@ -844,6 +845,21 @@ class MI355XAttentionBackendMixin:
             self._prefill_planned_for = None
         return ws
 
+    def _plan_versions(self, metadata: MI355XAttentionMetadata) -> tuple:
+        """The versions of the tensors that a tile plan is made from: torch counts
+        their in-place changes (but those of inference tensors)."""
+        tensors = (metadata.seq_lens, metadata.query_start_loc, metadata.block_tables)
+        return tuple(None if t.is_inference() else t._version for t in tensors)
+
+    def _take_prefill_plan(self, metadata: MI355XAttentionMetadata, device: torch.device) -> tuple[torch.Tensor, bool]:
+        """(prefill workspace, whether it holds ``metadata``'s plan); the launch
+        that follows leaves that plan there."""
+        workspace = self._get_prefill_workspace(metadata.prefill_max_tiles, device)
+        versions = self._plan_versions(metadata)
+        planned = self._prefill_planned_for is metadata and self._prefill_planned_versions == versions
+        self._prefill_planned_for, self._prefill_planned_versions = None, versions
+        return workspace, planned
+
     def _get_captured_plan(self, metadata: MI355XAttentionMetadata, device: torch.device) -> tuple[torch.Tensor, bool]:
         """(prefill workspace, whether it holds ``metadata``'s plan) for a launch
         that is being captured.
@@ -853,7 +869,8 @@ class MI355XAttentionBackendMixin:
         plan alone.  The first layer of a capture plans, the later ones on its
         stream run that plan.  The workspace is held meanwhile: given back, the
         pool would hand it to the next captured allocation."""
-        key = (_native.host_ops().capture_id(device.index), _native.stream_handle(device))
+        key = (_native.host_ops().capture_id(device.index), _native.stream_handle(device),
+               self._plan_versions(metadata))
         held = self._captured_plan
         if key[0] and held is not None and held[0] == key and held[1] is metadata:
             return held[2], True
@@ -1226,7 +1243,7 @@ class MI355XAttentionBackendMixin:
         # metadata builds it on the device, later layers stream it as it is
         # (the reference's FlashInfer wrapper plans once per step in build_plan,
         # nanovllm/layers/attention_backend.py:810-825, and runs per layer, :992-994).
-        workspace = self._get_prefill_workspace(metadata.prefill_max_tiles, q.device)
+        workspace, planned = self._take_prefill_plan(metadata, q.device)
         ops.paged_prefill(
             q,
             k_cache,
@@ -1239,7 +1256,7 @@ class MI355XAttentionBackendMixin:
             workspace,
             output,
             self.softmax_scale,
-            planned=self._prefill_planned_for is metadata,
+            planned=planned,
         )
         self._prefill_planned_for = metadata
 
@@ -1253,8 +1270,7 @@ class MI355XAttentionBackendMixin:
             if capturing:
                 prefill_workspace, planned = self._get_captured_plan(metadata, q.device)
             else:
-                prefill_workspace = self._get_prefill_workspace(metadata.prefill_max_tiles, q.device)
-                planned = self._prefill_planned_for is metadata
+                prefill_workspace, planned = self._take_prefill_plan(metadata, q.device)
             ops.paged_mixed_run(
                 q, k_cache, v_cache,
                 metadata.block_tables, metadata.seq_lens, metadata.query_start_loc,

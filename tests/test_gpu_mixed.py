@@ -14,6 +14,7 @@ import torch
 
 from my_vllm_amd.contract import AttentionRoute
 from my_vllm_amd.contract import BatchType
+from oracle.reference import paged_attention
 from workloads import config_mixed, make_paged_batch
 from tests._util import assert_attention_close, set_decode_planning
 from tests.test_gpu_prefill import expected, run_backend
@@ -402,3 +403,36 @@ def test_a_capture_plans_once_for_its_layers(gpu, monkeypatch):
             torch.cuda.synchronize()
             for i, out in enumerate(outs):
                 assert torch.equal(out, want[i % 3])
+
+
+@pytest.mark.parametrize("prefills", [2, 4])
+def test_changed_lengths_and_pages_are_planned_again(gpu, monkeypatch, prefills):
+    # Page tables or lengths changed in place between two forwards of one plan
+    # (page counts as they were): the tile plan is built again, for MIXED
+    # (prefills 2) as for PREFILL; unchanged ones stream it.
+    from my_vllm_amd import ops
+    from my_vllm_amd.attention_backend import MI355XAttentionBackend
+    from tests.test_gpu_prefill import to_device
+
+    monkeypatch.setattr(ops, "mixed_prefill_workgroups", lambda *a: 48)
+    planned = []
+    for name in ("paged_mixed_run", "paged_prefill"):
+        def spy(*a, run=getattr(ops, name), **k):
+            planned.append(k["planned"])
+            return run(*a, **k)
+        monkeypatch.setattr(ops, name, spy)
+    backend = MI355XAttentionBackend(32, 8, 128, 16, torch.bfloat16)
+    batch = make_paged_batch(179, [90, 200, 1, 1], [400, 200, 900, 1200], prefills, 32, 8)
+    common, q, kc, vc = to_device(batch, gpu)
+    empty = q.new_empty((0, 8, 128))
+    plan = backend.build_plan(common)
+    for step, change in enumerate((None, None, "pages", None, "lengths")):
+        if change == "pages":
+            common.block_tables[0, :25] = common.block_tables[2, :25].clone()
+        elif change == "lengths":
+            common.seq_lens[0] = 391
+        out = backend.forward(q, empty, empty, kc, vc, plan).clone()
+        assert planned == [False, True, False, True, False][:step + 1]
+        want = paged_attention(batch.q, batch.k_cache, batch.v_cache, common.block_tables.cpu(), batch.query_lengths,
+                               common.seq_lens.tolist())
+        assert_attention_close(out, want)
