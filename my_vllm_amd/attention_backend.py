@@ -537,8 +537,8 @@ class MI355XAttentionBackendMixin:
         # the first prefill launch of a step plans, the other layers reuse it.
         self._prefill_planned_for: MI355XAttentionMetadata | None = None
         self._prefill_planned_versions: tuple | None = None
-        # The plan of a captured MIXED step: its capture, stream and tensor
-        # versions, metadata and workspace.
+        # The plan of a captured step: its capture, stream and tensor versions,
+        # metadata and workspace.
         self._captured_plan: tuple[tuple, MI355XAttentionMetadata, torch.Tensor] | None = None
         self._staging = PinnedStaging()
         self._active_graph_state: MI355XFullDecodeGraphState | None = None
@@ -851,33 +851,35 @@ class MI355XAttentionBackendMixin:
         tensors = (metadata.seq_lens, metadata.query_start_loc, metadata.block_tables)
         return tuple(None if t.is_inference() else t._version for t in tensors)
 
-    def _take_prefill_plan(self, metadata: MI355XAttentionMetadata, device: torch.device) -> tuple[torch.Tensor, bool]:
-        """(prefill workspace, whether it holds ``metadata``'s plan); the launch
-        that follows leaves that plan there."""
-        workspace = self._get_prefill_workspace(metadata.prefill_max_tiles, device)
-        versions = self._plan_versions(metadata)
-        planned = self._prefill_planned_for is metadata and self._prefill_planned_versions == versions
-        self._prefill_planned_for, self._prefill_planned_versions = None, versions
-        return workspace, planned
-
-    def _get_captured_plan(self, metadata: MI355XAttentionMetadata, device: torch.device) -> tuple[torch.Tensor, bool]:
-        """(prefill workspace, whether it holds ``metadata``'s plan) for a launch
-        that is being captured.
+    def _take_prefill_plan(self, metadata: MI355XAttentionMetadata,
+                           device: torch.device) -> tuple[torch.Tensor, bool, tuple]:
+        """The prefill workspace of the launch that follows, whether it holds
+        ``metadata``'s plan, and what :meth:`_keep_prefill_plan` takes once the
+        launch went out (until then no plan counts as built).
 
         A graph plans for itself, in a workspace of its own pool, so its replays
-        see the lengths and page tables of their time and leave the eager steps'
-        plan alone.  The first layer of a capture plans, the later ones on its
-        stream run that plan.  The workspace is held meanwhile: given back, the
-        pool would hand it to the next captured allocation."""
-        key = (_native.host_ops().capture_id(device.index), _native.stream_handle(device),
-               self._plan_versions(metadata))
-        held = self._captured_plan
-        if key[0] and held is not None and held[0] == key and held[1] is metadata:
-            return held[2], True
-        nbytes = ops.prefill_workspace_bytes(metadata.prefill_max_tiles)
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        self._captured_plan = (key, metadata, workspace)
-        return workspace, False
+        see the lengths and page tables of their time, and no eager step lays
+        another plan there.  The first layer of a capture plans, the later ones
+        on its stream run that plan.  The workspace is held meanwhile: given
+        back, the pool would hand it to the next captured allocation."""
+        versions = self._plan_versions(metadata)
+        if torch.cuda.is_current_stream_capturing():
+            key = (_native.host_ops().capture_id(device.index), _native.stream_handle(device), versions)
+            held, self._captured_plan = self._captured_plan, None
+            if key[0] and held is not None and held[0] == key and held[1] is metadata:
+                return held[2], True, key
+            nbytes = ops.prefill_workspace_bytes(metadata.prefill_max_tiles)
+            return torch.empty(nbytes, dtype=torch.uint8, device=device), False, key
+        workspace = self._get_prefill_workspace(metadata.prefill_max_tiles, device)
+        planned = self._prefill_planned_for is metadata and self._prefill_planned_versions == versions
+        self._prefill_planned_for = None
+        return workspace, planned, (None, None, versions)
+
+    def _keep_prefill_plan(self, metadata: MI355XAttentionMetadata, workspace: torch.Tensor, key: tuple) -> None:
+        if key[0] is None:
+            self._prefill_planned_for, self._prefill_planned_versions = metadata, key[2]
+        else:
+            self._captured_plan = (key, metadata, workspace)
 
     def _get_workspace(self, nbytes: int, device: torch.device) -> torch.Tensor | None:
         if nbytes <= 0:
@@ -1243,7 +1245,7 @@ class MI355XAttentionBackendMixin:
         # metadata builds it on the device, later layers stream it as it is
         # (the reference's FlashInfer wrapper plans once per step in build_plan,
         # nanovllm/layers/attention_backend.py:810-825, and runs per layer, :992-994).
-        workspace, planned = self._take_prefill_plan(metadata, q.device)
+        workspace, planned, key = self._take_prefill_plan(metadata, q.device)
         ops.paged_prefill(
             q,
             k_cache,
@@ -1258,7 +1260,7 @@ class MI355XAttentionBackendMixin:
             self.softmax_scale,
             planned=planned,
         )
-        self._prefill_planned_for = metadata
+        self._keep_prefill_plan(metadata, workspace, key)
 
     def _run_mixed(self, q, k_cache, v_cache, common, metadata: MI355XAttentionMetadata, output) -> None:
         group = self.num_q_heads // self.num_kv_heads
@@ -1266,11 +1268,7 @@ class MI355XAttentionBackendMixin:
         workspace = self._get_workspace(ws_bytes, q.device)
         if metadata.mixed_prefill_workgroups:
             # The tile plan serves every layer of the step, as in _run_prefill.
-            capturing = torch.cuda.is_current_stream_capturing()
-            if capturing:
-                prefill_workspace, planned = self._get_captured_plan(metadata, q.device)
-            else:
-                prefill_workspace, planned = self._take_prefill_plan(metadata, q.device)
+            prefill_workspace, planned, key = self._take_prefill_plan(metadata, q.device)
             ops.paged_mixed_run(
                 q, k_cache, v_cache,
                 metadata.block_tables, metadata.seq_lens, metadata.query_start_loc,
@@ -1281,8 +1279,7 @@ class MI355XAttentionBackendMixin:
                 metadata.num_decode_part_slots, output, workspace, self.softmax_scale,
                 planned=planned,
             )
-            if not capturing:
-                self._prefill_planned_for = metadata
+            self._keep_prefill_plan(metadata, prefill_workspace, key)
             return
         ops.paged_mixed(
             q,

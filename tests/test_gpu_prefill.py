@@ -520,3 +520,47 @@ def test_tiles_in_turns(gpu, q, kv, turns, cut, dtype):
     for i, out in enumerate(outs):
         assert torch.equal(out, outs[i // 3 * 3])
         assert_attention_close(out, want)
+
+
+@pytest.mark.parametrize("mode", ["unified", "split"])
+def test_captured_prefill_plans_for_itself(gpu, mode):
+    # A PREFILL (or MIXED_SPLIT) step captured after an eager forward of the same
+    # plan: its graph plans, once for its layers, so replays follow the page
+    # tables of their time and survive eager steps that plan another batch.
+    q, kv = [90, 200, 1, 1], [400, 200, 900, 1200]
+    batch = make_paged_batch(231, q, kv, 4 if mode == "unified" else 2, 32, 8)
+    other = make_paged_batch(232, [40, 500], [500, 600], 2, 32, 8)
+    common, qd, kc, vc = to_device(batch, gpu)
+    o_common, oq, okc, ovc = to_device(other, gpu)
+    backend, eager = (MI355XAttentionBackend(32, 8, 128, 16, torch.bfloat16, attention_mode=mode) for _ in range(2))
+    empty = qd.new_empty((0, 8, 128))
+    plan = backend.build_plan(common)
+    backend.forward(qd, empty, empty, kc, vc, plan)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = [backend.forward(qd, empty, empty, k, v, plan).clone() for k, v in ((kc, vc), (vc, kc))]
+    o_plan = backend.build_plan(o_common)
+    tables = common.block_tables.clone()
+    for step in range(3):
+        common.block_tables[0, :25] = tables[2, :25].roll(step)
+        assert_attention_close(backend.forward(oq, empty, empty, okc, ovc, o_plan).cpu(), expected(other))
+        graph.replay()
+        torch.cuda.synchronize()
+        for out, (k, v) in zip(outs, ((kc, vc), (vc, kc))):
+            assert torch.equal(out, eager.forward(qd, empty, empty, k, v, eager.build_plan(common)))
+
+
+def test_no_plan_is_kept_of_a_launch_that_was_refused(gpu):
+    # A launch refused for its query's alignment lays no plan; the next one of
+    # the same step must build it.
+    batch = make_paged_batch(233, [90, 200], [400, 200], 2, 32, 8)
+    common, q, kc, vc = to_device(batch, gpu)
+    backend = MI355XAttentionBackend(32, 8, 128, 16, torch.bfloat16)
+    empty = q.new_empty((0, 8, 128))
+    plan = backend.build_plan(common)
+    shifted = torch.empty(q.numel() + 1, dtype=q.dtype, device=gpu)[1:].view(q.shape)
+    with pytest.raises(RuntimeError, match="aligned"):
+        backend.forward(shifted, empty, empty, kc, vc, plan)
+    assert backend._prefill_planned_for is None
+    assert_attention_close(backend.forward(q, empty, empty, kc, vc, plan).cpu(), expected(batch))
