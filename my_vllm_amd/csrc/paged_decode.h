@@ -341,8 +341,9 @@ __device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int 
 // page-table registers (readlane); the loop issues no memory access per
 // page other than the page itself.
 //
-// A split piece stores its partial when it ends; decode_merge_wave combines
-// the partials in the kernel that follows on the same stream.
+// A split piece stores its partial when it ends; decode_merge_kernel combines
+// the partials on the same stream, or, in launches that merge themselves
+// (kMergeInLaunch), the wavefront whose piece arrives last.
 //
 // `progress` (LDS, one int per wavefront of an 8-wavefront workgroup, or
 // nullptr): wavefronts w and w ^ 4 share a SIMD and stream the same pages for

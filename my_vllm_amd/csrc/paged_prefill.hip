@@ -449,8 +449,10 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_fixed_kernel(
 // (128 KB of LDS): the first `n_prefill` (a whole number per KV head) run the
 // prefill plan as the prefill-only kernels do, the rest run eight decode
 // wavefronts each, as the piece-list decode kernel does.  With kFixed the
-// plan has at most one item per prefill workgroup of a head; otherwise tiles
-// are claimed, and a decode workgroup whose pieces are done joins in.
+// plan has at most one item per prefill workgroup of a head.  Otherwise items
+// are dealt out to the prefill workgroups in turns up to kPrefillTurns rounds,
+// and a decode workgroup whose pieces are done ends; beyond that tiles are
+// claimed, and it joins in.
 //
 // The two parts have different bounds (the matrix cores and HBM), so they are
 // best run side by side; sharing every CU between decode wavefronts and a
@@ -464,7 +466,8 @@ __global__ __launch_bounds__(kPrefillPPThreads) void paged_prefill_fixed_kernel(
 // a step: 300 tokens over 1936 and 20 decodes of 2250 (32 / 8 heads, fp16)
 // 69 -> 47, 2 chunks over 4k and 64 decodes of 2700 211 -> 176, 4 chunks of a
 // budget of 8192 and 256 decodes of 4391 974 -> 914, 1 decode of 12695 beside
-// 109 prompt tokens (64 / 8 heads) 168 -> 20.  Split-K decode segments are
+// 109 prompt tokens (64 / 8 heads) 168 -> 20; small steps are left to that
+// kernel (mva_mixed_prefill_share).  Split-K decode segments are
 // merged by the merge kernel that follows: merging inside the launch cost 5
 // to 17 us more (the merges run one after another on the last wavefronts).
 template <typename T, bool kFixed>

@@ -92,7 +92,8 @@ __device__ inline typename FloatsOf<kPer>::type load_w(const void* w, int64_t i)
 // may alias the inputs.  Distinct rows never overlap, so reading an item's
 // rows before writing any of them is exact even in place.  The q / k outputs
 // are stored non-temporally (the launch does not read them again): 3 us of
-// 4000 tokens at 32 / 8 heads.
+// 4000 tokens at 32 / 8 heads by itself, level with the launches that read them
+// (norm, GEMM, this kernel, copy, norm, GEMM of 4099 tokens: 446.0 / 446.8 us).
 template <typename T, typename W, typename SlotT, int kPer, int kChunk>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(PrologueArgs a) {
   // Separate fp32 multiplies and adds, as torch evaluates the rotation (no

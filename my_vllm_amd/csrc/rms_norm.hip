@@ -218,8 +218,11 @@ int launch_rms(const RmsArgs& a, hipStream_t s) {
     // One 16-byte chunk a lane up to 8 wavefronts a row, two beyond.  One
     // wavefront a row with 8 chunks a lane (hidden 4096) left 61 rows on 16 CUs
     // (6.2 us a launch) and read and wrote 4096 rows in two separate bursts (33 us):
-    // see pick_prologue_kernel for a layer's launches.  Non-temporal stores:
-    // 110.4 against 120.9 us for those of 4000 tokens.
+    // see pick_prologue_kernel for a layer's launches.  Non-temporal stores: 110.4
+    // against 120.9 us for those of 4000 tokens, where nothing reads them.  The
+    // reader pays that back: norm of 4099 x 4096 20.7 / 22.1 us, with the GEMM
+    // (4096 x 6144) on its output 203.8 / 201.9; 2048 rows 100.8 / 101.3; norm,
+    // GEMM, prologue, copy, norm and GEMM of 4099 446.0 / 446.8.
     if (nvec <= 64) launch_vec<T, W, kAdd, 1, 1>(a, s);
     else if (nvec <= 128) launch_vec<T, W, kAdd, 2, 1>(a, s);
     else if (nvec <= 256) launch_vec<T, W, kAdd, 4, 1>(a, s);
