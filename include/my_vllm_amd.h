@@ -441,13 +441,14 @@ int mva_paged_mixed(const void* q, int64_t q_token_stride, int64_t q_head_stride
  * tokens and where mva_paged_mixed is estimated faster (small steps, and those
  * whose query lengths may be so uneven that a share of CUs fits only some of
  * what they can be); -1 for invalid arguments.  prefill_pages holds the pages
- * of each prefill sequence, max_query_len bounds their queries (0: unknown),
- * decode_pages and max_decode_pages are the decode sequences' total and
- * largest.  Host only.
+ * of each prefill sequence, max_query_len bounds their queries (0: unknown);
+ * num_decode_seqs decode sequences have decode_pages pages, the largest
+ * max_decode_pages.  Host only.
  */
 int64_t mva_mixed_prefill_share(const int64_t* prefill_pages, int64_t num_prefill_seqs,
-                                int64_t num_prefill_tokens, int64_t max_query_len, int64_t decode_pages,
-                                int64_t max_decode_pages, int num_q_heads, int num_kv_heads, int64_t num_cus);
+                                int64_t num_prefill_tokens, int64_t max_query_len, int64_t num_decode_seqs,
+                                int64_t decode_pages, int64_t max_decode_pages, int num_q_heads,
+                                int num_kv_heads, int64_t num_cus);
 
 /*
  * The share alone, for queries spread evenly over the prefill sequences: the

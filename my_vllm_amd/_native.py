@@ -183,7 +183,7 @@ _SIGNATURES = {
             _i32, _i32, _i32, _i32, _f32, _i32, _c_void_p,
         ],
     ),
-    "mva_mixed_prefill_share": (_i64, [_c_void_p, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _i64]),
+    "mva_mixed_prefill_share": (_i64, [_c_void_p, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _i64]),
     "mva_mixed_prefill_workgroups": (_i64, [_c_void_p, _i64, _i64, _i64, _i32, _i32, _i64]),
     "mva_paged_mixed_run": (
         _i32,

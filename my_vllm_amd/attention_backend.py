@@ -702,7 +702,8 @@ class MI355XAttentionBackendMixin:
                 cus = _num_cus(block_tables.device)
                 mixed_prefill_workgroups = ops.mixed_prefill_workgroups(
                     counts[:common.num_prefill_seqs], common.num_prefill_tokens, int(decode_counts.sum()),
-                    self.num_q_heads, self.num_kv_heads, cus, common.max_q_len, int(decode_counts.max()))
+                    self.num_q_heads, self.num_kv_heads, cus, common.max_q_len, common.num_decode_seqs,
+                    int(decode_counts.max()))
             if mixed_prefill_workgroups:
                 # Decode ranges for the CUs that the prefill tiles leave.
                 waves = max(1, cus - mixed_prefill_workgroups) * _LISTED_WAVES_PER_CU

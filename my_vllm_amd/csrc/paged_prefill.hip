@@ -936,31 +936,35 @@ extern "C" int mva_paged_mixed(const void* q, int64_t q_token_stride, int64_t q_
 
 // Host estimates for MIXED steps (see mva_mixed_prefill_share): the time of
 // mva_paged_mixed_run at a share of the CUs for its prefill part, and that of
-// mva_paged_mixed, in microseconds fitted to sweeps of the share over 730 drawn
-// steps on one MI355X (7000 timings; one prefill sequence or more, even and
-// skewed, 1 to 900 MB of decode K/V and more).  Of each timing over the
-// estimate, the 5th and 95th percentiles: decode part 0.90 and 1.09, fixed
-// prefill form 0.92 and 1.10, turns 0.88 and 1.20, mva_paged_mixed 0.84 and
-// 1.14 up to 30 us, 0.88 and 1.09 from 150 us on.  Tiles and pieces are counted
-// as plan_pieces counts them, but its prices are its own: the two need not
-// agree, and a share that is off costs time and nothing else.
+// mva_paged_mixed, in microseconds fitted to sweeps of the share over 1170 drawn
+// steps on one MI355X (11400 timings; one prefill sequence or more, even and
+// skewed, less than 1 MB to 2.5 GB of decode K/V).  Of a timing over the
+// estimate, the 5th and 95th percentiles: decode-bound 0.90 and 1.10,
+// prefill-bound with an item a workgroup 0.92 and 1.09, in rounds 0.89 and
+// 1.17; mva_paged_mixed 0.88 and 1.10 up to 30 us, 0.80 and 1.29 from there to
+// 150, 0.90 and 1.11 beyond.  Tiles and pieces are counted as plan_pieces counts
+// them, but its prices are its own: the two need not agree, and a share that is
+// off costs time and nothing else.
 namespace {
 
-// Decode part: a CU of eight wavefronts streams 1 MB in 24.1 beside 0.0367 per
-// MB of the launch, and all of them together no faster than 0.1752 (5.7 TB/s).
-constexpr double kDecodeStartUs = 9.7, kDecodeUsPerMB = 0.0367, kDecodeUsPerMBCu = 24.1, kDecodeMinUsPerMB = 0.1752;
+// Decode part: a CU of eight wavefronts streams 1 MB in 23.65 beside 0.0375 per
+// MB of the launch, and all of them together no faster than 0.1746 (5.7 TB/s).
+constexpr double kDecodeStartUs = 7.81, kDecodeUsPerMB = 0.0375, kDecodeUsPerMBCu = 23.65, kDecodeMinUsPerMB = 0.1746;
 // Prefill part, one item a workgroup: whole tiles, or tiles cut into k.
-constexpr double kWholeStartUs = 12.5, kWholeKeyUs = 1.37;
-constexpr double kCutStartUs = 17.0, kCutPieceUs = 0.95, kCutKeyUs = 1.41;
+constexpr double kWholeStartUs = 11.71, kWholeKeyUs = 1.334;
+constexpr double kCutStartUs = 15.75, kCutPieceUs = 1.017, kCutKeyUs = 1.347;
 // More tiles than workgroups: key tiles and items a workgroup, the tiles that
 // must share one, and what a cut plan in turns has on top.
-constexpr double kRoundsStartUs = 10.0, kRoundsKeyUs = 1.57, kRoundsItemUs = 4.7, kTogetherUs = 1.43;
-constexpr double kItemKeys = 2.5, kTurnsCutUs = 17.3;
+constexpr double kRoundsStartUs = 9.48, kRoundsKeyUs = 1.559, kRoundsItemUs = 4.56, kTogetherUs = 1.403;
+constexpr double kItemKeys = 2.5, kTurnsCutUs = 16.0;
+// The parts slow each other down: the longer one by kBeside of the shorter,
+// times the root of their ratio.
+constexpr double kBeside = 0.151;
 // mva_paged_mixed: the longest tile, the longest decode piece and its merge
-// (one pass of 32 chunks a query head after another), and the work of a CU,
-// in a root of squares.
-constexpr double kOneStartUs = 7.6, kOneKeyUs = 1.28, kOnePageUs = 0.9, kOneMergeUs = 0.58, kOnePassUs = 0.866,
-                 kOneChunkUs = 0.042, kOneWorkUs = 0.747, kOneTileUs = 5.6, kOneMBUs = 0.212;
+// (one pass of 32 chunks a query head after another), and the work of a CU
+// with its decode wavefronts' pieces, in a root of squares.
+constexpr double kOneStartUs = 4.05, kOneKeyUs = 1.287, kOnePageUs = 1.985, kOnePassUs = 0.912, kOneChunkUs = 0.031,
+                 kOneWorkUs = 0.778, kOneTileUs = 3.42, kOneMBUs = 0.164, kOnePieceUs = 14.95;
 constexpr double kMixedWavesPerCu = 6.0, kPiecesPerWave = 1.5;  // of its decode plan (plan_decode_claims)
 constexpr int64_t kListTiles = 1024;  // batches of more tiles are taken as even
 
@@ -972,6 +976,8 @@ struct PrefillEstimate {
   std::vector<int> keys;  // 64-key tiles of each 256-row tile, longest first (empty beyond kListTiles)
   // Pieces of all tiles when the longest is cut into k, once asked for.
   int64_t pieces[kPrefillMaxPieces + 1] = {};
+  // Of the step at each share: a lower bound, and its time, 0 where not priced yet.
+  std::vector<double> least_us, us;
 };
 
 // 64-key tiles that query tile t of a sequence of q queries and kv keys sees.
@@ -1045,8 +1051,11 @@ std::vector<int64_t> packed_queries(const int64_t* pages, int64_t n, int64_t tok
 
 // No prefill time on per_head workgroups per KV head is below this: the
 // tiles' work in equal parts.
-double least_prefill_us(const PrefillEstimate& e, int64_t per_head) {
-  return kRoundsStartUs + kWholeKeyUs * (e.work / (double)per_head);
+double least_prefill_us(const PrefillEstimate& e, int64_t per_head, int64_t max_tiles) {
+  if (max_tiles > per_head)
+    return kRoundsStartUs + (kRoundsKeyUs * e.work + kRoundsItemUs * (double)e.tiles) / (double)per_head;
+  const double even = std::max(e.work / (double)per_head, (double)e.longest / kPrefillMaxPieces);
+  return std::min(kWholeStartUs + kWholeKeyUs * e.longest, kCutStartUs + 2 * kCutPieceUs + kCutKeyUs * even);
 }
 
 // Time of the prefill part on per_head workgroups per KV head.
@@ -1082,43 +1091,45 @@ struct MixedStep {
   int num_kv_heads;
   int64_t num_cus;
 
-  double decode_us(int64_t p) const {
+  int64_t shares() const { return num_kv_heads < num_cus ? (num_cus - 1) / num_kv_heads : 1; }
+  // With a prefill part of prefill_us; grows with it.
+  double beside_us(int64_t p, double prefill_us) const {
     const int64_t left = num_cus - p * num_kv_heads;
-    const double d = kDecodeUsPerMB + kDecodeUsPerMBCu / (double)(left > 0 ? left : 1);
-    return kDecodeStartUs + mb * std::max(d, kDecodeMinUsPerMB);
+    const double rate = kDecodeUsPerMB + kDecodeUsPerMBCu / (double)(left > 0 ? left : 1);
+    const double decode_us = kDecodeStartUs + mb * std::max(rate, kDecodeMinUsPerMB);
+    const double longer = std::max(decode_us, prefill_us), shorter = std::min(decode_us, prefill_us);
+    return longer + kBeside * shorter * std::sqrt(shorter / longer);
+  }
+  // Prices e's lower bounds.
+  void bound(PrefillEstimate& e) const {
+    e.us.assign(shares() + 1, 0);
+    e.least_us.assign(shares() + 1, 0);
+    for (int64_t p = 1; p <= shares(); ++p) e.least_us[p] = beside_us(p, least_prefill_us(e, p, max_tiles));
   }
   double us(PrefillEstimate& e, int64_t p) const {
-    return std::max(decode_us(p), prefill_part_us(e, p, max_tiles, num_kv_heads));
+    if (e.us[p] == 0) e.us[p] = beside_us(p, prefill_part_us(e, p, max_tiles, num_kv_heads));
+    return e.us[p];
   }
-  double least_us(const PrefillEstimate& e, int64_t p) const { return std::max(decode_us(p), least_prefill_us(e, p)); }
-  int64_t shares() const { return num_kv_heads < num_cus ? (num_cus - 1) / num_kv_heads : 1; }
-  // The smallest share at which decode takes the least that prefill can: both
-  // times are near their lowest there.
-  int64_t meet(const PrefillEstimate& e) const {
-    int64_t lo = 1, hi = shares();
-    while (lo < hi) {
-      const int64_t mid = (lo + hi) / 2;
-      if (decode_us(mid) >= least_prefill_us(e, mid)) hi = mid;
-      else lo = mid + 1;
-    }
-    return lo;
-  }
-  // The lowest cost of any share, and the smallest share that has it.
-  // `start` is priced first, and most others fall to their lower bound: at one
-  // KV head, 255 shares, pricing each cost 15 to 250 us a step, now 4 to 12.
+  // The lowest cost of any share, and the smallest share within kNear of it
+  // (the decode part gains a little from more CUs where the estimate is level).
+  // The share of the lowest bound is priced first, and most others fall to
+  // theirs: at one KV head, 255 shares, pricing each cost 15 to 250 us a step.
   template <typename Cost, typename Least>
-  double lowest(int64_t start, Cost cost, Least least, int64_t* share) const {
-    double best = cost(start);
-    *share = start;
-    for (int64_t p = 1; p <= shares(); ++p) {
-      if (p == start || least(p) > best) continue;
-      const double c = cost(p);
-      if (c < best || (c == best && p < *share)) best = c, *share = p;
-    }
+  double lowest(Cost cost, Least least, int64_t* share) const {
+    constexpr double kNear = 1.01;
+    int64_t first = 1;
+    for (int64_t p = 2; p <= shares(); ++p)
+      if (least(p) < least(first)) first = p;
+    double best = cost(first);
+    for (int64_t p = 1; p <= shares(); ++p)
+      if (p != first && least(p) < best) best = std::min(best, cost(p));
+    *share = 1;
+    while (*share < shares() && (least(*share) > kNear * best || cost(*share) > kNear * best)) ++*share;
     return best;
   }
   double fastest(PrefillEstimate& e, int64_t* share) const {
-    return lowest(meet(e), [&](int64_t p) { return us(e, p); }, [&](int64_t p) { return least_us(e, p); }, share);
+    bound(e);
+    return lowest([&](int64_t p) { return us(e, p); }, [&](int64_t p) { return e.least_us[p]; }, share);
   }
   // Little decode beside many short tiles: the 128-row tiles of
   // mva_paged_mixed, two to a CU, start sooner.  64 / 8 heads, 13 decodes of
@@ -1130,16 +1141,20 @@ struct MixedStep {
     return max_tiles > share && e.work < 8.0 * (double)e.tiles && mb * kDecodeMinUsPerMB < 0.1 * step_us;
   }
   // Time of mva_paged_mixed with its own decode plan.
-  double one_launch_us(const PrefillEstimate& e, int64_t decode_pages, int64_t max_decode_pages, int group) const {
+  double one_launch_us(const PrefillEstimate& e, int64_t decode_seqs, int64_t decode_pages, int64_t max_decode_pages,
+                       int group) const {
     const double per_cu = (double)num_kv_heads / (double)num_cus;
-    const double piece = std::min(
-        std::max((double)decode_pages * num_kv_heads / (kPiecesPerWave * kMixedWavesPerCu * (double)num_cus), 4.0), 128.0);
+    const double waves = kMixedWavesPerCu * (double)num_cus;
+    const double piece =
+        std::min(std::max((double)decode_pages * num_kv_heads / (kPiecesPerWave * waves), 4.0), 128.0);
     const double chunks = std::ceil((double)max_decode_pages / piece);
     double decode = kOnePageUs * std::min(piece, (double)max_decode_pages);
-    if (chunks > 1)
-      decode += kOneMergeUs + group * (kOnePassUs * std::ceil(chunks / 32.0) + kOneChunkUs * chunks);
+    if (chunks > 1) decode += group * (kOnePassUs * std::ceil(chunks / 32.0) + kOneChunkUs * chunks);
+    const double pieces =
+        decode_seqs > 0 ? (double)decode_seqs * std::max(std::ceil((double)decode_pages / decode_seqs / piece), 1.0) : 0;
     const double prefill = kOneKeyUs * e.longest;
-    const double work = per_cu * (kOneWorkUs * e.half_work + kOneTileUs * (double)e.half_tiles) + kOneMBUs * mb;
+    const double work = per_cu * (kOneWorkUs * e.half_work + kOneTileUs * (double)e.half_tiles) + kOneMBUs * mb +
+                        kOnePieceUs * pieces * num_kv_heads / waves;
     return kOneStartUs + std::sqrt(prefill * prefill + decode * decode + work * work);
   }
 };
@@ -1178,26 +1193,27 @@ extern "C" int64_t mva_mixed_prefill_workgroups(const int64_t* prefill_pages, in
 }
 
 // The query lengths lie between two batches (packed_queries).  The share is the
-// one that loses least, as a factor of the lowest time at any share: to half
-// over the worse of the two, to half over evenly spread queries between them.
+// one that loses least, as a factor of the lowest time at any share: to a third
+// over the worse of the two, to two thirds over evenly spread queries.
 // Taken as evenly spread, a 2048-token prompt beside seven 8-token chunks over
 // 8000 (32 / 8 heads, 64 decodes of 2000) got 208 CUs for its prefill and 300
-// us, against 226 in mva_paged_mixed; the worse of the two alone gave the step
-// of a 8192-token budget 96 CUs (939 us) in place of 88 (922).  And a step whose
-// estimate is not below mva_paged_mixed's by kLaunchUs (its own launch of the
-// decode merges) and kMargin in either batch is left to that: steps of 15 to 25
-// us were 3 to 4 us slower on CUs of their own.  Over the drawn steps of the
-// fit, against mva_paged_mixed: 90 were slower by more than 3%, the worst by
-// 84%; now one, by 8%, and the mean time is lower too.
+// us, against 226 in mva_paged_mixed and 192 at the 168 CUs it gets now; the
+// worse of the two alone gave the step of a 8192-token budget 96 CUs (939 us) in
+// place of 88 (922).  And a step whose
+// estimate is not below mva_paged_mixed's by kLaunchUs in either batch is left to
+// that: steps of 15 to 25 us were 3 to 4 us slower on CUs of their own (the
+// launch of the decode merges).  Over 1230 drawn steps 136 were slower than
+// mva_paged_mixed by more than 3%, the worst by 84%; now 16, the worst by 14%,
+// and the mean time is 3.4% lower; over 300 drawn after the fit 34 and 7.
 extern "C" int64_t mva_mixed_prefill_share(const int64_t* prefill_pages, int64_t num_prefill_seqs,
-                                           int64_t num_prefill_tokens, int64_t max_query_len, int64_t decode_pages,
-                                           int64_t max_decode_pages, int num_q_heads, int num_kv_heads,
-                                           int64_t num_cus) try {
-  constexpr double kMargin = 1.05, kLaunchUs = 3.0;
+                                           int64_t num_prefill_tokens, int64_t max_query_len, int64_t num_decode_seqs,
+                                           int64_t decode_pages, int64_t max_decode_pages, int num_q_heads,
+                                           int num_kv_heads, int64_t num_cus) try {
+  constexpr double kLaunchUs = 1.0;
   MixedStep m;
   const int64_t n = num_prefill_seqs;
   if (!mixed_step(m, prefill_pages, n, num_prefill_tokens, decode_pages, num_q_heads, num_kv_heads, num_cus) ||
-      max_query_len < 0 || max_decode_pages < 0 || max_decode_pages > decode_pages)
+      max_query_len < 0 || num_decode_seqs < 0 || max_decode_pages < 0 || max_decode_pages > decode_pages)
     return -1;
   if (n == 0 || num_prefill_tokens == 0) return 0;
   const int group = num_q_heads / num_kv_heads;
@@ -1216,15 +1232,15 @@ extern "C" int64_t mva_mixed_prefill_share(const int64_t* prefill_pages, int64_t
     estimate(b, packed_queries(prefill_pages, n, num_prefill_tokens, max_query_len, b == 0));
   if (bounds == 2) {
     estimate(2, even_queries(prefill_pages, n, num_prefill_tokens));
-    auto lost = [&](auto us) { return us(2) / best[2] + std::max(us(0) / best[0], us(1) / best[1]); };
+    auto lost = [&](auto us) { return 2 * us(2) / best[2] + std::max(us(0) / best[0], us(1) / best[1]); };
     m.lowest(
-        share, [&](int64_t p) { return lost([&](int b) { return m.us(e[b], p); }); },
-        [&](int64_t p) { return lost([&](int b) { return m.least_us(e[b], p); }); }, &share);
+        [&](int64_t p) { return lost([&](int b) { return m.us(e[b], p); }); },
+        [&](int64_t p) { return lost([&](int b) { return e[b].least_us[p]; }); }, &share);
   }
   for (int b = 0; b < bounds; ++b) {
     const double us = m.us(e[b], share);
     if (m.short_tiles(e[b], share, us) ||
-        m.one_launch_us(e[b], decode_pages, max_decode_pages, group) < kMargin * us + kLaunchUs)
+        m.one_launch_us(e[b], num_decode_seqs, decode_pages, max_decode_pages, group) < us + kLaunchUs)
       return 0;
   }
   return share * num_kv_heads;

@@ -801,23 +801,23 @@ def paged_mixed(
 
 def mixed_prefill_workgroups(prefill_pages, num_prefill_tokens: int, decode_pages: int, num_q_heads: int,
                              num_kv_heads: int, num_cus: int, max_query_len: int | None = None,
-                             max_decode_pages: int | None = None) -> int:
+                             num_decode_seqs: int | None = None, max_decode_pages: int | None = None) -> int:
     """CUs :func:`paged_mixed_run` should give a step's prefill part:
     ``prefill_pages`` holds the pages of each prefill sequence,
     ``decode_pages`` those of all decode sequences.  With ``max_query_len`` (a
-    bound on the prefill queries of a sequence, 0 for none) and
-    ``max_decode_pages`` (of the longest decode sequence) the result is 0 where
+    bound on the prefill queries of a sequence, 0 for none), ``num_decode_seqs``
+    and ``max_decode_pages`` (of the longest of them) the result is 0 where
     :func:`paged_mixed` is expected to be faster
     (``mva_mixed_prefill_share``); without them queries are taken as evenly
     spread (``mva_mixed_prefill_workgroups``)."""
     pages = np.ascontiguousarray(prefill_pages, dtype=np.int64).reshape(-1)
     batch = (pages.ctypes.data, pages.size, int(num_prefill_tokens))
     machine = (int(num_q_heads), int(num_kv_heads), int(num_cus))
-    if max_query_len is None or max_decode_pages is None:
+    if max_query_len is None or num_decode_seqs is None or max_decode_pages is None:
         count = int(_native.query("mva_mixed_prefill_workgroups", *batch, int(decode_pages), *machine))
     else:
-        count = int(_native.query("mva_mixed_prefill_share", *batch, int(max_query_len), int(decode_pages),
-                                  int(max_decode_pages), *machine))
+        count = int(_native.query("mva_mixed_prefill_share", *batch, int(max_query_len), int(num_decode_seqs),
+                                  int(decode_pages), int(max_decode_pages), *machine))
     if count < 0:
         raise ValueError("invalid MIXED batch")
     return count

@@ -520,33 +520,36 @@ def test_mixed_prefill_workgroups_leave_cus_for_decode(hq, hkv, pages, tokens, d
     (32, 8, [500], 40, 40, [77, 600], False),
     (16, 2, [2], 2, 2, [34] * 16, False),
     (32, 8, [400, 200], 290, 200, [900, 1200], False),
-    (32, 8, [2048] + [8008] * 7, 2104, 2048, [2000] * 64, False),
     (32, 8, [4000, 16010], 4010, 4000, [4000] * 100, False),
     (32, 8, [2236], 300, 300, [2250] * 20, True),
     (32, 8, [4096] * 4, 2048, 512, [4391] * 256, True),
     (64, 8, [109], 109, 109, [12695], True),
     (16, 2, [1500] + [3050] * 3, 1650, 1500, [2000] * 60, True),
+    (32, 8, [2048] + [8008] * 7, 2104, 2048, [2000] * 64, True),
 ])
 def test_mixed_step_gets_cus_of_its_own_where_that_is_faster(hq, hkv, kv, tokens, longest, decode, alone):
     pages, decode_pages = ([-(-n // 16) for n in lens] for lens in (kv, decode))
-    share = ops.mixed_prefill_workgroups(pages, tokens, sum(decode_pages), hq, hkv, 256, longest, max(decode_pages))
+    share = ops.mixed_prefill_workgroups(pages, tokens, sum(decode_pages), hq, hkv, 256, longest, len(decode),
+                                         max(decode_pages))
     assert (share > 0) is alone and share % hkv == 0 and share < 256
+    if len(kv) == 8:  # 208 CUs, for evenly spread queries, starved decode: 300 us, 192 at 168
+        assert share <= 176
 
 
 def test_mixed_share_arguments():
     args = ([20, 4], 300, 50, 32, 8, 256)
     for pages in ([20, -1], [1 << 31, 4]):
-        for more in ((), (200, 9)):
+        for more in ((), (200, 7, 9)):
             with pytest.raises(ValueError):
                 ops.mixed_prefill_workgroups(pages, *args[1:], *more)
     # No walk over every tile of an absurd batch (the two would be 60 billion).
-    for more in ((), (10 ** 12, 9)):
+    for more in ((), (10 ** 12, 7, 9)):
         assert ops.mixed_prefill_workgroups([(1 << 31) - 1] * 2, 10 ** 12, 50, 32, 8, 256, *more) >= 0
-    assert ops.mixed_prefill_workgroups(*args, 0, 9) % 8 == 0  # no bound on the queries
-    for longest, decode in ((-1, 9), (200, -1), (200, 51)):
+    assert ops.mixed_prefill_workgroups(*args, 0, 7, 9) % 8 == 0  # no bound on the queries
+    for longest, seqs, decode in ((-1, 7, 9), (200, -1, 9), (200, 7, -1), (200, 7, 51)):
         with pytest.raises(ValueError):
-            ops.mixed_prefill_workgroups(*args, longest, decode)
-    assert ops.mixed_prefill_workgroups((), 0, 50, 32, 8, 256, 0, 9) == 0
+            ops.mixed_prefill_workgroups(*args, longest, seqs, decode)
+    assert ops.mixed_prefill_workgroups((), 0, 50, 32, 8, 256, 0, 7, 9) == 0
 
 
 @pytest.mark.parametrize("hq,hkv,pages,tokens,decode", [(8, 1, (128, 503, 503, 503), 2150, 15000),
