@@ -320,8 +320,9 @@ constexpr int64_t kArrivalBytes = (int64_t)kArrivalCounters * 4;
 constexpr int kStoreFlagInts = 65536;
 constexpr int64_t kStoreFlagBytes = (int64_t)kStoreFlagInts * 4;
 
+struct MergeParts;
 template <typename T, bool kAgent, int kWaves>
-__device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int wave, float* red);
+__device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int wave, MergeParts* parts);
 
 // One wavefront of a decode launch (`wave` in [0, num_waves)); `lds` is its
 // kDecodeWaveLdsBytes of LDS.
@@ -812,15 +813,19 @@ __device__ inline f32x4 part_load4(const float* a) {
 // of a wide merge.
 constexpr int kMergeRows = 32;
 constexpr int kWideMergeWaves = 8;
-// Floats of one merge of more than kMergeRows chunks in LDS: per wavefront of
-// the wide form a row of sums, the max and the weight sum.
-constexpr int kMergeLdsFloats = kWideMergeWaves * (kHeadDim + 2);
-
-// Sums over some chunks of a merge: the weighted rows (columns 4 * (lane % 32)
-// .. + 3), the weights, and the log-sum-exp they are relative to.
+// Sums over some chunks of a merge: of the weighted rows (columns 4 * (lane %
+// 32) .. + 3; lane half 0 the even rows of a block, half 1 the odd) and of the
+// weights (lane % 32: that row of a block), and the log-sum-exp they are
+// relative to.
 struct MergeSums {
   f32x4 acc;
   float m, wsum;
+};
+// The wide form's sums in LDS, one per wavefront.
+struct MergeParts {
+  f32x4 acc[kWideMergeWaves][64];
+  float wsum[kWideMergeWaves][32];
+  float m[kWideMergeWaves];
 };
 
 // The sums of chunks base .. base + 31, base + step .. base + step + 31, ...
@@ -866,39 +871,17 @@ __device__ __attribute__((always_inline)) inline MergeSums merge_chunks(const De
       acc += (half ? w1 : w0) * rows[j];
     }
   }
-#pragma unroll
-  for (int off = 16; off > 0; off >>= 1) wsum += __shfl_xor(wsum, off);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], 32);
   return {acc, m, wsum};
 }
 
-// Part v of kWideMergeWaves of a merge into its LDS (`red`, kMergeLdsFloats),
-// and the parts' total.
-__device__ __attribute__((always_inline)) inline void put_merge_part(float* red, int v, const MergeSums& s) {
-  const int lane = threadIdx.x & 63;
-  if (lane < 32) *reinterpret_cast<f32x4*>(red + v * kHeadDim + 4 * lane) = s.acc;
-  if (lane == 0) {
-    red[kWideMergeWaves * kHeadDim + v] = s.m;
-    red[kWideMergeWaves * (kHeadDim + 1) + v] = s.wsum;
-  }
-}
-__device__ __attribute__((always_inline)) inline MergeSums total_merge_parts(const float* red) {
-  const int col = 4 * (threadIdx.x & 31);
-  const float* const max_of = red + kWideMergeWaves * kHeadDim;
-  const float* const sum_of = max_of + kWideMergeWaves;
-  float mx = max_of[0];
-#pragma unroll
-  for (int v = 1; v < kWideMergeWaves; ++v) mx = fmaxf(mx, max_of[v]);
-  const float m_use = mx == -INFINITY ? 0.f : mx;
-  MergeSums s = {f32x4{0.f, 0.f, 0.f, 0.f}, mx, 0.f};
-#pragma unroll
-  for (int v = 0; v < kWideMergeWaves; ++v) {
-    const float f = fast_exp2(max_of[v] - m_use);
-    s.acc += f * *reinterpret_cast<const f32x4*>(red + v * kHeadDim + col);
-    s.wsum += f * sum_of[v];
-  }
-  return s;
+// Adds the sums of another part.
+__device__ __attribute__((always_inline)) inline void add_merge_part(MergeSums& total, const MergeSums& s) {
+  const float m = fmaxf(total.m, s.m);
+  const float m_use = m == -INFINITY ? 0.f : m;
+  const float a = fast_exp2(total.m - m_use), f = fast_exp2(s.m - m_use);
+  total.acc = total.acc * a + f * s.acc;
+  total.wsum = total.wsum * a + f * s.wsum;
+  total.m = m;
 }
 
 // Split-K merge of one (split segment, query head g): d is a piece
@@ -913,7 +896,7 @@ __device__ __attribute__((always_inline)) inline MergeSums total_merge_parts(con
 // So a wavefront requests 32 chunks at once (16-byte loads, two rows per
 // instruction: lane half 0 the even rows, half 1 the odd) together with
 // their log-sum-exps, and kWaves wavefronts of a workgroup take 32 chunks
-// each of every 32 * kWaves, meeting in LDS (`red`).
+// each of every 32 * kWaves, meeting in LDS (`parts`).
 // Measured, decode call of one sequence at 32 / 8 heads (256 chunks a head):
 // 30001 tokens 49.8 -> 32.3 us, 8192 tokens 32.4 -> 15.0 us against one
 // wavefront walking the chunks 16 at a time, 8 bytes a lane; 64 sequences of
@@ -925,8 +908,9 @@ __device__ __attribute__((always_inline)) inline MergeSums total_merge_parts(con
 // plan, and their bits are the same.  (Merges inside a launch walk the chunks
 // in one pass.)
 template <typename T, bool kAgent, int kWaves>
-__device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int wave, float* red) {
+__device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int wave, MergeParts* parts) {
   static_assert(kWaves == 1 || kWaves == kWideMergeWaves, "one wavefront, or one per part");
+  const int lane = threadIdx.x & 63;
   const int G = p.group;
   const int Hkv = p.num_kv_heads;
   const int n = d[4];
@@ -934,25 +918,41 @@ __device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int 
   const int64_t qrow = d[6];
   const int h = d[7];
   auto slot = [&](int k) -> int64_t { return ((int64_t)(pbase + k) * Hkv + h) * G + g; };
+  // One copy of merge_chunks in each form: these kernels run for a few
+  // microseconds, and fetching a second copy's code showed (0.3 us).
+  constexpr int kStep = kMergeRows * kWideMergeWaves;
   MergeSums s;
-  if (kAgent || n <= kMergeRows) {  // the same for every wavefront of the workgroup
-    if (wave != 0) return;
+  if constexpr (kAgent) {
     s = merge_chunks<kAgent>(p, slot, n, 0, kMergeRows);
   } else if constexpr (kWaves > 1) {
-    put_merge_part(red, wave, merge_chunks<kAgent>(p, slot, n, kMergeRows * wave, kMergeRows * kWideMergeWaves));
-    __syncthreads();
-    if (wave != 0) return;
-    s = total_merge_parts(red);
+    s = merge_chunks<kAgent>(p, slot, n, kMergeRows * wave, kStep);
+    if (n > kMergeRows) {  // the same for every wavefront of the workgroup
+      parts->acc[wave][lane] = s.acc;
+      if (lane < 32) parts->wsum[wave][lane] = s.wsum;
+      if (lane == 0) parts->m[wave] = s.m;
+      __syncthreads();
+      if (wave != 0) return;
+      auto add = [&](int v) { add_merge_part(s, {parts->acc[v][lane], parts->m[v], parts->wsum[v][lane & 31]}); };
+      add(1);
+      if (n > 2 * kMergeRows) {
+#pragma unroll
+        for (int v = 2; v < kWideMergeWaves; ++v) add(v);  // a part of no chunks adds zeros
+      }
+    } else if (wave != 0) {
+      return;
+    }
   } else {
 #pragma unroll 1
-    for (int v = 0; v < kWideMergeWaves; ++v)
-      put_merge_part(red, v, merge_chunks<kAgent>(p, slot, n, kMergeRows * v, kMergeRows * kWideMergeWaves));
-    // The wavefront's own LDS writes, in order.
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    s = total_merge_parts(red);
+    for (int v = 0; v < kWideMergeWaves && kMergeRows * v < n; ++v) {
+      const MergeSums part = merge_chunks<kAgent>(p, slot, n, kMergeRows * v, kStep);
+      if (v == 0) s = part;
+      else add_merge_part(s, part);
+    }
   }
-  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int off = 16; off > 0; off >>= 1) s.wsum += __shfl_xor(s.wsum, off);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) s.acc[e] += __shfl_xor(s.acc[e], 32);
   const float winv = s.wsum > 0.f ? 1.0f / s.wsum : 0.f;
   if (lane < 32) {
     typename Elem<T>::v4 y;

@@ -47,7 +47,6 @@ template <typename T, int kWide>
 __global__ __launch_bounds__(kWide == 1 ? 256 : 64 * kWide) void decode_merge_kernel(
     DecodeParams p, const int32_t* __restrict__ merges, int64_t num_waves, int64_t merge_blocks) {
   constexpr int kGroup = kWide == 1 ? 4 : kWide;  // wavefronts per workgroup
-  __shared__ __attribute__((aligned(16))) float red[(kWide == 1 ? kGroup : 1) * kMergeLdsFloats];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if ((int64_t)blockIdx.x >= merge_blocks) {
     const int64_t row = ((int64_t)blockIdx.x - merge_blocks) * kGroup + w;
@@ -59,8 +58,13 @@ __global__ __launch_bounds__(kWide == 1 ? 256 : 64 * kWide) void decode_merge_ke
   if (p.counts != nullptr && v >= (int64_t)max(sload(p.counts, 2), 0) * p.group) return;
   // v is wave-uniform: the descriptor comes in through scalar loads.
   const i32x8 d = ((const_i32x8*)merges)[v / p.group];
-  merge_segment<T, false, kWide>(p, d, (int)(v % p.group), kWide == 1 ? 0 : w,
-                                 kWide == 1 ? red + w * kMergeLdsFloats : red);
+  const int g = (int)(v % p.group);
+  if constexpr (kWide == 1) {
+    merge_segment<T, false, 1>(p, d, g, 0, nullptr);
+  } else {
+    __shared__ MergeParts parts;
+    merge_segment<T, false, kWide>(p, d, g, w, &parts);
+  }
 }
 
 // Wavefronts per merge of a launch of `num_merges` merges over
