@@ -898,7 +898,7 @@ __device__ __attribute__((always_inline)) inline void add_merge_part(MergeSums& 
 // their log-sum-exps, and kWaves wavefronts of a workgroup take 32 chunks
 // each of every 32 * kWaves, meeting in LDS (`parts`).
 // Measured, decode call of one sequence at 32 / 8 heads (256 chunks a head):
-// 30001 tokens 49.8 -> 32.3 us, 8192 tokens 32.4 -> 15.0 us against one
+// 30001 tokens 49.8 -> 32.9 us, 8192 tokens 32.4 -> 15.0 us against one
 // wavefront walking the chunks 16 at a time, 8 bytes a lane; 64 sequences of
 // 512-1024 tokens (5 chunks) 49.2 -> 48.8 us.
 //
@@ -906,7 +906,10 @@ __device__ __attribute__((always_inline)) inline void add_merge_part(MergeSums& 
 // its eight do, so the result does not depend on which of the two a launch
 // takes: a captured launch decides by its capacities, an eager one by its
 // plan, and their bits are the same.  (Merges inside a launch walk the chunks
-// in one pass.)
+// in one pass.)  One order for both costs 0.1 to 0.5 us a merge of more than
+// 32 chunks: 256 chunks 32.5 -> 32.9 us a call, one wavefront over 125 chunks
+// 8.2 -> 8.8 us the kernel.  Factors of all parts computed at once in lanes
+// were level with adding part after part.
 template <typename T, bool kAgent, int kWaves>
 __device__ void merge_segment(const DecodeParams& p, const i32x8& d, int g, int wave, MergeParts* parts) {
   static_assert(kWaves == 1 || kWaves == kWideMergeWaves, "one wavefront, or one per part");
